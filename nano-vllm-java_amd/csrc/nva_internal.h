@@ -210,6 +210,14 @@ constexpr int kRowTablePages = 64;
 // head) merge.
 constexpr int kMergeRowsMaxParts = 8;
 
+// The kernel on fp16 parts (head dims 64 and 128) behind the prefill functions: 32 queries of one
+// head per wave.
+constexpr int kPrefillSplitQueries = 32;
+bool prefill_split_supports(int head_dim);
+int prefill_split_waves(int head_dim);
+int prefill_split_blocks_per_cu(int head_dim, int heads_per_wg);
+hipError_t launch_prefill_split(const TileLaunch &a, int heads_per_wg, hipStream_t s);
+
 // Waves per prefill workgroup at this head dim (each wave owns 16 queries of one head; at
 // d = 512 a pair of waves shares them, one half of the head dims each).
 int prefill_waves(int head_dim);

@@ -1,4 +1,5 @@
-// Kernel (c): varlen causal prefill on fp32 MFMA over dense K/V or the paged KV cache.
+// Kernel (c) at head dims 256 and 512 (64 and 128: prefill_split.hip): varlen causal prefill on
+// fp32 MFMA over dense K/V or the paged KV cache.
 //
 // Semantics (layers/Attention.java:245-280 prefillDense / prefillWithCache, :328-396
 // attendJobs): query qi of a sequence with qLen queries and kLen keys sits at absolute
@@ -684,10 +685,8 @@ hipError_t launch_prefill_d(const TileLaunch &a, int hpw, hipStream_t s) {
 }  // namespace
 
 int prefill_waves(int head_dim) {
-  if (head_dim == 64) return tile_waves<64>();
-  if (head_dim == 256) return tile_waves<256>();
-  if (head_dim == 512) return tile_waves<512>();
-  return tile_waves<128>();
+  if (prefill_split_supports(head_dim)) return prefill_split_waves(head_dim);
+  return head_dim == 256 ? tile_waves<256>() : tile_waves<512>();
 }
 
 // At d = 512 a wave pair shares 16 queries (prefill512_kernel), one query head per workgroup;
@@ -697,6 +696,8 @@ int prefill_max_heads(int head_dim) {
 }
 
 int prefill_tile_queries(int head_dim, int heads_per_wg) {
+  if (prefill_split_supports(head_dim))
+    return kPrefillSplitQueries * (prefill_waves(head_dim) / heads_per_wg);
   const int query_blocks = head_dim == 512 ? prefill_waves(head_dim) / 2 : prefill_waves(head_dim);
   return 16 * (query_blocks / heads_per_wg);
 }
@@ -736,8 +737,7 @@ int blocks_per_cu_d(int hpw) {
 }  // namespace
 
 int prefill_blocks_per_cu(int head_dim, int heads_per_wg) {
-  if (head_dim == 64) return blocks_per_cu_d<64>(heads_per_wg);
-  if (head_dim == 256) return blocks_per_cu_d<256>(heads_per_wg);
+  if (prefill_split_supports(head_dim)) return prefill_split_blocks_per_cu(head_dim, heads_per_wg);
   if (head_dim == 512) {
     int b = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, prefill512_kernel<1>, 512, 0) !=
@@ -746,14 +746,14 @@ int prefill_blocks_per_cu(int head_dim, int heads_per_wg) {
       b = 1;
     return b;
   }
-  return blocks_per_cu_d<128>(heads_per_wg);
+  return blocks_per_cu_d<256>(heads_per_wg);
 }
 
 hipError_t launch_prefill_tiles(const TileLaunch &a, int hpw, hipStream_t s) {
   if (a.num_items <= 0 || a.num_slots <= 0) return hipSuccess;
   switch (a.head_dim) {
-    case 64: return launch_prefill_d<64>(a, hpw, s);
-    case 128: return launch_prefill_d<128>(a, hpw, s);
+    case 64:
+    case 128: return launch_prefill_split(a, hpw, s);
     case 256: return launch_prefill_d<256>(a, hpw, s);
     case 512:
       if (hpw != 1) return hipErrorInvalidValue;

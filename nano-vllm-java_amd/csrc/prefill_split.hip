@@ -1,0 +1,615 @@
+// Kernel (c) at head dims 64 and 128: varlen causal prefill on the fp16 matrix units at fp32
+// precision, over dense K/V or the paged KV cache.
+//
+// Semantics (layers/Attention.java:245-280 prefillDense / prefillWithCache, :328-396
+// attendJobs): query qi of a sequence with qLen queries and kLen keys sits at absolute
+// position aq = kLen - qLen + qi and sees keys [max(0, aq - W + 1) (window W > 0, else 0),
+// aq]; KV head kvh = h / rep; score = dot(q, k) * scale; out = softmax-weighted sum of v.
+//
+// Each fp32 operand (q, k, v and the probabilities) is split into two scaled fp16 parts and each
+// product taken as three fp16 ones with fp32 sums (split_f16.h), at 5.3 times the rate of
+// v_mfma_f32.
+//
+// Mapping onto CDNA4.  The grid and the stream-K segments are those of prefill.hip.  A segment
+// is a tile of 32 * NW / HPW queries of one sequence for HPW query heads of one KV head; each
+// wave owns 32 queries of one head, so one LDS read of a K or V operand (two parts, 32 bytes
+// a lane) feeds three 32 x 32 x 16 products.
+//   * Key tiles of 32 rows: each wave loads a share of the next tile's K and V rows into
+//     registers (8 floats of each per lane at a time) while the current tile is computed, then
+//     splits them and writes the parts to LDS, double-buffered, one barrier per tile.  K parts
+//     lie [key][dim], V parts [dim][key] in the key order of the PV contraction, so that both
+//     are read as 16-byte operands; 16-byte chunks are XOR-swizzled by the row (k_pos, part_pos) so
+//     that any 16 rows read at one column touch every bank once.
+//   * Scales: q per query; K and V per tile, from the tile's largest magnitude, which the waves
+//     exchange through LDS ahead of the barrier that the split waits for anyway.  A K tile's
+//     scale goes into the factor of its scores.  O^T is kept in the units of the largest V
+//     scale of the segment so far; a V tile whose own scale is smaller gets the difference
+//     through its probabilities.
+//   * S^T[key][query] = K Q^T, then O^T[dim][query] += V^T P^T: S^T leaves 16 keys of one query
+//     in each lane, which are the lane's B operand of PV once the contraction takes its keys in
+//     that order, so P never leaves registers.
+//   * Softmax in the log2 domain; the running max is moved, and O rescaled, only when a tile's
+//     max exceeds it by more than 2^8.  Only tiles that cross the causal diagonal, the window
+//     edge or the end of the keys are masked.
+//   * A tile with infinities, or whose rows lie further apart than one scale can hold, makes the
+//     workgroup take the segment again on fp32 instructions (scan_segment), and so does a wave
+//     that ends one with a sum that is not finite.
+//
+// Bound by vector and matrix instructions together (matrix units 43% busy at d = 128; the fp32
+// matrix kernel it replaces had them 85% busy).  Measured per layer call: a 2048-token chunk
+// after 12289 cached tokens, 32 q / 8 KV heads, d = 128: 3.31 -> 1.41 ms; four prompts of
+// 512-2048 tokens, 16 q / 8 KV: 272 -> 162 us; seven of 5-333 tokens at d = 64, 32 q / 8 KV:
+// 36.2 -> 30.0 us.  Error against float64 (rel-L2): 1.7e-6 -> 1.3e-6, 7.0e-7 -> 4.9e-7, 2.1e-7
+// -> 1.7e-7.
+#include "nva_internal.h"
+#include "nva_device.h"
+#include "split_f16.h"
+
+namespace nva {
+
+namespace {
+
+constexpr float kLog2e = 1.4426950408889634f;
+constexpr float kLazyRescale = 8.0f;  // log2 units
+constexpr int kProbExp = 7;            // probabilities, at most 2^8, are split as 2^7 p < 2^16
+constexpr int kVExpSpan = 40;          // a V tile's scale stays within 2^40 of the largest one's
+constexpr int KT = 32;                // keys per tile
+constexpr int QW = kPrefillSplitQueries;
+
+// Sum and max over lanes l and l ^ 32; both lanes get the same bits.
+__device__ __forceinline__ float sum_halves(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
+                                                  false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float max_halves(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
+                                                  false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// Offset (in fp16) of 16-byte chunk c of K row r of one part: 16 rows at any one column lie in
+// 16 different 16-byte columns of the 256-byte bank period (a row of 64 dims is half of one).
+template <int D>
+__device__ __forceinline__ int k_pos(int r, int c) {
+  const int x = D == 64 ? (r >> 1) & 7 : r & 15;
+  return r * D + ((c ^ x) << 3);
+}
+// Key (within the tile) at element j of V chunk c, step c / 2 and lane half c % 2 of the PV
+// contraction: the key of S^T register 8 (c / 2) + j.
+__device__ __forceinline__ int v_key(int c, int j) {
+  return 16 * (c >> 1) + 4 * (c & 1) + 8 * (j >> 2) + (j & 3);
+}
+
+// Row of key t: dense rows follow kbase; paged rows go through the LDS copy of the block
+// table, which starts at page blk0.
+__device__ __forceinline__ int64_t key_row(const KvView &kv, const int32_t *stab, int blk0,
+                                           int kbase, int t) {
+  if (!kv.paged) return (int64_t)kbase + t;
+  int blk, off;
+  if (kv.bs_shift >= 0) {
+    blk = t >> kv.bs_shift;
+    off = t & (kv.block_size - 1);
+  } else {
+    blk = t / kv.block_size;
+    off = t - blk * kv.block_size;
+  }
+  return (int64_t)stab[blk - blk0] * kv.block_size + off;
+}
+
+__device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
+
+// Where a query's results go: the output row, or the partial of one key chunk (rows of the tile
+// are laid out query-major, chunk-minor).
+struct Dest {
+  float *row;
+  size_t pidx;
+  bool partial;
+};
+__device__ __forceinline__ Dest destination(const TileLaunch &a, const TileItem &it, int qi, int h,
+                                            int D) {
+  Dest d;
+  d.partial = it.part >= 0;
+  d.pidx = 0;
+  if (!d.partial) {
+    d.row = a.out + ((size_t)(it.qstart + qi) * a.hq + h) * D;
+  } else {
+    d.pidx = ((size_t)it.part + (size_t)(qi - it.q0) * it.nsplit + it.split) * a.hq + h;
+    d.row = a.part_acc + d.pidx * D;
+  }
+  return d;
+}
+
+// The segment's result for 32 / DS queries (from tile query q0 on) on fp32 instructions, key by
+// key: 2 DS lanes share a query, D / (2 DS) dims each.  For segments that the split does not
+// fit; a few times slower than v_mfma_f32 tiles.
+template <int D, int DS>
+__device__ void scan_segment(const TileLaunch &a, const TileItem &it, const int32_t *stab, int blk0,
+                             int kvh, int h, int q0) {
+  constexpr int QN = QW / DS, DH = D / (2 * DS);
+  const int lane = threadIdx.x & 63;
+  const int dpart = lane / QN;
+  const int qi = q0 + lane % QN;
+  const bool qvalid = qi < it.qlen;
+  const int off = it.klen - it.qlen;
+  const int aq = off + (qvalid ? qi : it.qlen - 1);
+  const int lo = a.window > 0 ? max(0, aq - a.window + 1) : 0;
+  const float sl2 = a.scale * kLog2e;
+  const float *qp = a.q + ((size_t)(it.qstart + aq - off) * a.hq + h) * D + DH * dpart;
+  float q[DH], o[DH];
+#pragma unroll
+  for (int s = 0; s < DH; s += 4) {
+    const float4 x = ld4(qp + s);
+    q[s] = x.x, q[s + 1] = x.y, q[s + 2] = x.z, q[s + 3] = x.w;
+    o[s] = o[s + 1] = o[s + 2] = o[s + 3] = 0.0f;
+  }
+  float m = -INFINITY, l = 0.0f;
+  const size_t rs = (size_t)a.hkv * D;
+  const int q_last = min(q0 + QN, it.qlen) - 1;
+  const int k0 = max(it.ks, a.window > 0 ? max(0, off + q0 - a.window + 1) : 0);
+  const int k1 = min(it.ke, off + q_last + 1);
+#pragma unroll 1
+  for (int key = k0; key < k1; key++) {
+    const size_t at = (size_t)key_row(a.kv, stab, blk0, it.kbase, key) * rs + (size_t)kvh * D +
+                      (size_t)(DH * dpart);
+    float s = 0.0f;
+#pragma unroll
+    for (int c = 0; c < DH; c += 4) {
+      const float4 x = ld4(a.kv.k + at + c);
+      s = fmaf(x.x, q[c], s);
+      s = fmaf(x.y, q[c + 1], s);
+      s = fmaf(x.z, q[c + 2], s);
+      s = fmaf(x.w, q[c + 3], s);
+    }
+#pragma unroll
+    for (int x = 32; x >= QN; x >>= 1) s += __shfl_xor(s, x, 64);
+    s *= sl2;
+    const bool seen = key >= lo && key <= aq;
+    const float mn = seen && s > m ? s : m;
+    const float ms = mn == -INFINITY ? 0.0f : mn;
+    const float alpha = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - ms);
+    const float p = seen ? __builtin_amdgcn_exp2f(s - ms) : 0.0f;
+    if (mn != m) {
+      l *= alpha;
+#pragma unroll
+      for (int c = 0; c < DH; c++) o[c] *= alpha;
+      m = mn;
+    }
+    if (seen) {
+      l += p;
+#pragma unroll
+      for (int c = 0; c < DH; c += 4) {
+        const float4 x = ld4(a.kv.v + at + c);
+        o[c] = fmaf(p, x.x, o[c]);
+        o[c + 1] = fmaf(p, x.y, o[c + 1]);
+        o[c + 2] = fmaf(p, x.z, o[c + 2]);
+        o[c + 3] = fmaf(p, x.w, o[c + 3]);
+      }
+    }
+  }
+  if (!qvalid) return;
+  const Dest d = destination(a, it, qi, h, D);
+  const float inv = d.partial ? 1.0f : (l == 0.0f ? 0.0f : 1.0f / l);
+#pragma unroll
+  for (int c = 0; c < DH; c += 4)
+    *reinterpret_cast<float4 *>(d.row + DH * dpart + c) =
+        make_float4(o[c] * inv, o[c + 1] * inv, o[c + 2] * inv, o[c + 3] * inv);
+  if (d.partial && dpart == 0) {
+    a.part_m[d.pidx] = m;
+    a.part_l[d.pidx] = l;
+  }
+}
+
+// A wave's share of the workgroup's tiles: UW units of 64 lanes x 8 floats of K (RPU whole rows
+// each, a lane eight dims of one) and of V (one V chunk of 64 dims, a lane eight keys of one).
+template <int D, int NW>
+struct TileShare {
+  static constexpr int RPU = 64 / (D / 8);
+  static constexpr int UW = D / 16 / NW;
+  static_assert(RPU >= 1 && UW >= 1 && UW * NW * 16 == D, "tile does not split evenly over the waves");
+  const KvView &kv;
+  const float *k, *v;  // of this KV head
+  size_t rs;           // floats per token
+  const int32_t *stab;
+  int blk0, kbase, ke;
+  int wave, lane;
+  int cur_page, cur_id;  // page whose block id cur_id holds (wave-uniform)
+
+  __device__ int krow() const { return lane / (D / 8); }
+  __device__ int kchunk() const { return lane % (D / 8); }
+  __device__ int unit(int u) const { return u * NW + wave; }
+  // Row of key t, wave-uniform.
+  __device__ int64_t uniform_row(int t) {
+    const int pg = t >> kv.bs_shift;
+    if (pg != cur_page) {
+      cur_id = __builtin_amdgcn_readfirstlane(stab[pg - blk0]);
+      cur_page = pg;
+    }
+    return (int64_t)cur_id * kv.block_size + (t - (pg << kv.bs_shift));
+  }
+  // A full tile inside one page, or of dense rows: 32 consecutive rows.
+  __device__ bool one_run(int kt) const {
+    return kt + KT <= ke &&
+           (!kv.paged ||
+            (kv.bs_shift >= 0 && (kt >> kv.bs_shift) == ((kt + KT - 1) >> kv.bs_shift)));
+  }
+  // A full tile that starts at a multiple of 8 keys, over pages of at least 8: a K unit and each
+  // 4-key run of a V unit lie in one page.
+  __device__ bool short_runs(int kt) const {
+    return kt + KT <= ke && kv.bs_shift >= 3 && (kt & 7) == 0;
+  }
+  __device__ f32x8 load_krow(const float *row) const {
+    const float4 x = ld4(row + 8 * kchunk()), y = ld4(row + 8 * kchunk() + 4);
+    return f32x8{x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+  }
+
+  __device__ void load_k(int kt, f32x8 (&r)[UW]) {
+    const size_t lane_row = (size_t)krow() * rs;
+    if (one_run(kt)) {
+      const float *g = k + (kv.paged ? uniform_row(kt) : (int64_t)kbase + kt) * (int64_t)rs;
+#pragma unroll
+      for (int u = 0; u < UW; u++) r[u] = load_krow(g + (size_t)(unit(u) * RPU) * rs + lane_row);
+    } else if (short_runs(kt)) {
+#pragma unroll
+      for (int u = 0; u < UW; u++)
+        r[u] = load_krow(k + uniform_row(kt + unit(u) * RPU) * (int64_t)rs + lane_row);
+    } else {  // per-row addresses, rows past the chunk clamped to its last key (and masked)
+#pragma unroll
+      for (int u = 0; u < UW; u++) {
+        const int t = min(kt + unit(u) * RPU + krow(), ke - 1);
+        r[u] = load_krow(k + (size_t)key_row(kv, stab, blk0, kbase, t) * rs);
+      }
+    }
+  }
+  __device__ void load_v(int kt, f32x8 (&r)[UW]) {
+    if (one_run(kt)) {
+      const float *g = v + (kv.paged ? uniform_row(kt) : (int64_t)kbase + kt) * (int64_t)rs;
+#pragma unroll
+      for (int u = 0; u < UW; u++)
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+          r[u][j] = (g + (size_t)v_key(unit(u) & 3, j) * rs + 64 * (unit(u) >> 2))[lane];
+    } else if (short_runs(kt)) {
+#pragma unroll
+      for (int u = 0; u < UW; u++)
+#pragma unroll
+        for (int j = 0; j < 8; j += 4) {
+          const float *g = v + uniform_row(kt + v_key(unit(u) & 3, j)) * (int64_t)rs +
+                           64 * (unit(u) >> 2);
+#pragma unroll
+          for (int jj = 0; jj < 4; jj++) r[u][j + jj] = (g + (size_t)jj * rs)[lane];
+        }
+    } else {
+#pragma unroll
+      for (int u = 0; u < UW; u++) {
+        // One lane per row looks up the V rows; each lane then takes them in turn.
+        const int t = min(kt + v_key(unit(u) & 3, lane & 7), ke - 1);
+        const int64_t row = key_row(kv, stab, blk0, kbase, t);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+          const uint64_t x =
+              (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)row, j) |
+              (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(row >> 32), j) << 32;
+          r[u][j] = (v + (size_t)x * rs + 64 * (unit(u) >> 2))[lane];
+        }
+      }
+    }
+  }
+
+  // The share's parts to LDS; the second part lies KT * D further on.
+  __device__ void store_k(const f32x8 (&r)[UW], float scale, _Float16 *dst) const {
+#pragma unroll
+    for (int u = 0; u < UW; u++) {
+      const Split8 x = split8(r[u], scale);
+      _Float16 *d = dst + k_pos<D>(unit(u) * RPU + krow(), kchunk());
+      *reinterpret_cast<f16x8 *>(d) = x.hi;
+      *reinterpret_cast<f16x8 *>(d + KT * D) = x.lo;
+    }
+  }
+  __device__ void store_v(const f32x8 (&r)[UW], float scale, _Float16 *dst) const {
+#pragma unroll
+    for (int u = 0; u < UW; u++) {
+      const Split8 x = split8(r[u], scale);
+      _Float16 *d = dst + part_pos(64 * (unit(u) >> 2) + lane, unit(u) & 3);
+      *reinterpret_cast<f16x8 *>(d) = x.hi;
+      *reinterpret_cast<f16x8 *>(d + KT * D) = x.lo;
+    }
+  }
+  static __device__ float largest(const f32x8 (&r)[UW]) {
+    float m = 0.0f;
+#pragma unroll
+    for (int u = 0; u < UW; u++) m = abs_max(m, r[u]);
+    return m;
+  }
+};
+
+// Stages a segment's block ids in LDS, so that the tile loads never wait on a global load;
+// returns the first page.  Every wave of the workgroup calls it.
+__device__ __forceinline__ int stage_table(const TileLaunch &a, const TileItem &it, int32_t *stab) {
+  if (!a.kv.paged) return 0;
+  const int bs = a.kv.block_size;
+  const int blk0 = it.ks / bs;
+  const int npages = (it.ke - 1) / bs - blk0 + 1;
+  const int32_t *table = a.kv.table + (size_t)it.seq * a.kv.bt_stride + blk0;
+  for (int j = threadIdx.x; j < npages; j += blockDim.x) stab[j] = table[j];
+  __syncthreads();
+  return blk0;
+}
+
+}  // namespace
+
+// NW waves per workgroup.  At most 256 registers: two waves per SIMD.
+template <int D, int HPW, int NW>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
+prefill_split_kernel(TileLaunch a) {
+  constexpr int KS = D / 16;         // contraction steps of QK
+  constexpr int NB = D / 32;         // O^T blocks of 32 dims
+  constexpr int PART = KT * D;       // fp16 values of one part of a K (or V) tile
+  constexpr int UW = TileShare<D, NW>::UW;
+  __shared__ __attribute__((aligned(16))) _Float16 sk[2][2 * PART];
+  __shared__ __attribute__((aligned(16))) _Float16 sv[2][2 * PART];
+  __shared__ __attribute__((aligned(16))) float smax[2][2][NW];  // each wave's largest |k|, |v|
+  __shared__ int32_t stab[kPrefillTablePages];  // block ids of the pages this chunk touches
+
+  const int slot = blockIdx.x;
+  const int seg_end = a.seg_off[slot + 1];
+  const int rep = a.hq / a.hkv;
+  const int groups = rep / HPW;
+  const int kvh = blockIdx.y / groups;
+  // Wave-uniform, and known to be: every value derived from it lives in scalar registers.
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = kvh * rep + (blockIdx.y - kvh * groups) * HPW + wave % HPW;
+  const int qb = wave / HPW;
+  const int lane = threadIdx.x & 63;
+  const int i = lane & 31;     // MFMA row / column index of this lane
+  const int half = lane >> 5;  // MFMA k-slot
+  const int W = a.window;
+  // Scores are kept unscaled until the exponential; a negative scale goes into q's sign, so that
+  // the largest product is the largest score.
+  const float sl2 = fabsf(a.scale) * kLog2e;
+  const float qsign = a.scale < 0.0f ? -1.0f : 1.0f;
+  const size_t rs = (size_t)a.hkv * D;
+  const float *kbase = a.kv.k + (size_t)kvh * D;
+  const float *vbase = a.kv.v + (size_t)kvh * D;
+  const float one = opaque_one();
+
+  for (int seg = a.seg_off[slot]; seg < seg_end; seg++) {
+    // Every wave is done with the previous segment's LDS tiles and table before they are reused.
+    __syncthreads();
+    const TileItem it = a.items[seg];
+    const int off = it.klen - it.qlen;  // absolute position of query 0
+    // This lane's query (column i of S^T) and its visible key range.
+    const int wq0 = it.q0 + qb * QW;
+    const int qi = wq0 + i;
+    const bool qvalid = qi < it.qlen;
+    const int qic = qvalid ? qi : it.qlen - 1;
+    const int aq = off + qic;
+    const int vis_lo = W > 0 ? max(0, aq - W + 1) : 0;
+    const int vis_hi = aq + 1;
+    // The wave's 32 queries: bounds of their visible ranges.
+    const bool wave_active = wq0 < it.qlen;
+    const int wq1 = min(wq0 + QW - 1, it.qlen - 1);
+    const int wlo_min = W > 0 ? max(0, off + wq0 - W + 1) : 0;
+    const int wlo_max = W > 0 ? max(0, off + wq1 - W + 1) : 0;
+    const int whi_min = off + wq0 + 1;
+    const int whi_max = off + wq1 + 1;
+
+    // Q^T operand: lane (i, half) holds the parts of Q[query i][16 s + 8 half + 0..7] for the
+    // whole key loop (queries past the sequence read its last one).
+    Split8 q[KS];
+    float qscale;  // takes a product of scaled q and k (of exponent 0) to log2 units
+    {
+      const float *qp = a.q + ((size_t)(it.qstart + qic) * a.hq + h) * D + 8 * half;
+      f32x8 x[KS];
+      float mx = 0.0f;
+#pragma unroll
+      for (int s = 0; s < KS; s++) {
+        const float4 u = ld4(qp + 16 * s), v = ld4(qp + 16 * s + 4);
+        x[s] = f32x8{u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+        mx = abs_max(mx, x[s]);
+      }
+      const int e = split_exp(max_halves(mx));
+#pragma unroll
+      for (int s = 0; s < KS; s++) q[s] = split8(x[s], qsign * split_scale(e));
+      qscale = sl2 * split_unscale(e);
+    }
+    f32x16 o[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) o[b][r] = 0.0f;
+    float m_run = -INFINITY;  // log2 units
+    float l_run = 0.0f;
+    int o_exp = kMinExp;  // exponent of the V scale that o is in
+
+    TileShare<D, NW> share{a.kv, kbase, vbase, rs, stab, stage_table(a, it, stab), it.kbase, it.ke,
+                           wave, lane, -1, 0};
+    f32x8 rk[UW], rv[UW];  // this wave's share of the next tile, as loaded
+    auto load_tile = [&](int kt) {
+      share.load_k(kt, rk);
+      share.load_v(kt, rv);
+    };
+    // The tile in rk / rv: each wave's largest magnitudes, then (after a barrier) the exponents of
+    // its scales, and its parts in LDS.
+    auto share_max = [&](int b) {
+      const float m = max_waves(share.largest(rk), share.largest(rv));
+      if (i == 0) smax[b][half][wave] = m;
+    };
+    // A tile that does not fit one scale makes the segment unfit.
+    bool unfit = false;
+    int k_exp_in = kMinExp, v_exp_in = kMinExp, v_exp_max = kMinExp;
+    auto store_tile = [&](int b) {
+      const TileScales sc = tile_scales<NW>(smax[b][half][lane & (NW - 1)]);
+      unfit |= sc.unfit;
+      k_exp_in = sc.a;
+      v_exp_max = max(v_exp_max, sc.b);
+      v_exp_in = max(sc.b, v_exp_max - kVExpSpan);
+      share.store_k(rk, split_scale(k_exp_in), sk[b]);
+      share.store_v(rv, split_scale(v_exp_in), sv[b]);
+    };
+    auto read_split = [&](const _Float16 *p) {
+      return Split8{*reinterpret_cast<const f16x8 *>(p),
+                    *reinterpret_cast<const f16x8 *>(p + PART)};
+    };
+
+    // k_exp, v_exp: the tile's; v_max: the largest of the segment up to it, v_max >= v_exp.
+    auto compute_tile = [&](int kt, const _Float16 *tk, const _Float16 *tv, int k_exp, int v_exp,
+                            int v_max) {
+      if (!wave_active || kt >= whi_max || kt + KT <= wlo_min) return;
+      const bool full = (kt + KT <= whi_min) && (kt >= wlo_max);
+
+      // S^T = K Q^T: register r of st holds key kt + 8 (r / 4) + 4 half + r % 4 of query i.
+      f32x16 st;
+#pragma unroll
+      for (int r = 0; r < 16; r++) st[r] = 0.0f;
+#pragma unroll
+      for (int s = 0; s < KS; s++)
+        st = mfma_split(read_split(tk + k_pos<D>(i, 2 * s + half)), q[s], st);
+
+      float mx = -INFINITY;
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        if (!full) {
+          const int key = kt + 8 * (r >> 2) + 4 * half + (r & 3);
+          st[r] = (key >= vis_lo && key < vis_hi) ? st[r] : -INFINITY;
+        }
+        mx = fmaxf(mx, st[r]);
+      }
+      const float c = fmaxf(qscale * split_unscale(k_exp), 0x1p-126f);  // 0 * -inf is NaN
+      mx = max_halves(mx) * c;
+      const bool need = mx > m_run + kLazyRescale;
+      if (__any(need)) {
+        const float mn = need ? mx : m_run;
+        const float alpha = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - mn);
+        l_run *= alpha;
+#pragma unroll
+        for (int b = 0; b < NB; b++) o[b] *= alpha;
+        m_run = mn;
+      }
+      if (v_max != o_exp) {
+        const float alpha = __uint_as_float((uint32_t)max(0, 127 + o_exp - v_max) << 23);
+#pragma unroll
+        for (int b = 0; b < NB; b++) o[b] *= alpha;
+        o_exp = v_max;
+      }
+      const int p_exp = kProbExp + v_exp - v_max;
+      const float ms = (m_run == -INFINITY ? 0.0f : m_run) - (float)p_exp;
+      Split8 p[2];
+      float lt[2];
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        f32x8 e;
+#pragma unroll
+        for (int j = 0; j < 8; j++) e[j] = __builtin_amdgcn_exp2f(fmaf(st[8 * s + j], c, -ms));
+        lt[s] = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+        p[s] = split8_unscaled(e, one);
+      }
+      // One addition to the long sum per tile, without the probabilities' scale.
+      l_run = fmaf(lt[0] + lt[1], __uint_as_float((uint32_t)(127 - p_exp) << 23), l_run);
+
+      // O^T += V^T P^T, 16 keys a step (V chunk 2 s + half holds the lane's keys).
+#pragma unroll
+      for (int s = 0; s < 2; s++)
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+          o[b] = mfma_split(read_split(tv + part_pos(32 * b + i, 2 * s + half)), p[s], o[b]);
+    };
+
+    // At the barrier of tile t every wave is done with tile t - 1, whose buffer takes tile
+    // t + 1, tile t is in LDS, and so are the largest magnitudes of tile t + 1.
+    const int ntiles = (it.ke - it.ks + KT - 1) / KT;
+    load_tile(it.ks);
+    share_max(0);
+    __syncthreads();
+    store_tile(0);
+    if (ntiles > 1) load_tile(it.ks + KT);
+    for (int t = 0; t < ntiles; t++) {
+      const int kt = it.ks + t * KT;
+      const int b = t & 1;
+      const int k_exp = k_exp_in, v_exp = v_exp_in, v_max = v_exp_max;
+      if (t + 1 < ntiles) share_max(b ^ 1);
+      __syncthreads();
+      if (t + 1 < ntiles) store_tile(b ^ 1);
+      if (t + 2 < ntiles) load_tile(kt + 2 * KT);
+      compute_tile(kt, sk[b], sv[b], k_exp, v_exp, v_max);
+    }
+
+    if (!wave_active) continue;
+    const float l_tot = sum_halves(l_run);
+    float zero = 0.0f * l_tot;  // NaN if any sum is not finite
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) zero = fmaf(0.0f, o[b][r], zero);
+    if (unfit || __any(!(zero == 0.0f))) {
+      scan_segment<D, 1>(a, it, stab, share.blk0, kvh, h, wq0);
+      continue;
+    }
+    if (!qvalid) continue;
+    const Dest d = destination(a, it, qi, h, D);
+    const float inv = d.partial ? 1.0f : (l_tot == 0.0f ? 0.0f : 1.0f / l_tot);
+    const float vs = split_unscale(o_exp - kProbExp);
+    // Register r of o[b] is dim 32 b + 8 (r / 4) + 4 half + r % 4.
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+      for (int r = 0; r < 16; r += 4)
+        *reinterpret_cast<float4 *>(d.row + 32 * b + 2 * r + 4 * half) =
+            make_float4(o[b][r] * vs * inv, o[b][r + 1] * vs * inv, o[b][r + 2] * vs * inv,
+                        o[b][r + 3] * vs * inv);
+    if (d.partial && half == 0) {
+      a.part_m[d.pidx] = m_run;
+      a.part_l[d.pidx] = l_tot;
+    }
+  }
+}
+
+namespace {
+
+template <int D>
+constexpr int split_waves() {
+  return D == 64 ? 4 : 8;
+}
+
+template <int D, typename F>
+hipError_t with_heads(int hpw, F f) {
+  switch (hpw) {
+    case 1: return f(prefill_split_kernel<D, 1, split_waves<D>()>);
+    case 2: return f(prefill_split_kernel<D, 2, split_waves<D>()>);
+    case 4: return f(prefill_split_kernel<D, 4, split_waves<D>()>);
+    default: return hipErrorInvalidValue;
+  }
+}
+template <typename F>
+hipError_t with_kernel(int head_dim, int hpw, F f) {
+  return head_dim == 64 ? with_heads<64>(hpw, f) : with_heads<128>(hpw, f);
+}
+
+}  // namespace
+
+bool prefill_split_supports(int head_dim) { return head_dim == 64 || head_dim == 128; }
+int prefill_split_waves(int head_dim) {
+  return head_dim == 64 ? split_waves<64>() : split_waves<128>();
+}
+
+int prefill_split_blocks_per_cu(int head_dim, int hpw) {
+  int b = 0;
+  if (with_kernel(head_dim, hpw, [&](auto k) {
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(
+            &b, k, 64 * prefill_split_waves(head_dim), 0);
+      }) != hipSuccess ||
+      b < 1)
+    b = 1;
+  return b;
+}
+
+hipError_t launch_prefill_split(const TileLaunch &a, int hpw, hipStream_t s) {
+  const dim3 grid(a.num_slots, a.hkv * ((a.hq / a.hkv) / hpw));
+  const dim3 block(64 * prefill_split_waves(a.head_dim));
+  return with_kernel(a.head_dim, hpw, [&](auto k) {
+    hipLaunchKernelGGL(k, grid, block, 0, s, a);
+    return hipGetLastError();
+  });
+}
+
+}  // namespace nva

@@ -1,0 +1,150 @@
+// fp32 values as sums of two fp16 values, for contractions on the fp16 matrix units at fp32
+// precision (included by .hip sources only).
+//
+// x = hi + lo + e with hi = fp16(x) and lo = fp16(x - hi), both rounded to nearest (x - hi is
+// exact in fp32): hi holds 11 significant bits and lo, with its own sign and exponent, the next
+// 11 or 12, so |e| <= 2^-23 |x|, half an ulp of the fp32 value's own 24 bits away from it.  A
+// product x y is taken as lo hi' + hi lo' + hi hi', accumulated in fp32 with the largest last;
+// lo lo', below 2^-22 |x y| and of either sign, is left out.  The sum of n such products is off
+// by less than one fp32 accumulation of them, whose n roundings it does not make: the matrix
+// units round once per 16 products.
+//
+// fp16 has five exponent bits, so operands are scaled by powers of two (exact): the largest
+// magnitude of a block goes to [2^14, 2^15), below fp16's 65504, and the smallest step of lo,
+// 2^-24, is then 2^-38 of that magnitude: every element that matters next to the block's
+// largest keeps all its bits.  Blocks with infinities, or whose parts lie too far apart for one
+// scale, are detected by the users of this file and handled on fp32 instructions.
+//
+// Three v_mfma_f32_32x32x16_f16 do the work of eight v_mfma_f32_32x32x2_f32 at half the cycles
+// each: 5.3 times the fp32 matrix rate.  (Three bf16 parts need no scale but six products: the
+// board's power limit then holds the clock to 1.8 GHz, and the 12K + 2K prefill chunk at 32 query
+// heads took 2.05 ms however it was scheduled.)
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+namespace nva {
+
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// Eight values in two fp16 parts: one lane's operand of a 32x32x16 (or 16x16x32) product.
+struct Split8 {
+  f16x8 hi, lo;
+};
+
+// The parts of s x, s a power of two.  (x - hi comes from v_fma_mix_f32, which reads the fp16
+// half in place.)
+__device__ __forceinline__ Split8 split8(f32x8 x, float s) {
+  u32x4 hi, lo;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const float a = x[2 * j], b = x[2 * j + 1];
+    const f16x2 h = __builtin_convertvector(f32x2{s * a, s * b}, f16x2);
+    const f32x2 r{fmaf(s, a, -(float)h[0]), fmaf(s, b, -(float)h[1])};
+    hi[j] = __builtin_bit_cast(uint32_t, h);
+    lo[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, f16x2));
+  }
+  return Split8{__builtin_bit_cast(f16x8, hi), __builtin_bit_cast(f16x8, lo)};
+}
+
+// The parts of x itself.  `one` is 1.0f, opaque to the compiler (see opaque_one): with a
+// constant the residual would take a conversion and a subtraction each.
+__device__ __forceinline__ Split8 split8_unscaled(f32x8 x, float one) {
+  u32x4 hi, lo;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    const float a = x[2 * j], b = x[2 * j + 1];
+    const f16x2 h = __builtin_convertvector(f32x2{a, b}, f16x2);
+    const f32x2 r{fmaf(one, a, -(float)h[0]), fmaf(one, b, -(float)h[1])};
+    hi[j] = __builtin_bit_cast(uint32_t, h);
+    lo[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, f16x2));
+  }
+  return Split8{__builtin_bit_cast(f16x8, hi), __builtin_bit_cast(f16x8, lo)};
+}
+__device__ __forceinline__ float opaque_one() {
+  float one = 1.0f;
+  asm volatile("" : "+s"(one));
+  return one;
+}
+
+// Power-of-two scales of a block by the exponent field e of its largest magnitude (clamped to
+// [kMinExp, 255], so that every factor is a normal float): split_scale(e) takes that magnitude
+// to [2^14, 2^15), split_unscale(e) takes a result back.
+constexpr int kMinExp = 22;
+__device__ __forceinline__ int split_exp(float largest) {
+  return max((int)(__float_as_uint(largest) >> 23) & 255, kMinExp);
+}
+__device__ __forceinline__ float split_scale(int e) { return __uint_as_float((uint32_t)(268 - e) << 23); }
+__device__ __forceinline__ float split_unscale(int e) { return __uint_as_float((uint32_t)(e - 14) << 23); }
+
+// Largest magnitude of eight values.
+__device__ __forceinline__ float abs_max(float m, f32x8 x) {
+#pragma unroll
+  for (int j = 0; j < 8; j++) m = fmaxf(m, fabsf(x[j]));
+  return m;
+}
+
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp(uint32_t x) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float max_dpp(float x) {
+  return fmaxf(x, __uint_as_float(dpp<CTRL>(__float_as_uint(x))));
+}
+
+// The wave's maximum of a in lanes 0-31 and of b in lanes 32-63.
+__device__ __forceinline__ float max_waves(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false,
+                                                  false);
+  const float x = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  const auto t = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false,
+                                                  false);
+  float y = fmaxf(__uint_as_float(t[0]), __uint_as_float(t[1]));
+  y = max_dpp<0x128>(y);  // rotations by 8, 4, 2 and 1 within the 16 lanes of a row
+  y = max_dpp<0x124>(y);
+  y = max_dpp<0x122>(y);
+  return max_dpp<0x121>(y);
+}
+
+// Scales of a tile pair from its NW (4 or 8) waves' maxima: lanes 0-31 hold the first tensor's
+// (lane l that of wave l % NW), lanes 32-63 the second's.  A tile with an infinity, or whose
+// waves' maxima lie more than kShareSpan exponents apart (all-zero shares aside), does not fit
+// one scale: within the span the smallest share's smallest step is 2^-24 of its own largest.
+constexpr int kShareSpan = 14;
+struct TileScales {
+  int a, b;  // exponents (split_scale)
+  bool unfit;
+};
+template <int NW>
+__device__ __forceinline__ TileScales tile_scales(float largest) {
+  const uint32_t x = __float_as_uint(largest);
+  uint32_t hi = x, lo = x - 1;
+  hi = max(hi, dpp<0xB1>(hi)), lo = min(lo, dpp<0xB1>(lo));  // lanes ^ 1, ^ 2, then 8
+  hi = max(hi, dpp<0x4E>(hi)), lo = min(lo, dpp<0x4E>(lo));
+  if constexpr (NW == 8) hi = max(hi, dpp<0x141>(hi)), lo = min(lo, dpp<0x141>(lo));
+  const int e = (int)(hi >> 23);
+  const bool bad = e == 255 || e - (int)((lo + 1) >> 23) > kShareSpan;
+  const int es = e == 255 ? 141 : max(e, kMinExp);
+  return TileScales{__builtin_amdgcn_readlane(es, 0), __builtin_amdgcn_readlane(es, 32),
+                    __any(bad) != 0};
+}
+
+// Offset (in fp16) of 16-byte chunk c (0..3) of row r of a part whose rows hold 32 values, a
+// quarter of LDS's 256-byte bank period: 16 rows at any one column touch every bank once.
+__device__ __forceinline__ int part_pos(int r, int c) { return r * 32 + ((c ^ ((r >> 2) & 3)) << 3); }
+
+// c += a b, 32 x 32 x 16: lane l holds row (column) l % 32 of a (b) at k = 8 (l / 32) + 0..7;
+// c[r] is row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.
+__device__ __forceinline__ f32x16 mfma_split(const Split8 &a, const Split8 &b, f32x16 c) {
+  c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.lo, b.hi, c, 0, 0, 0);
+  c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a.hi, b.lo, c, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a.hi, b.hi, c, 0, 0, 0);
+}
+
+}  // namespace nva

@@ -1,0 +1,139 @@
+"""Prefill on split fp16 operands at magnitudes where the split can go wrong.
+
+The kernel scales q per query and K / V per 32-key tile by powers of two and falls back to fp32
+instructions where one scale cannot hold a tile.  Each case is compared with the oracle row by
+row (rel-L2 of every query row of every head), so that a small row beside a large one counts by
+itself.  Bar: 1e-5, the attention bar; non-finite results must be the oracle's.  Both sides sum
+up to 230 products per score and per output in fp32 (sqrt(230) * 2^-24 = 9e-7 of their size),
+and a score of size s moves its weight by s times that; s stays below 10."""
+
+import numpy as np
+import pytest
+
+from cases import Case
+from gpu_checks import dev, load_arena, say
+from nanollvm_amd import Attention, Context
+from nanollvm_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+
+SEQS = [(16, 70), (5, 33), (0, 2), (40, 190), (0, 31)]
+DENSE_SEQS = [(0, 70), (0, 33), (0, 2), (0, 190), (0, 31)]
+HEADS = [(64, 1), (64, 4), (128, 1), (128, 2)]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = Context(0)
+    yield c
+    c.close()
+
+
+def build(d, rep, layout, window=0, scale=None, seed=0):
+    rng = np.random.default_rng(seed + d + rep)
+    paged = layout != "dense"
+    wl = W.build(f"split d{d} rep{rep} {layout} w{window}", SEQS if paged else DENSE_SEQS,
+                 is_prefill=True, hq=2 * rep, hkv=2, d=d,
+                 scale=float(np.float32(scale if scale is not None else d ** -0.5)),
+                 window=window, rng=rng, paged=paged,
+                 block_size=int(layout[5:]) if paged else 256)
+    return Case(wl, seed=seed)
+
+
+def check(ctx, case, name):
+    wl = case.wl
+    say(name)
+    arena = load_arena(ctx, case)
+    try:
+        ctx.set(**wl.meta.context_args())
+        ctx.bind_kv_cache(arena)
+        with np.errstate(all="ignore"):
+            want, _, _ = case.oracle(threads=8)
+        out = Attention(wl.hq, wl.d, wl.scale, wl.hkv, wl.window, 0).forward(
+            dev(case.q), dev(case.k), dev(case.v), ctx)
+        ctx.sync()
+        got = out.cpu().numpy().astype(np.float64)
+    finally:
+        ctx.clear()
+        arena.close()
+    want = want.astype(np.float64)
+    odd = ~np.isfinite(want)
+    assert np.array_equal(got[odd], want[odd], equal_nan=True), "non-finite results differ"
+    assert np.all(np.isfinite(got[~odd])), "non-finite results where the oracle's are finite"
+    got[odd] = want[odd] = 0.0
+    err = np.linalg.norm(got - want, axis=-1)
+    size = np.linalg.norm(want, axis=-1)
+    rel = float(np.max(err / np.where(size > 0, size, 1.0)))
+    say(f"{name}: worst row rel_l2={rel:.3e}")
+    assert rel <= 1e-5, rel
+
+
+@pytest.mark.parametrize("layout", ["paged8", "paged16", "paged24", "paged4", "dense"])
+@pytest.mark.parametrize("window", [0, 37])
+@pytest.mark.parametrize("d,rep", HEADS)
+def test_page_sizes_and_window_starts(ctx, d, rep, window, layout):
+    """Pages of 8 tokens and more are read by whole runs, other sizes and unaligned window
+    starts row by row."""
+    check(ctx, build(d, rep, layout, window, seed=1), f"pages d{d} rep{rep} w{window} {layout}")
+
+
+@pytest.mark.parametrize("layout", ["paged16", "dense"])
+@pytest.mark.parametrize("d,rep", HEADS)
+def test_rows_of_unlike_size(ctx, d, rep, layout):
+    """K and V rows over 2^-6 .. 2^6 (within one scale's span), q rows over 2^-30 .. 2^0, and
+    whole sequences of V 2^+-50 apart (each its own tiles)."""
+    case = build(d, rep, layout, seed=2)
+    rng = np.random.default_rng(3)
+    T = case.wl.tokens
+    case.q *= np.exp2(rng.integers(-30, 1, (T, 1, 1))).astype(np.float32)
+    case.k *= np.exp2(rng.integers(-6, 2, (T, 1, 1))).astype(np.float32)
+    case.v *= np.exp2(rng.integers(-6, 7, (T, 1, 1))).astype(np.float32)
+    cu = case.wl.meta.cu_seqlens_q
+    for b in range(len(cu) - 1):
+        case.v[cu[b]:cu[b + 1]] *= np.float32(2.0 ** (50 if b % 2 else -50))
+        if case.paged:  # the sequence's cached rows with it
+            bs = case.wl.block_size
+            t = np.arange(case.wl.seqs[b][0])
+            rows = np.asarray(case.wl.tables[b], np.int64)[t // bs] * bs + t % bs
+            flat = case.v_cache.reshape(-1, case.wl.hkv, d)
+            flat[rows] *= np.float32(2.0 ** (50 if b % 2 else -50))
+    check(ctx, case, f"unlike rows d{d} rep{rep} {layout}")
+
+
+@pytest.mark.parametrize("layout", ["paged16", "dense"])
+@pytest.mark.parametrize("d,rep", HEADS)
+def test_rows_beyond_one_scale(ctx, d, rep, layout):
+    """One K row of 2^40 that every query weighs at 0, and one V row of 2^60 late in the same
+    tile: queries before it must keep the bits of their own small rows."""
+    case = build(d, rep, layout, seed=4)
+    first = int(case.wl.meta.cu_seqlens_q[3])
+    case.q[:, :, 0] = np.abs(case.q[:, :, 0]) + 0.5
+    case.k[first + 9] = 0.0
+    case.k[first + 9, :, 0] = -2.0 ** 40
+    case.v[first + 20] *= np.float32(2.0 ** 60)
+    check(ctx, case, f"beyond one scale d{d} rep{rep} {layout}")
+
+
+@pytest.mark.parametrize("layout", ["paged16", "dense"])
+@pytest.mark.parametrize("d,rep", HEADS)
+def test_infinities(ctx, d, rep, layout):
+    """An infinite V element reaches the queries that see it and no other; a key whose score is
+    -inf has weight 0."""
+    case = build(d, rep, layout, seed=5)
+    first = int(case.wl.meta.cu_seqlens_q[3])
+    case.q[:, :, 0] = np.abs(case.q[:, :, 0]) + 0.5
+    case.v[first + 100, :, 3] = np.inf
+    case.k[first + 7] = 0.0
+    case.k[first + 7, :, 0] = -np.inf
+    check(ctx, case, f"infinities d{d} rep{rep} {layout}")
+
+
+@pytest.mark.parametrize("d,rep", HEADS)
+def test_zeros_and_negative_scale(ctx, d, rep):
+    case = build(d, rep, "paged16", scale=-(d ** -0.5), seed=6)
+    check(ctx, case, f"negative scale d{d} rep{rep}")
+    case = build(d, rep, "dense", seed=7)
+    case.k[:40] = 0.0
+    case.v[20:90] = 0.0
+    case.q[60:] = 0.0
+    check(ctx, case, f"zeros d{d} rep{rep}")
