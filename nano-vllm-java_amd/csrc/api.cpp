@@ -160,14 +160,14 @@ struct Staging {
 // current step, built on the host and uploaded once, then reused by every layer with the same
 // configuration.
 struct PlanKey {
-  int window, mfma, tile_q, wg_per_item, blocks_per_cu;
+  int window, mfma, fp32_tiles, tile_q, wg_per_item, blocks_per_cu;
   int tile_groups;             // prefill grid height: KV heads x query-head groups
   int tokens;                  // rows of q / out in the forward call
   int paged;                   // keys through block tables (else dense k/v rows)
   int block_size, num_blocks;  // arena geometry the tables are checked against
   int head_dim, num_heads, num_kv_heads;  // size the work of a mixed plan's two kernels
   bool operator==(const PlanKey &o) const {
-    return window == o.window && mfma == o.mfma && tile_q == o.tile_q &&
+    return window == o.window && mfma == o.mfma && fp32_tiles == o.fp32_tiles && tile_q == o.tile_q &&
            head_dim == o.head_dim && num_heads == o.num_heads && num_kv_heads == o.num_kv_heads &&
            wg_per_item == o.wg_per_item && blocks_per_cu == o.blocks_per_cu &&
            tile_groups == o.tile_groups && tokens == o.tokens && paged == o.paged &&
@@ -322,11 +322,11 @@ struct DeviceGuard {
   }
 };
 
-int ctx_prefill_blocks_per_cu(nva_ctx *ctx, int head_dim, int hpw) {
-  const int key = head_dim * 16 + hpw;
+int ctx_prefill_blocks_per_cu(nva_ctx *ctx, int head_dim, int hpw, bool fp32) {
+  const int key = (head_dim * 16 + hpw) * 2 + (fp32 ? 1 : 0);
   auto it = ctx->occupancy.find(key);
   if (it != ctx->occupancy.end()) return it->second;
-  const int n = prefill_blocks_per_cu(head_dim, hpw);
+  const int n = fp32 ? prefill_fp32_blocks_per_cu(head_dim, hpw) : prefill_blocks_per_cu(head_dim, hpw);
   ctx->occupancy[key] = n;
   return n;
 }
@@ -529,7 +529,7 @@ nva_status get_plan(nva_ctx *ctx, const PlanKey &key, Plan **out) {
           ti.ks = W > 0 ? std::max(0, aq0 - W + 1) : 0;
           // Over small pages key tiles start at multiples of 8 keys, where the kernel reads
           // whole runs of rows from one page (the window masks the keys before it).
-          if (paged && key.block_size < 32) ti.ks &= ~7;
+          if (paged && key.block_size < 32 && !key.fp32_tiles) ti.ks &= ~7;
           ti.ke = aq1 + 1;
           ti.part = -1;
           ti.nsplit = 1;
@@ -910,12 +910,60 @@ KvView make_dense_view(const float *k, const float *v) {
   return view;
 }
 
+// Whether a prefill step runs on the fp32 tile kernel (prefill_fp32.hip) rather than the split one.
+// The split kernel multiplies 2.5 times as fast, but its tiles cover twice the queries, with half
+// the workgroups per CU, and a segment starts later; steps of a few short prompts or chunks leave
+// its waves idle.  Both kernels' times are estimated: the CU time of all key tiles (per tile, the
+// larger of a floor and the time of its active waves) over the CUs, or one tile's latency if that
+// is longer, plus the split kernel's later start.  The constants were fitted to the two kernels
+// on 40 drawn steps; fp32 / split us a layer at 40 q / 8 KV heads, d = 128: 2 + 16 + 208+3 tokens
+// 17.1 / 25.1, 230+11 and 211+15 21.1 / 27.5, 57 tokens 18.1 / 20.6, 280 tokens 45.7 / 36.7; at
+// d = 64, 140 and 245+58 tokens 27.4 / 29.3, 241+333 43.0 / 37.0; at d = 256, 1553+48 27.8 / 29.2,
+// 3736+100 43.6 / 38.9.
+bool use_fp32_tiles(nva_ctx *ctx, const nva_attn_desc &d, int hpw_fp32, int hpw_split, int window) {
+  struct Cost {
+    double floor, per_wave;  // CU us per key tile: at least, and per active wave
+    int per_cu;              // workgroups sharing the CU, so one tile's latency is floor * per_cu
+    int queries;             // queries (times heads) per wave
+  };
+  const int dim = d.head_dim;
+  const Cost fp32 = dim == 64    ? Cost{0.5, 0.28, 2, 16}
+                    : dim == 128 ? Cost{0.85, 0.56, 2, 16}
+                    : dim == 256 ? Cost{3.6, 1.2, 1, 16}
+                                 : Cost{5.0, 2.8, 1, 16};
+  const Cost split = dim == 64    ? Cost{0.6, 0.2, 3, 32}
+                     : dim == 128 ? Cost{2.5, 0.41, 1, 32}
+                     : dim == 256 ? Cost{6.5, 0.0, 1, 32}
+                                  : Cost{7.0, 0.0, 1, 32};
+  const double later = dim == 512 ? 3.0 : 2.0;  // us
+  auto estimate = [&](const Cost &c, int hpw, int tile_q) {
+    double sum = 0.0, longest = 0.0;
+    for (int b = 0; b < ctx->num_seqs; b++) {
+      const int qlen = ctx->cu_q[b + 1] - ctx->cu_q[b];
+      const int klen = ctx->cu_k[b + 1] - ctx->cu_k[b];
+      if (qlen < 2 || klen < qlen) continue;  // row kernel
+      for (int t0 = 0; t0 < qlen; t0 += tile_q) {
+        const int n = std::min(tile_q, qlen - t0);
+        const int first = klen - qlen + t0;
+        const int ks = window > 0 ? std::max(0, first - window + 1) : 0;
+        const double work = c.per_wave * hpw * ((n + c.queries - 1) / c.queries);
+        sum += std::max(c.floor, work) * ((first + n - ks + 31) / 32);
+        longest = std::max(longest, std::max(c.floor * c.per_cu, work));
+      }
+    }
+    return std::max(sum * (d.num_heads / hpw) / ctx->num_cus, longest);
+  };
+  return estimate(fp32, hpw_fp32, prefill_fp32_tile_queries(dim, hpw_fp32)) <=
+         estimate(split, hpw_split, prefill_tile_queries(dim, hpw_split)) + later;
+}
+
 // The plan of one attention call (the descriptor, the step, and whether keys are paged over
 // an arena of num_blocks pages of block_size tokens or dense rows), plus the query heads per
 // workgroup of the row and tile kernels.
 nva_status attention_plan(nva_ctx *ctx, const nva_attn_desc &d, int paged, int block_size,
                           int num_blocks, int num_tokens, Plan **plan, int *hpw_row,
-                          int *hpw_tile, bool *rows_mfma = nullptr) {
+                          int *hpw_tile, bool *rows_mfma = nullptr,
+                          bool *tiles_fp32 = nullptr) {
   const int rep = d.num_heads / d.num_kv_heads;
   // Query heads per row workgroup: the largest divisor of the GQA ratio the row kernel is built
   // for, so each K/V byte crosses HBM once per KV head (one head per workgroup at a ratio of 5
@@ -932,6 +980,11 @@ nva_status attention_plan(nva_ctx *ctx, const nva_attn_desc &d, int paged, int b
   // than with 4).
   *hpw_tile = largest_pow2_divisor_upto(rep, prefill_max_heads(d.head_dim));
   const bool mfma = ctx->is_prefill && prefill_kernel_supports(d.head_dim, *hpw_tile);
+  const int window = d.sliding_window > 0 ? d.sliding_window : 0;
+  const int hpw_fp32 = largest_pow2_divisor_upto(rep, prefill_fp32_max_heads(d.head_dim));
+  const bool fp32 = mfma && use_fp32_tiles(ctx, d, hpw_fp32, *hpw_tile, window);
+  if (fp32) *hpw_tile = hpw_fp32;
+  if (tiles_fp32) *tiles_fp32 = fp32;
   // The MFMA row kernel carries up to 16 heads of one KV head (it is used from 5).  Rows that
   // run beside MFMA prefill tiles (a mixed step) share the matrix pipes with them: there the row
   // kernel keeps 5 heads per KV head (40 query heads over 8 KV heads, Qwen3-4B-like mixed step:
@@ -952,11 +1005,14 @@ nva_status attention_plan(nva_ctx *ctx, const nva_attn_desc &d, int paged, int b
     return fail(ctx, NVA_E_UNSUPPORTED, "head_dim %d has no row kernel in this build",
                 d.head_dim);
   PlanKey key;
-  key.window = d.sliding_window > 0 ? d.sliding_window : 0;
+  key.window = window;
   key.mfma = mfma ? 1 : 0;
-  key.tile_q = mfma ? prefill_tile_queries(d.head_dim, *hpw_tile) : 0;
+  key.fp32_tiles = fp32 ? 1 : 0;
+  key.tile_q = !mfma  ? 0
+               : fp32 ? prefill_fp32_tile_queries(d.head_dim, *hpw_tile)
+                      : prefill_tile_queries(d.head_dim, *hpw_tile);
   key.wg_per_item = d.num_kv_heads * (rep / *hpw_row);
-  key.blocks_per_cu = mfma ? ctx_prefill_blocks_per_cu(ctx, d.head_dim, *hpw_tile) : 0;
+  key.blocks_per_cu = mfma ? ctx_prefill_blocks_per_cu(ctx, d.head_dim, *hpw_tile, fp32) : 0;
   key.tile_groups = mfma ? d.num_kv_heads * (rep / *hpw_tile) : 0;
   key.tokens = num_tokens;
   key.paged = paged;
@@ -1039,9 +1095,9 @@ nva_status run_attention(nva_ctx *ctx, const nva_attn_desc &d, const KvView &vie
                          Scratch *scr) {
   Plan *plan = nullptr;
   int hpw_row = 0, hpw_tile = 0;
-  bool rows_mfma = false;
+  bool rows_mfma = false, tiles_fp32 = false;
   nva_status st = attention_plan(ctx, d, view.paged, view.block_size, num_blocks, num_tokens,
-                                 &plan, &hpw_row, &hpw_tile, &rows_mfma);
+                                 &plan, &hpw_row, &hpw_tile, &rows_mfma, &tiles_fp32);
   if (st != NVA_OK) return st;
   const int window = d.sliding_window > 0 ? d.sliding_window : 0;
 
@@ -1107,7 +1163,10 @@ nva_status run_attention(nva_ctx *ctx, const nva_attn_desc &d, const KvView &vie
     t.part_l = pm + parts;
     t.part_acc = pm + 2 * parts;
     Timed tm(ctx, "prefill");
-    HIP_TRY(ctx, launch_prefill_tiles(t, hpw_tile, ctx->stream), "prefill kernel launch");
+    HIP_TRY(ctx,
+            tiles_fp32 ? launch_prefill_fp32(t, hpw_tile, ctx->stream)
+                       : launch_prefill_tiles(t, hpw_tile, ctx->stream),
+            "prefill kernel launch");
     tm.done();
   }
   if (plan->num_rows > 0) {

@@ -210,17 +210,12 @@ constexpr int kRowTablePages = 64;
 // head) merge.
 constexpr int kMergeRowsMaxParts = 8;
 
-// The kernel on fp16 parts (head dims 64 and 128) behind the prefill functions: 32 queries of one
-// head per wave.
-constexpr int kPrefillSplitQueries = 32;
-bool prefill_split_supports(int head_dim);
-int prefill_split_waves(int head_dim);
-int prefill_split_blocks_per_cu(int head_dim, int heads_per_wg);
-hipError_t launch_prefill_split(const TileLaunch &a, int heads_per_wg, hipStream_t s);
+// The fp32 tile kernel of small steps (prefill_fp32.hip), the same questions.
+int prefill_fp32_max_heads(int head_dim);
+int prefill_fp32_tile_queries(int head_dim, int heads_per_wg);
+int prefill_fp32_blocks_per_cu(int head_dim, int heads_per_wg);
+hipError_t launch_prefill_fp32(const TileLaunch &a, int heads_per_wg, hipStream_t s);
 
-// Waves per prefill workgroup at this head dim (each wave owns 16 queries of one head; at
-// d = 512 a pair of waves shares them, one half of the head dims each).
-int prefill_waves(int head_dim);
 // Most query heads one prefill workgroup carries at this head dim.
 int prefill_max_heads(int head_dim);
 // Query rows per prefill workgroup for a given heads-per-workgroup choice.

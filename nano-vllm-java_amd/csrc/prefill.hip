@@ -1,112 +1,91 @@
-// Kernel (c) at head dims 256 and 512 (64 and 128: prefill_split.hip): varlen causal prefill on
-// fp32 MFMA over dense K/V or the paged KV cache.
+// Kernel (c): varlen causal prefill on the fp16 matrix units at fp32 precision, over dense K/V or
+// the paged KV cache.  (Small steps: prefill_fp32.hip.)
 //
 // Semantics (layers/Attention.java:245-280 prefillDense / prefillWithCache, :328-396
 // attendJobs): query qi of a sequence with qLen queries and kLen keys sits at absolute
 // position aq = kLen - qLen + qi and sees keys [max(0, aq - W + 1) (window W > 0, else 0),
 // aq]; KV head kvh = h / rep; score = dot(q, k) * scale; out = softmax-weighted sum of v.
-// Keys come from dense k/v rows (prefillDense) or from the cache through the block table
-// (prefillWithCache).
 //
-// Mapping onto CDNA4.  The grid is exactly as many workgroups per head group as can be
-// resident at once; each runs the segments of its slot of a stream-K schedule (equal numbers
-// of 32-key tiles per slot; a query tile whose keys straddle slots is split and its partials
-// merged).  The whole step's K/V (tens of MB) stays in the 256 MB Infinity Cache, which all
-// XCDs share, so slots need no XCD-aware placement.  A segment is a tile of 16 * 8 / HPW queries of one
-// sequence for HPW query heads of one KV head, over a key range [ks, ke).  The 8 waves of the
-// workgroup each own 16 queries of one head.
-//   * Key tiles of 32 rows of K and V are copied HBM -> LDS with 16-byte loads that write LDS
-//     directly (no register staging), double-buffered so the next tile streams in while this
-//     one is used; one barrier per tile.  A full tile inside one page (or of dense rows) is 32
-//     consecutive rows: its copies are buffer loads from a wave-uniform descriptor plus fixed
-//     32-bit lane offsets, no per-lane address arithmetic; the last tile of a chunk and tiles
-//     that cross a page compute each row's address (rows past the chunk clamped).  Rows are
-//     stored unpadded; K rows have their 16-byte chunks XOR-swizzled (kswz) so the column
-//     reads of QK are conflict-free, V rows are read along the row and need no swizzle.  The
-//     block ids of the segment's pages are staged in LDS once, so a paged tile load never
-//     waits on a global table read.
-//   * Per tile each wave computes (D = 128)
-//       S^T[key][query] = K Q^T      64 x v_mfma_f32_16x16x4_f32, K from LDS (ds_read_b128),
-//                                    Q (16 queries x D/4 per lane) resident in registers;
-//       O^T[dim][query] += V^T P^T   64 x v_mfma_f32_16x16x4_f32, one ds_read_b128 of V feeds
-//                                    4 MFMAs (output block 4*hh + b holds dims 64*hh + 4r + b).
-//     With S transposed each lane holds 8 keys of ONE query: the row max is an in-lane max plus
-//     exchanges with lane^16 and lane^32, and P^T lands exactly in the registers the PV MFMA
-//     reads as its B operand (the key order of the contraction is permuted to match), so P
-//     never touches LDS.
-//   * Softmax runs in the log2 domain (scale * log2 e folded into the score, v_exp_f32), and the
-//     running max is only moved -- and O rescaled -- when a tile's max exceeds it by more than
-//     2^8, which after the first tiles almost never happens.
-//   * Only tiles that cross the causal diagonal, the window edge or the end of the keys are
-//     masked.
+// Each fp32 operand (q, k, v and the probabilities) is split into two scaled fp16 parts and each
+// product taken as three fp16 ones with fp32 sums (split_f16.h), at 5.3 times the rate of
+// v_mfma_f32.
+//
+// Mapping onto CDNA4.  The grid is exactly as many workgroups per head group as can be resident
+// at once; each runs the segments of its slot of a stream-K schedule (equal numbers of 32-key
+// tiles per slot; a query tile whose keys straddle slots is split and its partials merged).  A
+// segment is a tile of 32 * NW / HPW queries of one sequence for HPW query heads of one KV head; each
+// wave owns 32 queries of one head, so one LDS read of a K or V operand (two parts, 32 bytes
+// a lane) feeds three 32 x 32 x 16 products.
+//   * Key tiles of 32 rows: each wave loads a share of the next tile's K and V rows into
+//     registers (8 floats of each per lane at a time) while the current tile is computed, then
+//     splits them and writes the parts to LDS, double-buffered, one barrier per tile.  K parts
+//     lie [key][dim], V parts [dim][key] in the key order of the PV contraction, so that both
+//     are read as 16-byte operands; 16-byte chunks are XOR-swizzled by the row (k_pos, part_pos) so
+//     that any 16 rows read at one column touch every bank once.
+//   * Scales: q per query; K and V per tile, from the tile's largest magnitude, which the waves
+//     exchange through LDS ahead of the barrier that the split waits for anyway.  A K tile's
+//     scale goes into the factor of its scores.  O^T is kept in the units of the largest V
+//     scale of the segment so far; a V tile whose own scale is smaller gets the difference
+//     through its probabilities.
+//   * S^T[key][query] = K Q^T, then O^T[dim][query] += V^T P^T: S^T leaves 16 keys of one query
+//     in each lane, which are the lane's B operand of PV once the contraction takes its keys in
+//     that order, so P never leaves registers.
+//   * Softmax in the log2 domain; the running max is moved, and O rescaled, only when a tile's
+//     max exceeds it by more than 2^8.  Only tiles that cross the causal diagonal, the window
+//     edge or the end of the keys are masked.
+//   * A wave whose sums are not finite at the end of a segment (infinities in the inputs), or
+//     whose results are so small beside a tile's largest |k| or |v| that the steps of the split
+//     would show in them, takes its queries again on fp32 instructions (scan_segment).
+//   * Operands are read from LDS two steps ahead of their products and the next tile is split
+//     and stored after QK: 14% fewer cycles than in source order, 4% less time.
+//
+// Bound by the board's power where steps are large: at d = 128 the matrix units are 47% busy at
+// 2.0 GHz (40% at 2.2 GHz before the reads moved ahead), and splitting the waves into early and
+// late ones, raising their priority around QK or interleaving the split with the products changed
+// nothing.  At d = 512 reloads of spilled registers wait for the V loads in flight.  Measured per
+// layer call, against fp32 matrix instructions: a 2048-token chunk after 12289 cached tokens,
+// 32 q / 8 KV heads, d = 128: 3.31 -> 1.33 ms; prompts of 512-2048 tokens: 16 q / 8 KV heads,
+// d = 128, 270 -> 155 us; 4 q / 1 KV, d = 256, window 512, 126 -> 111 us; 8 q / 1 KV, d = 512,
+// 681 -> 474 us; seven prompts of 5-333 tokens, 32 q / 8 KV, d = 64: 35.1 -> 30.5 us.  Error
+// against float64 (rel-L2): 1.7e-6 -> 1.3e-6, 6.9e-7 -> 4.8e-7, 9.6e-7 -> 4.7e-7, 1.0e-6 ->
+// 6.1e-7, 2.1e-7 -> 1.7e-7.
 #include "nva_internal.h"
 #include "nva_device.h"
+#include "split_f16.h"
 
 namespace nva {
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLazyRescale = 8.0f;  // log2 units
+constexpr int kProbExp = 7;            // probabilities, at most 2^8, are split as 2^7 p < 2^16
+// Largest factor from products of scaled q and k (off by about 2^-7 from the steps of the split)
+// to scores: their error stays below 2^-20.
+constexpr float kMaxScoreUnit = 0x1p-13f;
+constexpr int kVExpSpan = 40;          // a V tile's scale stays within 2^40 of the largest one's
+constexpr int KT = 32;                // keys per tile
+constexpr int kAhead = 2;             // operand reads in flight ahead of their products
+constexpr int kKeepReads = 0x6;       // sched_barrier: only VALU and SALU move across
+constexpr int QW = 32;                // queries per wave
 
-}  // namespace
-
-// Pages of one key chunk whose block ids are staged in LDS (the host splits chunks to fit).
-constexpr int kTablePages = kPrefillTablePages;
-
-namespace {
-
-__device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
-
-// The pair {x[lane], x[lane ^ 16]} (resp. lane ^ 32) in every lane, by gfx950's row-swap
-// instructions: both outputs of the swap of x with itself hold one of the two values.
-struct Pair {
-  float a, b;
-};
-__device__ __forceinline__ Pair pair_xor16(float x) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false,
-                                                  false);
-  return {__uint_as_float(r[0]), __uint_as_float(r[1])};
-}
-__device__ __forceinline__ Pair pair_xor32(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
-                                                  false);
-  return {__uint_as_float(r[0]), __uint_as_float(r[1])};
-}
-// Max and sum over the four lanes {i, i+16, i+32, i+48}; every lane gets the same bits.
-__device__ __forceinline__ float max4_lanes(float x) {
-  const Pair p = pair_xor16(x);
-  const Pair q = pair_xor32(fmaxf(p.a, p.b));
-  return fmaxf(q.a, q.b);
-}
-__device__ __forceinline__ float sum4_lanes(float x) {
-  const Pair p = pair_xor16(x);
-  const Pair q = pair_xor32(p.a + p.b);
-  return q.a + q.b;
-}
-__device__ __forceinline__ void st4(float *p, float4 v) { *reinterpret_cast<float4 *>(p) = v; }
-
-// LDS position of chunk c of K row r (and, being an involution, the chunk at position c):
-// the low three bits are XORed with r & 7; from d = 256 on, where a lane group's 16 or more
-// chunks span a whole 256-byte bank period, bit 3 is also XORed with bit 4 of the chunk, which
-// tells adjacent lane groups apart (a lane group reads chunks 16g + j at d = 256 and, in the
-// half-row waves of d = 512, 64 half + 16g + j).  Measured with SQ_LDS_BANK_CONFLICT: zero
-// conflicts for d = 128, 256 and 512 (r & 15 alone: 33% of the LDS-active cycles at d = 128;
-// at d = 512, bit 3 from the parity of c / 32: 30%).
+// Offset (in fp16) of 16-byte chunk c of K row r of one part: 16 rows at any one column lie in
+// 16 different 16-byte columns of the 256-byte bank period (a row of 64 dims is half of one).
 template <int D>
-__device__ __forceinline__ int kswz(int c, int r) {
-  constexpr int GS = D / 16;  // chunks per lane group of a full-row read
-  int x = r & 7;
-  if constexpr (GS >= 16) x |= ((c >> 4) & 1) << 3;
-  return c ^ x;
+__device__ __forceinline__ int k_pos(int r, int c) {
+  const int x = D == 64 ? (r >> 1) & 7 : r & 15;
+  return r * D + ((c ^ x) << 3);
+}
+// Key (within the tile) at element j of V chunk c, step c / 2 and lane half c % 2 of the PV
+// contraction: the key of S^T register 8 (c / 2) + j.
+__device__ __forceinline__ int v_key(int c, int j) {
+  return 16 * (c >> 1) + 4 * (c & 1) + 8 * (j >> 2) + (j & 3);
 }
 
 // Row of key t: dense rows follow kbase; paged rows go through the LDS copy of the block
 // table, which starts at page blk0.
-__device__ __forceinline__ int64_t tile_row(const KvView &kv, const int32_t *stab, int blk0,
-                                            int kbase, int t) {
+__device__ __forceinline__ int64_t key_row(const KvView &kv, const int32_t *stab, int blk0,
+                                           int kbase, int t) {
   if (!kv.paged) return (int64_t)kbase + t;
   int blk, off;
   if (kv.bs_shift >= 0) {
@@ -119,51 +98,281 @@ __device__ __forceinline__ int64_t tile_row(const KvView &kv, const int32_t *sta
   return (int64_t)stab[blk - blk0] * kv.block_size + off;
 }
 
+__device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
+
+// Where a query's results go: the output row, or the partial of one key chunk (rows of the tile
+// are laid out query-major, chunk-minor).
+struct Dest {
+  float *row;
+  size_t pidx;
+  bool partial;
+};
+__device__ __forceinline__ Dest destination(const TileLaunch &a, const TileItem &it, int qi, int h,
+                                            int D) {
+  Dest d;
+  d.partial = it.part >= 0;
+  d.pidx = 0;
+  if (!d.partial) {
+    d.row = a.out + ((size_t)(it.qstart + qi) * a.hq + h) * D;
+  } else {
+    d.pidx = ((size_t)it.part + (size_t)(qi - it.q0) * it.nsplit + it.split) * a.hq + h;
+    d.row = a.part_acc + d.pidx * D;
+  }
+  return d;
+}
+
+// The segment's result for 32 / DS queries (from tile query q0 on) on fp32 instructions, key by
+// key: 2 DS lanes share a query, D / (2 DS) dims each.  For segments that the split does not
+// fit; a few times slower than v_mfma_f32 tiles.
+template <int D, int DS>
+__device__ void scan_segment(const TileLaunch &a, const TileItem &it, const int32_t *stab, int blk0,
+                             int kvh, int h, int q0) {
+  constexpr int QN = QW / DS, DH = D / (2 * DS);
+  const int lane = threadIdx.x & 63;
+  const int dpart = lane / QN;
+  const int qi = q0 + lane % QN;
+  const bool qvalid = qi < it.qlen;
+  const int off = it.klen - it.qlen;
+  const int aq = off + (qvalid ? qi : it.qlen - 1);
+  const int lo = a.window > 0 ? max(0, aq - a.window + 1) : 0;
+  const float sl2 = a.scale * kLog2e;
+  const float *qp = a.q + ((size_t)(it.qstart + aq - off) * a.hq + h) * D + DH * dpart;
+  float q[DH], o[DH];
+#pragma unroll
+  for (int s = 0; s < DH; s += 4) {
+    const float4 x = ld4(qp + s);
+    q[s] = x.x, q[s + 1] = x.y, q[s + 2] = x.z, q[s + 3] = x.w;
+    o[s] = o[s + 1] = o[s + 2] = o[s + 3] = 0.0f;
+  }
+  float m = -INFINITY, l = 0.0f;
+  const size_t rs = (size_t)a.hkv * D;
+  const int q_last = min(q0 + QN, it.qlen) - 1;
+  const int k0 = max(it.ks, a.window > 0 ? max(0, off + q0 - a.window + 1) : 0);
+  const int k1 = min(it.ke, off + q_last + 1);
+#pragma unroll 1
+  for (int key = k0; key < k1; key++) {
+    const size_t at = (size_t)key_row(a.kv, stab, blk0, it.kbase, key) * rs + (size_t)kvh * D +
+                      (size_t)(DH * dpart);
+    float s = 0.0f;
+#pragma unroll
+    for (int c = 0; c < DH; c += 4) {
+      const float4 x = ld4(a.kv.k + at + c);
+      s = fmaf(x.x, q[c], s);
+      s = fmaf(x.y, q[c + 1], s);
+      s = fmaf(x.z, q[c + 2], s);
+      s = fmaf(x.w, q[c + 3], s);
+    }
+#pragma unroll
+    for (int x = 32; x >= QN; x >>= 1) s += __shfl_xor(s, x, 64);
+    s *= sl2;
+    const bool seen = key >= lo && key <= aq;
+    const float mn = seen && s > m ? s : m;
+    const float ms = mn == -INFINITY ? 0.0f : mn;
+    const float alpha = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - ms);
+    const float p = seen ? __builtin_amdgcn_exp2f(s - ms) : 0.0f;
+    if (mn != m) {
+      l *= alpha;
+#pragma unroll
+      for (int c = 0; c < DH; c++) o[c] *= alpha;
+      m = mn;
+    }
+    if (seen) {
+      l += p;
+#pragma unroll
+      for (int c = 0; c < DH; c += 4) {
+        const float4 x = ld4(a.kv.v + at + c);
+        o[c] = fmaf(p, x.x, o[c]);
+        o[c + 1] = fmaf(p, x.y, o[c + 1]);
+        o[c + 2] = fmaf(p, x.z, o[c + 2]);
+        o[c + 3] = fmaf(p, x.w, o[c + 3]);
+      }
+    }
+  }
+  if (!qvalid) return;
+  const Dest d = destination(a, it, qi, h, D);
+  const float inv = d.partial ? 1.0f : (l == 0.0f ? 0.0f : 1.0f / l);
+#pragma unroll
+  for (int c = 0; c < DH; c += 4)
+    *reinterpret_cast<float4 *>(d.row + DH * dpart + c) =
+        make_float4(o[c] * inv, o[c + 1] * inv, o[c + 2] * inv, o[c + 3] * inv);
+  if (d.partial && dpart == 0) {
+    a.part_m[d.pidx] = m;
+    a.part_l[d.pidx] = l;
+  }
+}
+
+// Whether a query's sums (o in units of 2^kProbExp and the V scale; every lane of the query has
+// its part) cannot stand: one is not finite, or the result lies more than 2^14 below the largest
+// |v|, where the steps of the split V would show in it.
+template <int NB>
+__device__ __forceinline__ bool unsound(const f32x16 (&o)[NB], float l, int o_exp) {
+  float zero = 0.0f * l, top = 0.0f;
+#pragma unroll
+  for (int b = 0; b < NB; b++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      zero = fmaf(0.0f, o[b][r], zero);  // NaN if any is not finite
+      top = fmaxf(top, fabsf(o[b][r]));
+    }
+  top = max_halves(top);
+  // (At the smallest scale, V holds nothing but zeros and values below 2^-105.)
+  return !(zero == 0.0f) || (top < l * (float)(1 << kProbExp) && o_exp > kMinExp);
+}
+
+// A wave's share of the workgroup's tiles: UW units of 64 lanes x 8 floats of K (RPU whole rows
+// each, a lane eight dims of one) and of V (one V chunk of 64 dims, a lane eight keys of one).
+template <int D, int NW>
+struct TileShare {
+  static constexpr int RPU = 64 / (D / 8);
+  static constexpr int UW = D / 16 / NW;
+  static_assert(RPU >= 1 && UW >= 1 && UW * NW * 16 == D, "tile does not split evenly over the waves");
+  const KvView &kv;
+  const float *k, *v;  // of this KV head
+  size_t rs;           // floats per token
+  const int32_t *stab;
+  int blk0, kbase, ke;
+  int wave, lane;
+  int cur_page, cur_id;  // page whose block id cur_id holds (wave-uniform)
+
+  __device__ int krow() const { return lane / (D / 8); }
+  __device__ int kchunk() const { return lane % (D / 8); }
+  __device__ int unit(int u) const { return u * NW + wave; }
+  // Row of key t, wave-uniform.
+  __device__ int64_t uniform_row(int t) {
+    const int pg = t >> kv.bs_shift;
+    if (pg != cur_page) {
+      cur_id = __builtin_amdgcn_readfirstlane(stab[pg - blk0]);
+      cur_page = pg;
+    }
+    return (int64_t)cur_id * kv.block_size + (t - (pg << kv.bs_shift));
+  }
+  // A full tile inside one page, or of dense rows: 32 consecutive rows.
+  __device__ bool one_run(int kt) const {
+    return kt + KT <= ke &&
+           (!kv.paged ||
+            (kv.bs_shift >= 0 && (kt >> kv.bs_shift) == ((kt + KT - 1) >> kv.bs_shift)));
+  }
+  // A full tile that starts at a multiple of 8 keys, over pages of at least 8: a K unit and each
+  // 4-key run of a V unit lie in one page.
+  __device__ bool short_runs(int kt) const {
+    return kt + KT <= ke && kv.bs_shift >= 3 && (kt & 7) == 0;
+  }
+  __device__ f32x8 load_krow(const float *row) const {
+    const float4 x = ld4(row + 8 * kchunk()), y = ld4(row + 8 * kchunk() + 4);
+    return f32x8{x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w};
+  }
+
+  __device__ void load_k(int kt, f32x8 (&r)[UW]) {
+    const size_t lane_row = (size_t)krow() * rs;
+    if (one_run(kt)) {
+      const float *g = k + (kv.paged ? uniform_row(kt) : (int64_t)kbase + kt) * (int64_t)rs;
+#pragma unroll
+      for (int u = 0; u < UW; u++) r[u] = load_krow(g + (size_t)(unit(u) * RPU) * rs + lane_row);
+    } else if (short_runs(kt)) {
+#pragma unroll
+      for (int u = 0; u < UW; u++)
+        r[u] = load_krow(k + uniform_row(kt + unit(u) * RPU) * (int64_t)rs + lane_row);
+    } else {  // per-row addresses, rows past the chunk clamped to its last key (and masked)
+#pragma unroll
+      for (int u = 0; u < UW; u++) {
+        const int t = min(kt + unit(u) * RPU + krow(), ke - 1);
+        r[u] = load_krow(k + (size_t)key_row(kv, stab, blk0, kbase, t) * rs);
+      }
+    }
+  }
+  __device__ void load_v(int kt, f32x8 (&r)[UW]) {
+    if (one_run(kt)) {
+      const float *g = v + (kv.paged ? uniform_row(kt) : (int64_t)kbase + kt) * (int64_t)rs;
+#pragma unroll
+      for (int u = 0; u < UW; u++)
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+          r[u][j] = (g + (size_t)v_key(unit(u) & 3, j) * rs + 64 * (unit(u) >> 2))[lane];
+    } else if (short_runs(kt)) {
+#pragma unroll
+      for (int u = 0; u < UW; u++)
+#pragma unroll
+        for (int j = 0; j < 8; j += 4) {
+          const float *g = v + uniform_row(kt + v_key(unit(u) & 3, j)) * (int64_t)rs +
+                           64 * (unit(u) >> 2);
+#pragma unroll
+          for (int jj = 0; jj < 4; jj++) r[u][j + jj] = (g + (size_t)jj * rs)[lane];
+        }
+    } else {
+#pragma unroll
+      for (int u = 0; u < UW; u++) {
+        // One lane per row looks up the V rows; each lane then takes them in turn.
+        const int t = min(kt + v_key(unit(u) & 3, lane & 7), ke - 1);
+        const int64_t row = key_row(kv, stab, blk0, kbase, t);
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+          const uint64_t x =
+              (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)row, j) |
+              (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(row >> 32), j) << 32;
+          r[u][j] = (v + (size_t)x * rs + 64 * (unit(u) >> 2))[lane];
+        }
+      }
+    }
+  }
+
+  // The share's parts to LDS; the second part lies KT * D further on.
+  __device__ void store_k(const f32x8 (&r)[UW], float scale, _Float16 *dst) const {
+#pragma unroll
+    for (int u = 0; u < UW; u++) {
+      const Split8 x = split8(r[u], scale);
+      _Float16 *d = dst + k_pos<D>(unit(u) * RPU + krow(), kchunk());
+      *reinterpret_cast<f16x8 *>(d) = x.hi;
+      *reinterpret_cast<f16x8 *>(d + KT * D) = x.lo;
+    }
+  }
+  __device__ void store_v(const f32x8 (&r)[UW], float scale, _Float16 *dst) const {
+#pragma unroll
+    for (int u = 0; u < UW; u++) {
+      const Split8 x = split8(r[u], scale);
+      _Float16 *d = dst + part_pos(64 * (unit(u) >> 2) + lane, unit(u) & 3);
+      *reinterpret_cast<f16x8 *>(d) = x.hi;
+      *reinterpret_cast<f16x8 *>(d + KT * D) = x.lo;
+    }
+  }
+  static __device__ float largest(const f32x8 (&r)[UW]) {
+    float m = 0.0f;
+#pragma unroll
+    for (int u = 0; u < UW; u++) m = abs_max(m, r[u]);
+    return m;
+  }
+};
+
+// Stages a segment's block ids in LDS, so that the tile loads never wait on a global load;
+// returns the first page.  Every wave of the workgroup calls it.
+__device__ __forceinline__ int stage_table(const TileLaunch &a, const TileItem &it, int32_t *stab) {
+  if (!a.kv.paged) return 0;
+  const int bs = a.kv.block_size;
+  const int blk0 = it.ks / bs;
+  const int npages = (it.ke - 1) / bs - blk0 + 1;
+  const int32_t *table = a.kv.table + (size_t)it.seq * a.kv.bt_stride + blk0;
+  for (int j = threadIdx.x; j < npages; j += blockDim.x) stab[j] = table[j];
+  __syncthreads();
+  return blk0;
+}
+
 }  // namespace
 
-// NW waves per workgroup, KT keys per tile.  Four waves per SIMD (at most 128 VGPRs) for
-// d <= 128; d = 256 needs more than 128 registers for its Q and O blocks, and d = 512 keeps
-// its O blocks in AGPRs (one wave per SIMD).
-template <int D, int HPW, int KT, int NW>
-__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 4 : 1)))
-prefill_kernel(TileLaunch a) {
-  constexpr int KB = KT / 16;      // 16-key MFMA blocks per key tile
-  constexpr int DQ = D / 4;        // QK contraction steps per lane group g: dims [DQ*g, DQ*g+DQ)
-  constexpr int NB = D / 16;       // O^T blocks of 16 dims: block 4*hh+bb holds dims 64*hh+4r+bb
-  constexpr int H64 = D / 64;      // 64-dim halves of a V row (one ds_read_b128 each)
-  constexpr int C4 = D / 4;        // 16-byte chunks per K/V row
-  constexpr int NI = KT * C4 / 64;  // load instructions per tensor per tile (64 chunks each)
-  constexpr int LPW = NI / NW;     // load instructions per wave per tensor per tile
-  constexpr int TILE = KT * D;     // floats per K (or V) tile
-  static_assert(LPW >= 1 && NI % NW == 0, "tile does not split evenly over the waves");
-  __shared__ __attribute__((aligned(16))) float sk0[TILE];
-  __shared__ __attribute__((aligned(16))) float sv0[TILE];
-  __shared__ __attribute__((aligned(16))) float sk1[TILE];
-  __shared__ __attribute__((aligned(16))) float sv1[TILE];
-  __shared__ int32_t stab[kTablePages];  // block ids of the pages this chunk touches
+// NW waves per workgroup.  At most 256 registers and two waves per SIMD at d = 128, 168 and three
+// at d = 64.
+template <int D, int HPW, int NW>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(D == 64 ? 3 : 2)))
+prefill_split_kernel(TileLaunch a) {
+  constexpr int KS = D / 16;         // contraction steps of QK
+  constexpr int NB = D / 32;         // O^T blocks of 32 dims
+  constexpr int PART = KT * D;       // fp16 values of one part of a K (or V) tile
+  constexpr int UW = TileShare<D, NW>::UW;
+  __shared__ __attribute__((aligned(16))) _Float16 sk[2][2 * PART];
+  __shared__ __attribute__((aligned(16))) _Float16 sv[2][2 * PART];
+  __shared__ __attribute__((aligned(16))) float smax[2][2][NW];  // each wave's largest |k|, |v|
+  __shared__ int32_t stab[kPrefillTablePages];  // block ids of the pages this chunk touches
 
   const int slot = blockIdx.x;
   const int seg_end = a.seg_off[slot + 1];
-  // Byte offsets of this lane's copies within a tile whose 32 rows are consecutive rows of the
-  // K/V arrays (every full tile of a dense step, and of a paged one when it lies in one page):
-  // such a tile is copied from one wave-uniform base plus these fixed offsets.
-  uint32_t koff[LPW], voff[LPW];
-  {
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t rsb = (uint32_t)(a.hkv * D) * 4u;
-#pragma unroll
-    for (int p = 0; p < LPW; p++) {
-      const int q = (p * NW + wave) * 64 + lane;  // chunk q of the tile, row-major
-      const int r = q / C4, pos = q - r * C4;
-      koff[p] = (uint32_t)r * rsb + (uint32_t)kswz<D>(pos, r) * 16u;
-      voff[p] = (uint32_t)r * rsb + (uint32_t)pos * 16u;
-    }
-  }
-  for (int seg = a.seg_off[slot]; seg < seg_end; seg++) {
-  // Every wave is done with the previous segment's LDS tiles and table before they are reused.
-  __syncthreads();
-  const TileItem it = a.items[seg];
   const int rep = a.hq / a.hkv;
   const int groups = rep / HPW;
   const int kvh = blockIdx.y / groups;
@@ -172,595 +381,567 @@ prefill_kernel(TileLaunch a) {
   const int h = kvh * rep + (blockIdx.y - kvh * groups) * HPW + wave % HPW;
   const int qb = wave / HPW;
   const int lane = threadIdx.x & 63;
-  const int i = lane & 15;   // MFMA row/column index of this lane
-  const int g = lane >> 4;   // MFMA k-slot (lane group)
+  const int i = lane & 31;     // MFMA row / column index of this lane
+  const int half = lane >> 5;  // MFMA k-slot
   const int W = a.window;
-  const int off = it.klen - it.qlen;  // absolute position of query 0
-  const float sl2 = a.scale * kLog2e;
-
-  // This lane's query (column i of S^T) and its visible key range.
-  const int qi = it.q0 + qb * 16 + i;
-  const bool qvalid = qi < it.qlen;
-  const int qic = qvalid ? qi : it.qlen - 1;
-  const int aq = off + qic;
-  const int vis_lo = W > 0 ? max(0, aq - W + 1) : 0;
-  const int vis_hi = aq + 1;
-  // The wave's 16 queries: bounds of their visible ranges.
-  const int wq0 = it.q0 + qb * 16;
-  const bool wave_active = wq0 < it.qlen;
-  const int wq1 = min(wq0 + 15, it.qlen - 1);
-  const int wlo_min = W > 0 ? max(0, off + wq0 - W + 1) : 0;
-  const int wlo_max = W > 0 ? max(0, off + wq1 - W + 1) : 0;
-  const int whi_min = off + wq0 + 1;
-  const int whi_max = off + wq1 + 1;
-
-  // Q^T operand: lane (i, g) holds Q[query i][DQ*g + s], s < DQ, for the whole key loop.
-  // Read from a wave-uniform row base plus a 32-bit lane offset (queries past the sequence
-  // read its last one; a wave with none reads that one too).
-  float qr[DQ];
-  {
-    const int wq0c = min(wq0, it.qlen - 1);
-    const float *qw = a.q + ((size_t)(it.qstart + wq0c) * a.hq + h) * D;
-    const uint32_t lo = (uint32_t)(qic - wq0c) * (uint32_t)(a.hq * D) + (uint32_t)(DQ * g);
-#pragma unroll
-    for (int s = 0; s < DQ; s += 4) {
-      const float4 x = ld4(qw + lo + s);
-      qr[s] = x.x;
-      qr[s + 1] = x.y;
-      qr[s + 2] = x.z;
-      qr[s + 3] = x.w;
-    }
-  }
-
-  f32x4 o[NB];
-#pragma unroll
-  for (int b = 0; b < NB; b++) o[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  float m_run = -INFINITY;  // log2 units
-  float l_run = 0.0f;
-
+  // Scores are kept unscaled until the exponential; a negative scale goes into q's sign, so that
+  // the largest product is the largest score.
+  const float sl2 = fabsf(a.scale) * kLog2e;
+  const float qsign = a.scale < 0.0f ? -1.0f : 1.0f;
   const size_t rs = (size_t)a.hkv * D;
   const float *kbase = a.kv.k + (size_t)kvh * D;
   const float *vbase = a.kv.v + (size_t)kvh * D;
-  // Stage the chunk's block ids in LDS once, so the tile loads never wait on a global load.
-  int blk0 = 0;
-  if (a.kv.paged) {
-    const int bs = a.kv.block_size;
-    blk0 = it.ks / bs;
-    const int npages = (it.ke - 1) / bs - blk0 + 1;
-    const int32_t *table = a.kv.table + (size_t)it.seq * a.kv.bt_stride + blk0;
-    for (int j = threadIdx.x; j < npages; j += blockDim.x) stab[j] = table[j];
+  const float one = opaque_one();
+
+  for (int seg = a.seg_off[slot]; seg < seg_end; seg++) {
+    // Every wave is done with the previous segment's LDS tiles and table before they are reused.
     __syncthreads();
-  }
-  // Load instruction gi copies chunks [64 gi, 64 gi + 64) of the tile in row-major order (a
-  // whole number of rows for d <= 256, half a row at d = 512): lane l takes chunk q = 64 gi + l,
-  // i.e. position q % C4 of tile row q / C4.
-  const int lrow = C4 <= 64 ? lane / C4 : 0;  // rows within one instruction (d <= 256)
-  const int lpos = C4 <= 64 ? lane - lrow * C4 : 0;
-  int cur_page = -1;  // page whose block id cur_id holds (wave-uniform)
-  int cur_id = 0;
-  auto issue_tile = [&](int kt, float *dk, float *dv) {
-    // A full tile inside one page (or of dense rows): one uniform row base, fixed offsets
-    // (32-bit: the tile's rows must span less than 2 GiB).
-    if (kt + KT <= it.ke && rs < (size_t)(1 << 22) &&
-        (!a.kv.paged || (a.kv.bs_shift >= 0 && (kt >> a.kv.bs_shift) ==
-                                                   ((kt + KT - 1) >> a.kv.bs_shift)))) {
-      int64_t row0;
-      if (!a.kv.paged) {
-        row0 = (int64_t)it.kbase + kt;
-      } else {
-        const int pg = kt >> a.kv.bs_shift;
-        if (pg != cur_page) {
-          cur_id = __builtin_amdgcn_readfirstlane(stab[pg - blk0]);
-          cur_page = pg;
+    const TileItem it = a.items[seg];
+    const int off = it.klen - it.qlen;  // absolute position of query 0
+    // This lane's query (column i of S^T) and its visible key range.
+    const int wq0 = it.q0 + qb * QW;
+    const int qi = wq0 + i;
+    const bool qvalid = qi < it.qlen;
+    const int qic = qvalid ? qi : it.qlen - 1;
+    const int aq = off + qic;
+    const int vis_lo = W > 0 ? max(0, aq - W + 1) : 0;
+    const int vis_hi = aq + 1;
+    // The wave's 32 queries: bounds of their visible ranges.
+    const bool wave_active = wq0 < it.qlen;
+    const int wq1 = min(wq0 + QW - 1, it.qlen - 1);
+    const int wlo_min = W > 0 ? max(0, off + wq0 - W + 1) : 0;
+    const int wlo_max = W > 0 ? max(0, off + wq1 - W + 1) : 0;
+    const int whi_min = off + wq0 + 1;
+    const int whi_max = off + wq1 + 1;
+
+    // The first tile's loads are issued before Q is read: a short segment waits once for both.
+    TileShare<D, NW> share{a.kv, kbase, vbase, rs, stab, stage_table(a, it, stab), it.kbase, it.ke,
+                           wave, lane, -1, 0};
+    f32x8 rk[UW], rv[UW];  // this wave's share of the next tile, as loaded
+    auto load_tile = [&](int kt) {
+      share.load_k(kt, rk);
+      share.load_v(kt, rv);
+    };
+    load_tile(it.ks);
+
+    // Q^T operand: lane (i, half) holds the parts of Q[query i][16 s + 8 half + 0..7] for the
+    // whole key loop (queries past the sequence read its last one).
+    Split8 q[KS];
+    float qscale;  // takes a product of scaled q and k (of exponent 0) to log2 units
+    {
+      const float *qp = a.q + ((size_t)(it.qstart + qic) * a.hq + h) * D + 8 * half;
+      f32x8 x[KS];
+      float mx = 0.0f;
+#pragma unroll
+      for (int s = 0; s < KS; s++) {
+        const float4 u = ld4(qp + 16 * s), v = ld4(qp + 16 * s + 4);
+        x[s] = f32x8{u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+        mx = abs_max(mx, x[s]);
+      }
+      const int e = split_exp(max_halves(mx));
+#pragma unroll
+      for (int s = 0; s < KS; s++) q[s] = split8(x[s], qsign * split_scale(e));
+      qscale = sl2 * split_unscale(e);
+    }
+    f32x16 o[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) o[b][r] = 0.0f;
+    float m_run = -INFINITY;  // log2 units
+    float l_run = 0.0f;
+    int o_exp = kMinExp;  // exponent of the V scale that o is in
+    bool coarse = false;  // the split's steps show in this query's result
+
+    // The tile in rk / rv: each wave's largest magnitudes, then (after a barrier) the exponents of
+    // its scales, and its parts in LDS.
+    auto share_max = [&](int b) {
+      const float m = max_waves(share.largest(rk), share.largest(rv));
+      if (i == 0) smax[b][half][wave] = m;
+    };
+    int k_exp_in = kMinExp, v_exp_in = kMinExp, v_exp_max = kMinExp;
+    auto take_scales = [&](int b) {
+      const TileExps sc = tile_exps<NW>(smax[b][half][lane & (NW - 1)]);
+      k_exp_in = sc.a;
+      v_exp_max = max(v_exp_max, sc.b);
+      v_exp_in = max(sc.b, v_exp_max - kVExpSpan);
+    };
+    auto store_tile = [&](int b) {
+      share.store_k(rk, split_scale(k_exp_in), sk[b]);
+      share.store_v(rv, split_scale(v_exp_in), sv[b]);
+    };
+    auto read_split = [&](const _Float16 *p) {
+      return Split8{*reinterpret_cast<const f16x8 *>(p),
+                    *reinterpret_cast<const f16x8 *>(p + PART)};
+    };
+
+    // k_exp, v_exp: the tile's; v_max: the largest of the segment up to it, v_max >= v_exp.
+    // The next tile (in rk / rv) is split and stored to buffer nb among the products of QK, and
+    // the one after it loaded (next_kt; none if < 0).
+    auto compute_tile = [&](int kt, const _Float16 *tk, const _Float16 *tv, int k_exp, int v_exp,
+                            int v_max, int nb, int next_kt) {
+      if (!wave_active || kt >= whi_max || kt + KT <= wlo_min) {
+        store_tile(nb);
+        if (next_kt >= 0) load_tile(next_kt);
+        return;
+      }
+      const bool full = (kt + KT <= whi_min) && (kt >= wlo_max);
+
+      // S^T = K Q^T: register r of st holds key kt + 8 (r / 4) + 4 half + r % 4 of query i.
+      f32x16 st;
+#pragma unroll
+      for (int r = 0; r < 16; r++) st[r] = 0.0f;
+      // Operands are read kAhead steps before their products (the compiler would read each right
+      // before its use and wait out the LDS latency every time).
+      Split8 f[kAhead + 1];
+      auto read_k = [&](int s) { return read_split(tk + k_pos<D>(i, 2 * s + half)); };
+      auto read_v = [&](int u) {
+        return read_split(tv + part_pos(32 * (u % NB) + i, 2 * (u / NB) + half));
+      };
+#pragma unroll
+      for (int s = 0; s < kAhead; s++) f[s] = read_k(s);
+#pragma unroll
+      for (int s = 0; s < KS; s++) {
+        if (s + kAhead < KS) f[(s + kAhead) % (kAhead + 1)] = read_k(s + kAhead);
+        __builtin_amdgcn_sched_barrier(kKeepReads);
+        st = mfma_split(f[s % (kAhead + 1)], q[s], st);
+      }
+#pragma unroll
+      for (int u = 0; u < kAhead; u++) f[u] = read_v(u);
+      __builtin_amdgcn_sched_barrier(kKeepReads);
+      store_tile(nb);
+      if (next_kt >= 0) load_tile(next_kt);
+
+      if (!full) {
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int key = kt + 8 * (r >> 2) + 4 * half + (r & 3);
+          st[r] = (key >= vis_lo && key < vis_hi) ? st[r] : -INFINITY;
         }
-        row0 = (int64_t)cur_id * a.kv.block_size + (kt - (pg << a.kv.bs_shift));
       }
-      const int tile_bytes = KT * (int)rs * 4;
-      const float *gk0 = kbase + row0 * (int64_t)rs;
-      const float *gv0 = vbase + row0 * (int64_t)rs;
+      float mx = -INFINITY;
 #pragma unroll
-      for (int p = 0; p < LPW; p++) {
-        const int gi = p * NW + wave;
-        copy16_to_lds(gk0, tile_bytes, koff[p], dk + gi * 256);
-        copy16_to_lds(gv0, tile_bytes, voff[p], dv + gi * 256);
+      for (int r = 0; r < 16; r++) mx = fmaxf(mx, st[r]);
+      const float c = fmaxf(qscale * split_unscale(k_exp), 0x1p-126f);  // 0 * -inf is NaN
+      coarse |= c > kMaxScoreUnit;
+      mx = max_halves(mx) * c;
+      const bool need = mx > m_run + kLazyRescale;
+      if (__any(need)) {
+        const float mn = need ? mx : m_run;
+        const float alpha = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - mn);
+        l_run *= alpha;
+#pragma unroll
+        for (int b = 0; b < NB; b++) o[b] *= alpha;
+        m_run = mn;
       }
-      return;
-    }
-    // Last (partial) tile, or one that crosses a page: per-row addresses, rows past the chunk
-    // clamped to its last key.
+      if (v_max != o_exp) {
+        const float alpha = __uint_as_float((uint32_t)max(0, 127 + o_exp - v_max) << 23);
 #pragma unroll
-    for (int p = 0; p < LPW; p++) {
-      const int gi = p * NW + wave;
-      int r, pos;
-      if constexpr (C4 <= 64) {
-        r = gi * (64 / C4) + lrow;
-        pos = lpos;
-      } else {
-        const int q = gi * 64 + lane;
-        r = q / C4;
-        pos = q - r * C4;
+        for (int b = 0; b < NB; b++) o[b] *= alpha;
+        o_exp = v_max;
       }
-      const int key = min(kt + r, it.ke - 1);  // rows past the chunk are loaded but masked
-      const int64_t row = tile_row(a.kv, stab, blk0, it.kbase, key);
-      // K chunks are XOR-swizzled (kswz) for the column reads of QK; V rows are read
-      // along the row, which is conflict-free unswizzled.
-      const float *gk = kbase + row * rs + kswz<D>(pos, r) * 4;
-      const float *gv = vbase + row * rs + pos * 4;
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void *)gk,
-          (__attribute__((address_space(3))) void *)(dk + gi * 256), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void *)gv,
-          (__attribute__((address_space(3))) void *)(dv + gi * 256), 16, 0, 0);
-    }
-  };
-
-  auto compute_tile = [&](int kt, const float *sk, const float *sv) {
-    if (!wave_active || kt >= whi_max || kt + KT <= wlo_min) return;
-    const bool full = (kt + KT <= whi_min) && (kt >= wlo_max);
-
-    // S^T = K Q^T per 16-key block kb: A[key][k] = K[16kb + i][DQ*g + s] (lane i, g),
-    // B[k][query] = qr[s].  Chunk c = (DQ/4)*g + j of row 16kb+i sits at kswz(c, i).  Chunk
-    // j of every block is read at once, so each LDS wait is followed by 4 * KB MFMAs that
-    // alternate between the blocks' accumulators.
-    f32x4 st[KB];
+      const int p_exp = kProbExp + v_exp - v_max;
+      const float ms = (m_run == -INFINITY ? 0.0f : m_run) - (float)p_exp;
+      Split8 p[2];
+      float lt[2];
 #pragma unroll
-    for (int blk = 0; blk < KB; blk++) st[blk] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const float *kb[DQ / 4];
+      for (int s = 0; s < 2; s++) {
+        f32x8 e;
 #pragma unroll
-    for (int j = 0; j < DQ / 4; j++) kb[j] = sk + i * D + 4 * kswz<D>((DQ / 4) * g + j, i);
-#pragma unroll
-    for (int s = 0; s < DQ; s += 4) {
-      float4 kk[KB];
-#pragma unroll
-      for (int blk = 0; blk < KB; blk++) kk[blk] = ld4(kb[s >> 2] + blk * 16 * D);
-#pragma unroll
-      for (int blk = 0; blk < KB; blk++)
-        st[blk] = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[blk].x, qr[s], st[blk], 0, 0, 0);
-#pragma unroll
-      for (int blk = 0; blk < KB; blk++)
-        st[blk] = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[blk].y, qr[s + 1], st[blk], 0, 0, 0);
-#pragma unroll
-      for (int blk = 0; blk < KB; blk++)
-        st[blk] = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[blk].z, qr[s + 2], st[blk], 0, 0, 0);
-#pragma unroll
-      for (int blk = 0; blk < KB; blk++)
-        st[blk] = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[blk].w, qr[s + 3], st[blk], 0, 0, 0);
-    }
-
-    // p[4*blk + v] holds key kt + 16*blk + 4*g + v for query i (log2-scaled).
-    float p[4 * KB];
-    float mx = -INFINITY;
-#pragma unroll
-    for (int blk = 0; blk < KB; blk++)
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        float x = st[blk][v] * sl2;
-        if (!full) {
-          const int key = kt + 16 * blk + 4 * g + v;
-          x = (key >= vis_lo && key < vis_hi) ? x : -INFINITY;
-        }
-        p[4 * blk + v] = x;
-        mx = fmaxf(mx, x);
+        for (int j = 0; j < 8; j++) e[j] = __builtin_amdgcn_exp2f(fmaf(st[8 * s + j], c, -ms));
+        lt[s] = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+        p[s] = split8_unscaled(e, one);
       }
-    mx = max4_lanes(mx);
-    const bool need = mx > m_run + kLazyRescale;
-    if (__any(need)) {
-      const float mn = need ? mx : m_run;
-      const float alpha = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - mn);
-      l_run *= alpha;
-#pragma unroll
-      for (int b = 0; b < NB; b++) o[b] *= alpha;
-      m_run = mn;
-    }
-    const float ms = m_run == -INFINITY ? 0.0f : m_run;
-#pragma unroll
-    for (int s = 0; s < 4 * KB; s++) {
-      p[s] = __builtin_amdgcn_exp2f(p[s] - ms);
-      l_run += p[s];
-    }
+      // One addition to the long sum per tile, without the probabilities' scale.
+      l_run = fmaf(lt[0] + lt[1], __uint_as_float((uint32_t)(127 - p_exp) << 23), l_run);
 
-    // O^T += V^T P^T: step s contracts key 16*(s/4) + 4*g + s%4 (= p[s] in this lane).  The A
-    // operand of block 4*hh + bb is V[key][64*hh + 4*i + bb], one ds_read_b128 per hh.
-    const float *vrow = sv + 4 * g * D + 4 * i;
+      // O^T += V^T P^T, 16 keys a step (V chunk 2 s + half holds the lane's keys).
 #pragma unroll
-    for (int s = 0; s < 4 * KB; s++) {
-      const float *vp = vrow + (16 * (s >> 2) + (s & 3)) * D;
-#pragma unroll
-      for (int hh = 0; hh < H64; hh++) {
-        const float4 vv = ld4(vp + 64 * hh);
-        o[4 * hh + 0] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.x, p[s], o[4 * hh + 0], 0, 0, 0);
-        o[4 * hh + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.y, p[s], o[4 * hh + 1], 0, 0, 0);
-        o[4 * hh + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.z, p[s], o[4 * hh + 2], 0, 0, 0);
-        o[4 * hh + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.w, p[s], o[4 * hh + 3], 0, 0, 0);
+      for (int u = 0; u < 2 * NB; u++) {
+        if (u + kAhead < 2 * NB) f[(u + kAhead) % (kAhead + 1)] = read_v(u + kAhead);
+        __builtin_amdgcn_sched_barrier(kKeepReads);
+        o[u % NB] = mfma_split(f[u % (kAhead + 1)], p[u / NB], o[u % NB]);
       }
-    }
-  };
+    };
 
-  // Double-buffered key loop with one barrier per tile: at the barrier of tile t every wave
-  // has finished tile t-1 (so its buffer can be refilled with tile t+1) and tile t has landed.
-  const int ntiles = (it.ke - it.ks + KT - 1) / KT;
-  issue_tile(it.ks, sk0, sv0);
-  for (int t = 0; t < ntiles; t += 2) {
-    const int kt = it.ks + t * KT;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's copies of tile t landed
+    // At the barrier of tile t every wave is done with tile t - 1, whose buffer takes tile
+    // t + 1, tile t is in LDS, and so are the largest magnitudes of tile t + 1.
+    const int ntiles = (it.ke - it.ks + KT - 1) / KT;
+    share_max(0);
     __syncthreads();
-    if (t + 1 < ntiles) issue_tile(kt + KT, sk1, sv1);
-    compute_tile(kt, sk0, sv0);
-    if (t + 1 >= ntiles) break;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (t + 2 < ntiles) issue_tile(kt + 2 * KT, sk0, sv0);
-    compute_tile(kt + KT, sk1, sv1);
-  }
+    take_scales(0);
+    store_tile(0);
+    if (ntiles > 1) load_tile(it.ks + KT);
+    for (int t = 0; t < ntiles; t++) {
+      const int kt = it.ks + t * KT;
+      const int b = t & 1;
+      const int k_exp = k_exp_in, v_exp = v_exp_in, v_max = v_exp_max;
+      share_max(b ^ 1);  // the last tile stores itself once more, where nothing reads it
+      __syncthreads();
+      take_scales(b ^ 1);
+      compute_tile(kt, sk[b], sv[b], k_exp, v_exp, v_max, b ^ 1, t + 2 < ntiles ? kt + 2 * KT : -1);
+    }
 
-  const float l_tot = sum4_lanes(l_run);
-  if (!qvalid || !wave_active) continue;
-  // Lane (i, g) holds O^T rows r = 4g + v of every block: dims 64*hh + 4r + bb.
-  float *op;
-  float inv = 1.0f;
-  const bool partial = it.part >= 0;
-  size_t pidx = 0;
-  if (!partial) {
-    inv = l_tot == 0.0f ? 0.0f : 1.0f / l_tot;
-    op = a.out + ((size_t)(it.qstart + qi) * a.hq + h) * D;
-  } else {
-    // Partial of one key chunk: rows of the tile are laid out query-major, chunk-minor.
-    pidx = ((size_t)it.part + (size_t)(qi - it.q0) * it.nsplit + it.split) * a.hq + h;
-    op = a.part_acc + pidx * D;
-  }
+    if (!wave_active) continue;
+    const float l_tot = sum_halves(l_run);
+    if (__any(coarse || unsound<NB>(o, l_tot, o_exp))) {
+      scan_segment<D, 1>(a, it, stab, share.blk0, kvh, h, wq0);
+      continue;
+    }
+    if (!qvalid) continue;
+    const Dest d = destination(a, it, qi, h, D);
+    const float inv = d.partial ? 1.0f : (l_tot == 0.0f ? 0.0f : 1.0f / l_tot);
+    const float vs = split_unscale(o_exp - kProbExp);
+    // Register r of o[b] is dim 32 b + 8 (r / 4) + 4 half + r % 4.
 #pragma unroll
-  for (int v = 0; v < 4; v++) {
-    const int r = 4 * g + v;
+    for (int b = 0; b < NB; b++)
 #pragma unroll
-    for (int hh = 0; hh < H64; hh++)
-      st4(op + 64 * hh + 4 * r, make_float4(o[4 * hh][v] * inv, o[4 * hh + 1][v] * inv,
-                                          o[4 * hh + 2][v] * inv, o[4 * hh + 3][v] * inv));
+      for (int r = 0; r < 16; r += 4)
+        *reinterpret_cast<float4 *>(d.row + 32 * b + 2 * r + 4 * half) =
+            make_float4(o[b][r] * vs * inv, o[b][r + 1] * vs * inv, o[b][r + 2] * vs * inv,
+                        o[b][r + 3] * vs * inv);
+    if (d.partial && half == 0) {
+      a.part_m[d.pidx] = m_run;
+      a.part_l[d.pidx] = l_tot;
+    }
   }
-  if (partial && g == 0) {
-    a.part_m[pidx] = m_run;
-    a.part_l[pidx] = l_tot;
-  }
-  }  // segments
 }
 
-// Head dim 512 (Gemma 4 global layers) with the head split over a wave pair: one 8-wave
-// workgroup per CU, waves w and w + 4 own the same 16 queries and the dims [256 h, 256 h + 256)
-// of half h = w / 4.  Each wave forms the partial S^T of its half (64 MFMAs per 16-key tile),
-// the pair adds the two partials through LDS in a fixed order (S = S_0 + S_1 in both waves, so
-// both hold the same scores and run the same softmax) and each accumulates O^T for its own
-// 256 dims.  Q and O take 64 registers each instead of 128, so two waves fit per SIMD and
-// one covers the other's LDS waits (one 256-dim wave per SIMD left the matrix pipe idle for
-// every LDS read).  Every wave executes the exchange barrier of every tile, active or not.
-template <int HPW>
+// Head dims 256 and 512: the dims of 32 queries are split over DS = D / 128 waves, which keeps a
+// wave's Q, O and operand registers at those of d = 128 and eight waves (two per SIMD) on a CU.
+// Each wave contracts its 128 dims of QK; the partial S^T meet in LDS and are added in a fixed
+// order (S_0 + S_1, or (S_0 + S_1) + (S_2 + S_3)), so the DS waves hold the same scores, run the
+// same softmax and accumulate their own 128 dims of O^T.
+//
+// One LDS buffer for K and one for V, each refilled while the other is in use: V of tile t is
+// split and stored during QK of tile t, K of tile t + 1 during PV of tile t.  At d = 512 the
+// tiles take 128 KB, so the partial scores are added pairwise in place (16 KB instead of 32),
+// which costs one more barrier.
+template <int D, int HPW>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
-prefill512_kernel(TileLaunch a) {
-  constexpr int D = 512, DH = 256, KT = 16, NW = 8;
-  constexpr int DQ = DH / 4;         // QK steps per lane group: dims DH*half + DQ*g + [0, DQ)
-  constexpr int NB = DH / 16;        // O^T blocks of the half: block 4*hh+bb, dims 64*hh+4r+bb
-  constexpr int H64 = DH / 64;
-  constexpr int C4 = D / 4;          // 16-byte chunks per K/V row
-  constexpr int NI = KT * C4 / 64;   // load instructions per tensor per tile
-  constexpr int LPW = NI / NW;
-  constexpr int TILE = KT * D;
-  static_assert(HPW == 1, "one query head per workgroup");
-  static_assert(LPW >= 1 && NI % NW == 0, "tile does not split evenly over the waves");
-  __shared__ __attribute__((aligned(16))) float sk0[TILE];
-  __shared__ __attribute__((aligned(16))) float sv0[TILE];
-  __shared__ __attribute__((aligned(16))) float sk1[TILE];
-  __shared__ __attribute__((aligned(16))) float sv1[TILE];
-  __shared__ f32x4 spart[NW][64];  // each wave's partial S^T of the current tile
-  __shared__ int32_t stab[kTablePages];
+prefill_split_wide_kernel(TileLaunch a) {
+  constexpr int NW = 8, DW = 128, DS = D / DW;
+  constexpr int KS = DW / 16, NB = DW / 32;
+  constexpr int PART = KT * D;
+  constexpr int UW = TileShare<D, NW>::UW;
+  constexpr int SLOTS = DS == 2 ? NW : NW / 2;
+  static_assert(DS == 2 || DS == 4, "two or four waves share a query group");
+  __shared__ __attribute__((aligned(16))) _Float16 sk[2 * PART], sv[2 * PART];
+  __shared__ __attribute__((aligned(16))) float spart[SLOTS][4][64][4];  // partial S^T
+  __shared__ float smax[2][NW];  // each wave's largest |k| (of the next tile), |v|
+  __shared__ int32_t stab[kPrefillTablePages];
 
   const int slot = blockIdx.x;
   const int seg_end = a.seg_off[slot + 1];
-  for (int seg = a.seg_off[slot]; seg < seg_end; seg++) {
-  __syncthreads();
-  const TileItem it = a.items[seg];
   const int rep = a.hq / a.hkv;
-  const int kvh = blockIdx.y / rep;
+  const int groups = rep / HPW;
+  const int kvh = blockIdx.y / groups;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int h = blockIdx.y;  // one head per workgroup: grid y runs over the query heads
-  const int half = wave >> 2;
-  const int qb = wave & 3;
+  const int ds = wave % DS, qg = wave / DS;  // dims [128 ds, 128 ds + 128) of query group qg
+  const int h = kvh * rep + (blockIdx.y - kvh * groups) * HPW + qg % HPW;
+  const int qb = qg / HPW;
   const int lane = threadIdx.x & 63;
-  const int i = lane & 15;
-  const int g = lane >> 4;
+  const int i = lane & 31, half = lane >> 5;
   const int W = a.window;
-  const int off = it.klen - it.qlen;
-  const float sl2 = a.scale * kLog2e;
-
-  const int qi = it.q0 + qb * 16 + i;
-  const bool qvalid = qi < it.qlen;
-  const int qic = qvalid ? qi : it.qlen - 1;
-  const int aq = off + qic;
-  const int vis_lo = W > 0 ? max(0, aq - W + 1) : 0;
-  const int vis_hi = aq + 1;
-  const int wq0 = it.q0 + qb * 16;
-  const bool wave_active = wq0 < it.qlen;
-  const int wq1 = min(wq0 + 15, it.qlen - 1);
-  const int wlo_min = W > 0 ? max(0, off + wq0 - W + 1) : 0;
-  const int wlo_max = W > 0 ? max(0, off + wq1 - W + 1) : 0;
-  const int whi_min = off + wq0 + 1;
-  const int whi_max = off + wq1 + 1;
-
-  float qr[DQ];
-  {
-    const float *qp = a.q + ((size_t)(it.qstart + qic) * a.hq + h) * D + DH * half + DQ * g;
-#pragma unroll
-    for (int s = 0; s < DQ; s += 4) {
-      const float4 x = ld4(qp + s);
-      qr[s] = x.x;
-      qr[s + 1] = x.y;
-      qr[s + 2] = x.z;
-      qr[s + 3] = x.w;
-    }
-  }
-  f32x4 o[NB];
-#pragma unroll
-  for (int b = 0; b < NB; b++) o[b] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  float m_run = -INFINITY;
-  float l_run = 0.0f;
-
+  // Scores are kept unscaled until the exponential; a negative scale goes into q's sign.  (Not 0:
+  // 0 * -inf is NaN.)
+  const float sl2 = fmaxf(fabsf(a.scale) * kLog2e, 0x1p-126f);
+  const float qsign = a.scale < 0.0f ? -1.0f : 1.0f;
   const size_t rs = (size_t)a.hkv * D;
-  const float *kbase = a.kv.k + (size_t)kvh * D;
-  const float *vbase = a.kv.v + (size_t)kvh * D;
-  int blk0 = 0;
-  if (a.kv.paged) {
-    const int bs = a.kv.block_size;
-    blk0 = it.ks / bs;
-    const int npages = (it.ke - 1) / bs - blk0 + 1;
-    const int32_t *table = a.kv.table + (size_t)it.seq * a.kv.bt_stride + blk0;
-    for (int j = threadIdx.x; j < npages; j += blockDim.x) stab[j] = table[j];
-    __syncthreads();
-  }
-  auto issue_tile = [&](int kt, float *dk, float *dv) {
-#pragma unroll
-    for (int p = 0; p < LPW; p++) {
-      const int gi = p * NW + wave;
-      const int q = gi * 64 + lane;
-      const int r = q / C4;
-      const int pos = q - r * C4;
-      const int key = min(kt + r, it.ke - 1);
-      const int64_t row = tile_row(a.kv, stab, blk0, it.kbase, key);
-      const float *gk = kbase + row * rs + kswz<D>(pos, r) * 4;
-      const float *gv = vbase + row * rs + pos * 4;
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void *)gk,
-          (__attribute__((address_space(3))) void *)(dk + gi * 256), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds(
-          (const __attribute__((address_space(1))) void *)gv,
-          (__attribute__((address_space(3))) void *)(dv + gi * 256), 16, 0, 0);
-    }
-  };
+  const float one = opaque_one();
 
-  auto compute_tile = [&](int kt, const float *sk, const float *sv) {
-    const bool active = wave_active && kt < whi_max && kt + KT > wlo_min;
-    f32x4 st = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    if (active) {
-      // Partial S^T over this half: A[key][k] = K[i][DH*half + DQ*g + s], chunk
-      // 64*half + 16*g + s/4 of row i, at kswz(chunk, i).
-      const float *kr = sk + i * D;
+  for (int seg = a.seg_off[slot]; seg < seg_end; seg++) {
+    __syncthreads();
+    const TileItem it = a.items[seg];
+    const int off = it.klen - it.qlen;
+    const int wq0 = it.q0 + qb * QW;
+    const int qi = wq0 + i;
+    const bool qvalid = qi < it.qlen;
+    const int qic = qvalid ? qi : it.qlen - 1;
+    const int aq = off + qic;
+    const int vis_lo = W > 0 ? max(0, aq - W + 1) : 0;
+    const int vis_hi = aq + 1;
+    const bool group_active = wq0 < it.qlen;
+    const int wq1 = min(wq0 + QW - 1, it.qlen - 1);
+    const int wlo_min = W > 0 ? max(0, off + wq0 - W + 1) : 0;
+    const int wlo_max = W > 0 ? max(0, off + wq1 - W + 1) : 0;
+    const int whi_min = off + wq0 + 1;
+    const int whi_max = off + wq1 + 1;
+
+    // The first tile's loads are issued before Q is read: a short segment waits once for both.
+    TileShare<D, NW> share{a.kv, a.kv.k + (size_t)kvh * D, a.kv.v + (size_t)kvh * D, rs, stab,
+                           stage_table(a, it, stab), it.kbase, it.ke, wave, lane, -1, 0};
+    f32x8 rk[UW], rv[UW];
+    share.load_k(it.ks, rk);
+    share.load_v(it.ks, rv);
+
+    Split8 q[KS];  // lane (i, half): the parts of Q[query i][128 ds + 16 s + 8 half + 0..7]
+    float qscale;
+    {
+      const float *qp = a.q + ((size_t)(it.qstart + qic) * a.hq + h) * D + DW * ds + 8 * half;
+      f32x8 x[KS];
+      float mx = 0.0f;
 #pragma unroll
-      for (int s = 0; s < DQ; s += 4) {
-        const float4 kk = ld4(kr + 4 * kswz<D>(64 * half + 16 * g + (s >> 2), i));
-        st = __builtin_amdgcn_mfma_f32_16x16x4f32(kk.x, qr[s], st, 0, 0, 0);
-        st = __builtin_amdgcn_mfma_f32_16x16x4f32(kk.y, qr[s + 1], st, 0, 0, 0);
-        st = __builtin_amdgcn_mfma_f32_16x16x4f32(kk.z, qr[s + 2], st, 0, 0, 0);
-        st = __builtin_amdgcn_mfma_f32_16x16x4f32(kk.w, qr[s + 3], st, 0, 0, 0);
+      for (int s = 0; s < KS; s++) {
+        const float4 u = ld4(qp + 16 * s), v = ld4(qp + 16 * s + 4);
+        x[s] = f32x8{u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+        mx = abs_max(mx, x[s]);
       }
-      spart[wave][lane] = st;
-    }
-    __syncthreads();
-    if (!active) return;
-    const f32x4 other = spart[wave ^ 4][lane];
-    st = half == 0 ? st + other : other + st;  // S_0 + S_1 in both waves of the pair
-    const bool full = (kt + KT <= whi_min) && (kt >= wlo_max);
-
-    // p[v] holds key kt + 4*g + v for query i (log2-scaled).
-    float p[4];
-    float mx = -INFINITY;
+      const int e = split_exp(max_halves(mx));
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-      float x = st[v] * sl2;
-      if (!full) {
-        const int key = kt + 4 * g + v;
-        x = (key >= vis_lo && key < vis_hi) ? x : -INFINITY;
+      for (int s = 0; s < KS; s++) q[s] = split8(x[s], qsign * split_scale(e));
+      qscale = split_unscale(e);
+    }
+    f32x16 o[NB];
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) o[b][r] = 0.0f;
+    float m_run = -INFINITY;  // log2 units
+    float l_run = 0.0f;
+    int o_exp = kMinExp;  // exponent of the V scale that o is in
+    bool coarse = false;  // the split's steps show in this query's result
+
+    int k_exp_in = kMinExp, v_exp = kMinExp, v_max = kMinExp;
+    auto share_max = [&](int t, float m) {
+      const float x = max_waves(m, m);
+      if (lane == 0) smax[t][wave] = x;
+    };
+    auto store_k = [&]() {
+      const TileExps sc = tile_exps<NW>(smax[0][lane & 7]);
+      k_exp_in = sc.a;
+      share.store_k(rk, split_scale(sc.a), sk);
+    };
+    auto store_v = [&]() {
+      const TileExps sc = tile_exps<NW>(smax[1][lane & 7]);
+      v_max = max(v_max, sc.a);
+      v_exp = max(sc.a, v_max - kVExpSpan);
+      share.store_v(rv, split_scale(v_exp), sv);
+    };
+    auto read_split = [&](const _Float16 *p) {
+      return Split8{*reinterpret_cast<const f16x8 *>(p),
+                    *reinterpret_cast<const f16x8 *>(p + PART)};
+    };
+
+    const int ntiles = (it.ke - it.ks + KT - 1) / KT;
+    share_max(0, share.largest(rk));
+    share_max(1, share.largest(rv));
+    __syncthreads();
+    store_k();
+    if (ntiles > 1) share.load_k(it.ks + KT, rk);
+    __syncthreads();
+    for (int t = 0; t < ntiles; t++) {
+      const int kt = it.ks + t * KT;
+      const bool more = t + 1 < ntiles;
+      const bool active = group_active && kt < whi_max && kt + KT > wlo_min;
+      const float c = qscale * split_unscale(k_exp_in);
+
+      // K of tile t is in LDS; V of tile t is in rv, its maxima in smax[1]; PV of tile t - 1 is
+      // done everywhere.
+      store_v();
+      if (more) share.load_v(kt + KT, rv);
+      f32x16 st;
+#pragma unroll
+      for (int r = 0; r < 16; r++) st[r] = 0.0f;
+      if (active) {
+        auto read_k = [&](int s) {
+          return read_split(sk + k_pos<D>(i, (DW / 8) * ds + 2 * s + half));
+        };
+        Split8 f[kAhead + 1];
+#pragma unroll
+        for (int s = 0; s < kAhead; s++) f[s] = read_k(s);
+#pragma unroll
+        for (int s = 0; s < KS; s++) {
+          if (s + kAhead < KS) f[(s + kAhead) % (kAhead + 1)] = read_k(s + kAhead);
+          __builtin_amdgcn_sched_barrier(kKeepReads);
+          st = mfma_split(f[s % (kAhead + 1)], q[s], st);
+        }
+        coarse |= c * sl2 > kMaxScoreUnit;
+        st *= c;  // a power of two: the partial score in its own units
       }
-      p[v] = x;
-      mx = fmaxf(mx, x);
-    }
-    mx = max4_lanes(mx);
-    const bool need = mx > m_run + kLazyRescale;
-    if (__any(need)) {
-      const float mn = need ? mx : m_run;
-      const float alpha = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - mn);
-      l_run *= alpha;
+      auto put = [&](int sl) {
 #pragma unroll
-      for (int b = 0; b < NB; b++) o[b] *= alpha;
-      m_run = mn;
-    }
-    const float ms = m_run == -INFINITY ? 0.0f : m_run;
+        for (int r = 0; r < 16; r += 4)
+          *reinterpret_cast<float4 *>(spart[sl][r >> 2][lane]) =
+              make_float4(st[r], st[r + 1], st[r + 2], st[r + 3]);
+      };
+      auto get = [&](int sl) {
+        f32x16 x;
 #pragma unroll
-    for (int v = 0; v < 4; v++) {
-      p[v] = __builtin_amdgcn_exp2f(p[v] - ms);
-      l_run += p[v];
-    }
-
-    // O^T += V^T P^T over this half's dims: step s contracts key 4*g + s (= p[s] in this lane).
-    const float *vrow = sv + 4 * g * D + DH * half + 4 * i;
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-      const float *vp = vrow + s * D;
-#pragma unroll
-      for (int hh = 0; hh < H64; hh++) {
-        const float4 vv = ld4(vp + 64 * hh);
-        o[4 * hh + 0] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.x, p[s], o[4 * hh + 0], 0, 0, 0);
-        o[4 * hh + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.y, p[s], o[4 * hh + 1], 0, 0, 0);
-        o[4 * hh + 2] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.z, p[s], o[4 * hh + 2], 0, 0, 0);
-        o[4 * hh + 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv.w, p[s], o[4 * hh + 3], 0, 0, 0);
+        for (int r = 0; r < 16; r += 4) {
+          const float4 y = ld4(spart[sl][r >> 2][lane]);
+          x[r] = y.x, x[r + 1] = y.y, x[r + 2] = y.z, x[r + 3] = y.w;
+        }
+        return x;
+      };
+      if (more) share_max(0, share.largest(rk));
+      if constexpr (DS == 2) {
+        if (active) put(wave);
+        __syncthreads();
+        if (active) {
+          const f32x16 other = get(wave ^ 1);
+          st = st + other;
+        }
+      } else {
+        if (active && (ds & 1)) put(wave >> 1);
+        __syncthreads();
+        if (active && !(ds & 1)) {
+          st = st + get(wave >> 1);
+          put(wave >> 1);
+        }
+        __syncthreads();
+        if (active) {
+          const f32x16 lo = get(2 * qg), hi = get(2 * qg + 1);
+          st = lo + hi;
+        }
       }
+
+      // V of tile t is in LDS; QK of tile t is done everywhere, the maxima of K of tile t + 1 are
+      // in smax[0].
+      if (more) {
+        store_k();
+        if (t + 2 < ntiles) share.load_k(kt + 2 * KT, rk);
+      }
+      if (active) {
+        const bool full = (kt + KT <= whi_min) && (kt >= wlo_max);
+        if (!full) {
+#pragma unroll
+          for (int r = 0; r < 16; r++) {
+            const int key = kt + 8 * (r >> 2) + 4 * half + (r & 3);
+            st[r] = (key >= vis_lo && key < vis_hi) ? st[r] : -INFINITY;
+          }
+        }
+        float mx = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 16; r++) mx = fmaxf(mx, st[r]);
+        mx = max_halves(mx) * sl2;
+        const bool need = mx > m_run + kLazyRescale;
+        if (__any(need)) {
+          const float mn = need ? mx : m_run;
+          const float alpha = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - mn);
+          l_run *= alpha;
+#pragma unroll
+          for (int b = 0; b < NB; b++) o[b] *= alpha;
+          m_run = mn;
+        }
+        if (v_max != o_exp) {
+          const float alpha = __uint_as_float((uint32_t)max(0, 127 + o_exp - v_max) << 23);
+#pragma unroll
+          for (int b = 0; b < NB; b++) o[b] *= alpha;
+          o_exp = v_max;
+        }
+        const int p_exp = kProbExp + v_exp - v_max;
+        const float ms = (m_run == -INFINITY ? 0.0f : m_run) - (float)p_exp;
+        Split8 p[2];
+        float lt[2];
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          f32x8 e;
+#pragma unroll
+          for (int j = 0; j < 8; j++) e[j] = __builtin_amdgcn_exp2f(fmaf(st[8 * s + j], sl2, -ms));
+          lt[s] = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+          p[s] = split8_unscaled(e, one);
+        }
+        l_run = fmaf(lt[0] + lt[1], __uint_as_float((uint32_t)(127 - p_exp) << 23), l_run);
+        auto read_v = [&](int u) {
+          return read_split(sv + part_pos(DW * ds + 32 * (u % NB) + i, 2 * (u / NB) + half));
+        };
+        Split8 f[kAhead + 1];
+#pragma unroll
+        for (int u = 0; u < kAhead; u++) f[u] = read_v(u);
+#pragma unroll
+        for (int u = 0; u < 2 * NB; u++) {
+          if (u + kAhead < 2 * NB) f[(u + kAhead) % (kAhead + 1)] = read_v(u + kAhead);
+          __builtin_amdgcn_sched_barrier(kKeepReads);
+          o[u % NB] = mfma_split(f[u % (kAhead + 1)], p[u / NB], o[u % NB]);
+        }
+      }
+      if (more) share_max(1, share.largest(rv));
+      __syncthreads();
     }
-  };
 
-  const int ntiles = (it.ke - it.ks + KT - 1) / KT;
-  issue_tile(it.ks, sk0, sv0);
-  for (int t = 0; t < ntiles; t += 2) {
-    const int kt = it.ks + t * KT;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (t + 1 < ntiles) issue_tile(kt + KT, sk1, sv1);
-    compute_tile(kt, sk0, sv0);
-    if (t + 1 >= ntiles) break;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (t + 2 < ntiles) issue_tile(kt + 2 * KT, sk0, sv0);
-    compute_tile(kt + KT, sk1, sv1);
-  }
-
-  const float l_tot = sum4_lanes(l_run);
-  if (!qvalid || !wave_active) continue;
-  float *op;
-  float inv = 1.0f;
-  const bool partial = it.part >= 0;
-  size_t pidx = 0;
-  if (!partial) {
-    inv = l_tot == 0.0f ? 0.0f : 1.0f / l_tot;
-    op = a.out + ((size_t)(it.qstart + qi) * a.hq + h) * D + DH * half;
-  } else {
-    pidx = ((size_t)it.part + (size_t)(qi - it.q0) * it.nsplit + it.split) * a.hq + h;
-    op = a.part_acc + pidx * D + DH * half;
-  }
+    const float l_tot = sum_halves(l_run);
+    if (__syncthreads_or(coarse || unsound<NB>(o, l_tot, o_exp))) {
+      const int q0 = wq0 + ds * (QW / DS);
+      if (q0 < it.qlen) scan_segment<D, DS>(a, it, stab, share.blk0, kvh, h, q0);
+      continue;
+    }
+    if (!qvalid) continue;
+    const Dest d = destination(a, it, qi, h, D);
+    const float inv = d.partial ? 1.0f : (l_tot == 0.0f ? 0.0f : 1.0f / l_tot);
+    const float vs = split_unscale(o_exp - kProbExp);
 #pragma unroll
-  for (int v = 0; v < 4; v++) {
-    const int r = 4 * g + v;
+    for (int b = 0; b < NB; b++)
 #pragma unroll
-    for (int hh = 0; hh < H64; hh++)
-      st4(op + 64 * hh + 4 * r, make_float4(o[4 * hh][v] * inv, o[4 * hh + 1][v] * inv,
-                                          o[4 * hh + 2][v] * inv, o[4 * hh + 3][v] * inv));
+      for (int r = 0; r < 16; r += 4)
+        *reinterpret_cast<float4 *>(d.row + DW * ds + 32 * b + 2 * r + 4 * half) =
+            make_float4(o[b][r] * vs * inv, o[b][r + 1] * vs * inv, o[b][r + 2] * vs * inv,
+                        o[b][r + 3] * vs * inv);
+    if (d.partial && half == 0 && ds == 0) {
+      a.part_m[d.pidx] = m_run;
+      a.part_l[d.pidx] = l_tot;
+    }
   }
-  if (partial && g == 0 && half == 0) {
-    a.part_m[pidx] = m_run;
-    a.part_l[pidx] = l_tot;
-  }
-  }  // segments
 }
 
 namespace {
 
-// Keys per tile and waves per workgroup for head dim D.
 template <int D>
-constexpr int key_tile() {
-  return D == 512 ? 16 : 32;
+constexpr int split_waves() {
+  return D == 64 ? 4 : 8;
 }
-template <int D>
-constexpr int tile_waves() {
-  return 8;
-}
+// Waves that share 32 queries.
+constexpr int dim_waves(int head_dim) { return head_dim <= 128 ? 1 : head_dim / 128; }
 
-template <int D>
-hipError_t launch_prefill_d(const TileLaunch &a, int hpw, hipStream_t s) {
-  constexpr int KT = key_tile<D>(), NW = tile_waves<D>();
-  const dim3 grid(a.num_slots, a.hkv * ((a.hq / a.hkv) / hpw)), block(64 * NW);
-  switch (hpw) {
-    case 1: hipLaunchKernelGGL((prefill_kernel<D, 1, KT, NW>), grid, block, 0, s, a); break;
-    case 2: hipLaunchKernelGGL((prefill_kernel<D, 2, KT, NW>), grid, block, 0, s, a); break;
-    case 4:
-      if constexpr (NW >= 4) {
-        hipLaunchKernelGGL((prefill_kernel<D, 4, KT, NW>), grid, block, 0, s, a);
-        break;
-      }
-      return hipErrorInvalidValue;
-    case 8:
-      if constexpr (NW >= 8) {
-        hipLaunchKernelGGL((prefill_kernel<D, 8, KT, NW>), grid, block, 0, s, a);
-        break;
-      }
-      return hipErrorInvalidValue;
+// Calls f with the kernel for this head dim and number of query heads per workgroup.
+template <typename F>
+hipError_t with_kernel(int head_dim, int hpw, F f) {
+  switch (head_dim * 8 + hpw) {
+    case 64 * 8 + 1: return f(prefill_split_kernel<64, 1, split_waves<64>()>);
+    case 128 * 8 + 1: return f(prefill_split_kernel<128, 1, split_waves<128>()>);
+    case 128 * 8 + 2: return f(prefill_split_kernel<128, 2, split_waves<128>()>);
+    case 256 * 8 + 1: return f(prefill_split_wide_kernel<256, 1>);
+    case 256 * 8 + 2: return f(prefill_split_wide_kernel<256, 2>);
+    case 512 * 8 + 1: return f(prefill_split_wide_kernel<512, 1>);
     default: return hipErrorInvalidValue;
   }
-  return hipGetLastError();
 }
+
+int waves(int head_dim) { return head_dim == 64 ? split_waves<64>() : split_waves<128>(); }
 
 }  // namespace
 
-int prefill_waves(int head_dim) {
-  if (prefill_split_supports(head_dim)) return prefill_split_waves(head_dim);
-  return head_dim == 256 ? tile_waves<256>() : tile_waves<512>();
-}
-
-// At d = 512 a wave pair shares 16 queries (prefill512_kernel), one query head per workgroup;
-// otherwise each wave owns 16 queries and up to a quarter of the waves share a head group.
-int prefill_max_heads(int head_dim) {
-  return head_dim == 512 ? 1 : std::max(1, prefill_waves(head_dim) / 4);
-}
+// Most query heads one prefill workgroup carries at this head dim: a quarter of its waves.
+int prefill_max_heads(int head_dim) { return head_dim == 64 || head_dim == 512 ? 1 : 2; }
 
 int prefill_tile_queries(int head_dim, int heads_per_wg) {
-  if (prefill_split_supports(head_dim))
-    return kPrefillSplitQueries * (prefill_waves(head_dim) / heads_per_wg);
-  const int query_blocks = head_dim == 512 ? prefill_waves(head_dim) / 2 : prefill_waves(head_dim);
-  return 16 * (query_blocks / heads_per_wg);
+  return QW * (waves(head_dim) / dim_waves(head_dim) / heads_per_wg);
 }
 
 bool prefill_kernel_supports(int head_dim, int heads_per_wg) {
   return (head_dim == 64 || head_dim == 128 || head_dim == 256 || head_dim == 512) &&
-         (heads_per_wg == 1 || heads_per_wg == 2 || heads_per_wg == 4 || heads_per_wg == 8) &&
-         heads_per_wg <= prefill_max_heads(head_dim);
+         (heads_per_wg == 1 || heads_per_wg == 2) && heads_per_wg <= prefill_max_heads(head_dim);
 }
-
-namespace {
 
 // Uncached: the caller (one context per device) keeps the answer.  The query reads the
 // current device's properties, so the caller makes its device current first.
-template <int D, int HPW>
-int blocks_per_cu() {
-  constexpr int NW = tile_waves<D>();
+int prefill_blocks_per_cu(int head_dim, int heads_per_wg) {
   int b = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &b, prefill_kernel<D, HPW, key_tile<D>(), NW>, 64 * NW, 0) != hipSuccess ||
+  if (with_kernel(head_dim, heads_per_wg, [&](auto k) {
+        return hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, k, 64 * waves(head_dim), 0);
+      }) != hipSuccess ||
       b < 1)
     b = 1;
   return b;
 }
 
-template <int D>
-int blocks_per_cu_d(int hpw) {
-  constexpr int NW = tile_waves<D>();
-  switch (hpw) {
-    case 1: return blocks_per_cu<D, 1>();
-    case 2: return blocks_per_cu<D, 2>();
-    case 4: return blocks_per_cu<D, NW >= 4 ? 4 : 1>();
-    default: return blocks_per_cu<D, NW >= 8 ? 8 : 1>();
-  }
-}
-
-}  // namespace
-
-int prefill_blocks_per_cu(int head_dim, int heads_per_wg) {
-  if (prefill_split_supports(head_dim)) return prefill_split_blocks_per_cu(head_dim, heads_per_wg);
-  if (head_dim == 512) {
-    int b = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, prefill512_kernel<1>, 512, 0) !=
-            hipSuccess ||
-        b < 1)
-      b = 1;
-    return b;
-  }
-  return blocks_per_cu_d<256>(heads_per_wg);
-}
-
 hipError_t launch_prefill_tiles(const TileLaunch &a, int hpw, hipStream_t s) {
   if (a.num_items <= 0 || a.num_slots <= 0) return hipSuccess;
-  switch (a.head_dim) {
-    case 64:
-    case 128: return launch_prefill_split(a, hpw, s);
-    case 256: return launch_prefill_d<256>(a, hpw, s);
-    case 512:
-      if (hpw != 1) return hipErrorInvalidValue;
-      hipLaunchKernelGGL((prefill512_kernel<1>), dim3(a.num_slots, a.hq), dim3(512), 0, s, a);
-      return hipGetLastError();
-    default: return hipErrorInvalidValue;
-  }
+  const dim3 grid(a.num_slots, a.hkv * ((a.hq / a.hkv) / hpw)), block(64 * waves(a.head_dim));
+  return with_kernel(a.head_dim, hpw, [&](auto k) {
+    hipLaunchKernelGGL(k, grid, block, 0, s, a);
+    return hipGetLastError();
+  });
 }
 
 }  // namespace nva

@@ -11,9 +11,10 @@
 //
 // fp16 has five exponent bits, so operands are scaled by powers of two (exact): the largest
 // magnitude of a block goes to [2^14, 2^15), below fp16's 65504, and the smallest step of lo,
-// 2^-24, is then 2^-38 of that magnitude: every element that matters next to the block's
-// largest keeps all its bits.  Blocks with infinities, or whose parts lie too far apart for one
-// scale, are detected by the users of this file and handled on fp32 instructions.
+// 2^-24, is then 2^-38 of that magnitude.  The users of this file choose the blocks, or check
+// their results, so that this step stays below 2^-24 of what it is added to; infinities become
+// NaN in lo and so in the sums they enter, which the users detect.  Both are then taken again on
+// fp32 instructions.
 //
 // Three v_mfma_f32_32x32x16_f16 do the work of eight v_mfma_f32_32x32x2_f32 at half the cycles
 // each: 5.3 times the fp32 matrix rate.  (Three bf16 parts need no scale but six products: the
@@ -89,6 +90,18 @@ __device__ __forceinline__ float abs_max(float m, f32x8 x) {
   return m;
 }
 
+// Sum and max over lanes l and l ^ 32; both lanes get the same bits.
+__device__ __forceinline__ float sum_halves(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
+                                                  false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float max_halves(float x) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
+                                                  false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
 template <int CTRL>
 __device__ __forceinline__ uint32_t dpp(uint32_t x) {
   return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, CTRL, 0xf, 0xf, true);
@@ -112,27 +125,19 @@ __device__ __forceinline__ float max_waves(float a, float b) {
   return max_dpp<0x121>(y);
 }
 
-// Scales of a tile pair from its NW (4 or 8) waves' maxima: lanes 0-31 hold the first tensor's
-// (lane l that of wave l % NW), lanes 32-63 the second's.  A tile with an infinity, or whose
-// waves' maxima lie more than kShareSpan exponents apart (all-zero shares aside), does not fit
-// one scale: within the span the smallest share's smallest step is 2^-24 of its own largest.
-constexpr int kShareSpan = 14;
-struct TileScales {
-  int a, b;  // exponents (split_scale)
-  bool unfit;
+// Scale exponents of a tile pair from its NW (4 or 8) waves' maxima: lanes 0-31 hold the first
+// tensor's (lane l that of wave l % NW), lanes 32-63 the second's.
+struct TileExps {
+  int a, b;
 };
 template <int NW>
-__device__ __forceinline__ TileScales tile_scales(float largest) {
-  const uint32_t x = __float_as_uint(largest);
-  uint32_t hi = x, lo = x - 1;
-  hi = max(hi, dpp<0xB1>(hi)), lo = min(lo, dpp<0xB1>(lo));  // lanes ^ 1, ^ 2, then 8
-  hi = max(hi, dpp<0x4E>(hi)), lo = min(lo, dpp<0x4E>(lo));
-  if constexpr (NW == 8) hi = max(hi, dpp<0x141>(hi)), lo = min(lo, dpp<0x141>(lo));
-  const int e = (int)(hi >> 23);
-  const bool bad = e == 255 || e - (int)((lo + 1) >> 23) > kShareSpan;
-  const int es = e == 255 ? 141 : max(e, kMinExp);
-  return TileScales{__builtin_amdgcn_readlane(es, 0), __builtin_amdgcn_readlane(es, 32),
-                    __any(bad) != 0};
+__device__ __forceinline__ TileExps tile_exps(float largest) {
+  uint32_t m = __float_as_uint(largest);
+  m = max(m, dpp<0xB1>(m));  // lanes ^ 1, ^ 2, then 7 - lane
+  m = max(m, dpp<0x4E>(m));
+  if constexpr (NW == 8) m = max(m, dpp<0x141>(m));
+  const int e = split_exp(__uint_as_float(m));
+  return TileExps{__builtin_amdgcn_readlane(e, 0), __builtin_amdgcn_readlane(e, 32)};
 }
 
 // Offset (in fp16) of 16-byte chunk c (0..3) of row r of a part whose rows hold 32 values, a

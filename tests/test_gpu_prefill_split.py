@@ -1,14 +1,17 @@
 """Prefill on split fp16 operands at magnitudes where the split can go wrong.
 
-The kernel scales q per query and K / V per 32-key tile by powers of two and falls back to fp32
-instructions where one scale cannot hold a tile.  Each case is compared with the oracle row by
-row (rel-L2 of every query row of every head), so that a small row beside a large one counts by
-itself.  Bar: 1e-5, the attention bar; non-finite results must be the oracle's.  Both sides sum
-up to 230 products per score and per output in fp32 (sqrt(230) * 2^-24 = 9e-7 of their size),
-and a score of size s moves its weight by s times that; s stays below 10."""
+The kernel scales q per query and K / V per 32-key tile by powers of two and takes queries whose
+results are small beside their tiles again on fp32 instructions.  Each case is compared row by row
+(rel-L2 of every query row of every head), so that a small row beside a large one counts by itself:
+with float64 where the inputs are finite, with the oracle where they are not (non-finite results
+must be the oracle's).  Bar: 1e-5, the attention bar: up to 2100 fp32 products per output give
+sqrt(2100) * 2^-24 = 2.7e-6 of their size, a few times that where they cancel, and a score of size
+s < 10 moves its weight by s times its own error.  (The fp32 oracle itself is 2.0e-5 off on the
+long rows of unlike size.)"""
 
 import numpy as np
 import pytest
+import torch
 
 from cases import Case
 from gpu_checks import dev, load_arena, say
@@ -17,9 +20,12 @@ from nanollvm_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
 
+# The last sequence gives the step work enough for the split kernel (steps of short sequences run
+# on the fp32 one).  A window leaves few keys per query, so it takes more queries.
 SEQS = [(16, 70), (5, 33), (0, 2), (40, 190), (0, 31)]
 DENSE_SEQS = [(0, 70), (0, 33), (0, 2), (0, 190), (0, 31)]
-HEADS = [(64, 1), (64, 4), (128, 1), (128, 2)]
+LONG, LONG_WINDOW = [(0, 2100)], [(0, 6300)]
+HEADS = [(64, 1), (64, 4), (128, 1), (128, 2), (256, 1), (256, 4), (512, 1), (512, 2)]
 
 
 @pytest.fixture(scope="module")
@@ -32,12 +38,39 @@ def ctx():
 def build(d, rep, layout, window=0, scale=None, seed=0):
     rng = np.random.default_rng(seed + d + rep)
     paged = layout != "dense"
-    wl = W.build(f"split d{d} rep{rep} {layout} w{window}", SEQS if paged else DENSE_SEQS,
+    wl = W.build(f"split d{d} rep{rep} {layout} w{window}",
+                 (SEQS if paged else DENSE_SEQS) + (LONG_WINDOW if window else LONG),
                  is_prefill=True, hq=2 * rep, hkv=2, d=d,
                  scale=float(np.float32(scale if scale is not None else d ** -0.5)),
                  window=window, rng=rng, paged=paged,
-                 block_size=int(layout[5:]) if paged else 256)
+                 block_size=int(layout[5:]) if paged else 256, pool_cap=20000)
     return Case(wl, seed=seed)
+
+
+def exact(case, kc, vc):
+    """The step's attention in float64."""
+    wl, m = case.wl, case.wl.meta
+    rep = wl.hq // wl.hkv
+    out = np.zeros(case.q.shape)
+    for b, (c, n) in enumerate(wl.seqs):
+        q0 = int(m.cu_seqlens_q[b])
+        if wl.tables is None:
+            k, v = case.k[q0:q0 + n], case.v[q0:q0 + n]
+        else:
+            t = np.arange(c + n)
+            rows = np.asarray(wl.tables[b], np.int64)[t // wl.block_size] * wl.block_size
+            rows += t % wl.block_size
+            k, v = (x.reshape(-1, wl.hkv, wl.d)[rows] for x in (kc, vc))
+        k, v, q = (torch.from_numpy(x).cuda().double() for x in (k, v, case.q[q0:q0 + n]))
+        at = torch.arange(c, c + n, device="cuda")[:, None]
+        key = torch.arange(c + n, device="cuda")[None, :]
+        seen = (key <= at) & ((key > at - wl.window) if wl.window else True)
+        for h in range(wl.hq):
+            kt = k[:, h // rep].T.contiguous()
+            s = (q[:, h].contiguous() @ kt * wl.scale).masked_fill(~seen, -np.inf)
+            p = torch.softmax(s, dim=-1)
+            out[q0:q0 + n, h] = (p @ v[:, h // rep].contiguous()).cpu().numpy()
+    return out
 
 
 def check(ctx, case, name):
@@ -48,7 +81,7 @@ def check(ctx, case, name):
         ctx.set(**wl.meta.context_args())
         ctx.bind_kv_cache(arena)
         with np.errstate(all="ignore"):
-            want, _, _ = case.oracle(threads=8)
+            want, kc, vc = case.oracle(threads=8)
         out = Attention(wl.hq, wl.d, wl.scale, wl.hkv, wl.window, 0).forward(
             dev(case.q), dev(case.k), dev(case.v), ctx)
         ctx.sync()
@@ -56,7 +89,8 @@ def check(ctx, case, name):
     finally:
         ctx.clear()
         arena.close()
-    want = want.astype(np.float64)
+    finite = all(np.isfinite(x).all() for x in (case.q, case.k, case.v))
+    want = exact(case, kc, vc) if finite else want.astype(np.float64)
     odd = ~np.isfinite(want)
     assert np.array_equal(got[odd], want[odd], equal_nan=True), "non-finite results differ"
     assert np.all(np.isfinite(got[~odd])), "non-finite results where the oracle's are finite"
@@ -103,14 +137,16 @@ def test_rows_of_unlike_size(ctx, d, rep, layout):
 @pytest.mark.parametrize("layout", ["paged16", "dense"])
 @pytest.mark.parametrize("d,rep", HEADS)
 def test_rows_beyond_one_scale(ctx, d, rep, layout):
-    """One K row of 2^40 that every query weighs at 0, and one V row of 2^60 late in the same
-    tile: queries before it must keep the bits of their own small rows."""
+    """One K row of 2^40 that every query weighs at 0, one V row of 2^60 late in the same tile
+    (queries before it must keep the bits of their own rows) and a sequence whose first V row,
+    in the dense layout all that its first query sees, is 2^-40 beside its tile's others."""
     case = build(d, rep, layout, seed=4)
     first = int(case.wl.meta.cu_seqlens_q[3])
     case.q[:, :, 0] = np.abs(case.q[:, :, 0]) + 0.5
     case.k[first + 9] = 0.0
     case.k[first + 9, :, 0] = -2.0 ** 40
     case.v[first + 20] *= np.float32(2.0 ** 60)
+    case.v[0] *= np.float32(2.0 ** -40)
     check(ctx, case, f"beyond one scale d{d} rep{rep} {layout}")
 
 
@@ -135,5 +171,5 @@ def test_zeros_and_negative_scale(ctx, d, rep):
     case = build(d, rep, "dense", seed=7)
     case.k[:40] = 0.0
     case.v[20:90] = 0.0
-    case.q[60:] = 0.0
+    case.q[60:300] = 0.0
     check(ctx, case, f"zeros d{d} rep{rep}")
