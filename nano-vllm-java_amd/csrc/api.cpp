@@ -418,13 +418,15 @@ int largest_pow2_divisor_upto(int rep, int cap) {
 // the two kernels: the tiles' time scales as 1/f, while the rows, being HBM-bound, keep
 // 1 - f^1.8 of the whole chip's bandwidth.  That is below what the rows keep alone on the
 // remaining CUs of a CU-masked stream (85% on half of the CUs, 68% on 3/8, 49% on 1/4), since
-// beside tile workgroups they lose bandwidth too; for the Qwen3-4B-like mixed step it picks 160
-// CUs, the best of a sweep over 128..208.  Solo rates: rows 6.5 TB/s, tiles 100 / 80 / 70
-// TFLOP/s at head dim <= 128 / 256 / 512.
-int64_t mixed_tile_cus(int num_cus, double row_bytes, double tile_flops, int head_dim) {
+// beside tile workgroups they lose bandwidth too.  Rates: rows 6.5 TB/s, tiles 200 TFLOP/s at
+// head dim <= 128 (the fp32 tiles of small steps 100), 80 / 70 at 256 / 512.  The tile rate is
+// what the model fits best with, below the 330 that the tiles reach alone: four 512-token chunks
+// beside 64 rows of 4096-16384 keys at 32 q / 8 KV heads take 1040 us at 100, 1005 at 150, 955 at
+// 200, 988 at 250, 1020 at 350 and 1300 at 500.
+int64_t mixed_tile_cus(int num_cus, double row_bytes, double tile_flops, int head_dim, bool fp32) {
   const double tr = row_bytes / 6.5e12;
   const double tt =
-      tile_flops / (head_dim <= 128 ? 100e12 : head_dim <= 256 ? 80e12 : 70e12);
+      tile_flops / (head_dim <= 128 ? (fp32 ? 100e12 : 200e12) : head_dim <= 256 ? 80e12 : 70e12);
   int best_s = 8;
   double best = 1e300;
   for (int s = 1; s < 16; s++) {
@@ -579,7 +581,8 @@ nva_status get_plan(nva_ctx *ctx, const PlanKey &key, Plan **out) {
       }
       const double flops = 4.0 * key.head_dim * key.num_heads * pairs;
       resident = std::max<int64_t>(key.tile_groups,
-                                   mixed_tile_cus(ctx->num_cus, row_bytes, flops, key.head_dim));
+                                   mixed_tile_cus(ctx->num_cus, row_bytes, flops, key.head_dim,
+                                                key.fp32_tiles != 0));
     }
     slots = (int)std::max<int64_t>(1, std::min<int64_t>(total, resident / key.tile_groups));
     const int64_t page_cap =
