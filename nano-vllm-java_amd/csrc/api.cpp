@@ -2132,23 +2132,21 @@ nva_status nva_linear_forward(nva_ctx *ctx, const float *x, int rows, int in,
     tm.done();
     return NVA_OK;
   }
-  // K slices: the count s that minimises a per-CU cost model.  Two 128 x 64 workgroups share a
-  // CU and run their K tiles together at about 1.8 us per pair of 128 x 64 x 32 tiles, so the
-  // kernel takes ceil(tiles * s / (2 CUs)) rounds of ceil(K tiles / s) K tiles; s > 1 adds the
-  // partial planes (written, then read by the reduce, at about 5 TB/s) and the reduce launch.
-  // Every slice keeps at least 4 K tiles.
+  // K slices: the count s that minimises a per-CU cost model.  A CU runs its 128 x 128
+  // workgroups' K tiles at about 2.3 us each, so the kernel takes ceil(tiles * s / CUs) rounds of
+  // ceil(K tiles / s) K tiles; s > 1 adds the partial planes (written, then read by the reduce,
+  // at about 5 TB/s) and the reduce launch.  Every slice keeps at least 4 K tiles.
   const int64_t tiles = (int64_t)((out + linear_tile_cols() - 1) / linear_tile_cols()) *
                         ((rows + linear_tile_rows() - 1) / linear_tile_rows());
   const int bk = linear_k_tile();
   const int nkt = (in + bk - 1) / bk;
-  const int64_t slots = 2 * (int64_t)cus;
   int splits = 1;
   double best = 0.0;
   for (int sl = 1; sl <= std::max(1, nkt / 4); sl++) {
     const int per = (nkt + sl - 1) / sl;
     if (sl > 1 && (nkt + per - 1) / per != sl) continue;  // same slices as a smaller count
-    const double rounds = (double)((tiles * sl + slots - 1) / slots);
-    double us = rounds * per * 1.8;
+    const double rounds = (double)((tiles * sl + cus - 1) / cus);
+    double us = rounds * per * 2.3;
     if (sl > 1) us += 2.0 * sl * (double)rows * out * 4.0 / 5.0e6 + 3.0;
     if (sl == 1 || us < best) {
       best = us;

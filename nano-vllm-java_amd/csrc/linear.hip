@@ -1,4 +1,4 @@
-// Linear.Row (o_proj): y[M, N] = x[M, K] W[N, K]^T (+ bias) in fp32 on MFMA.
+// Linear.Row (o_proj): y[M, N] = x[M, K] W[N, K]^T (+ bias) at fp32 precision on MFMA.
 //
 // Semantics (tensor/Ops.java:84-124 linear, tensor/MatmulRuntime.java:234-255): W is the
 // row-major [out, in] weight, x the [rows, in] activations (the attention output
@@ -14,27 +14,17 @@
 //   * skinny_kernel when the 32 x 32 blocks of y number at most one per CU (decode batches of
 //     tens to a few hundred rows): one block per workgroup, K split over its eight waves, each
 //     streaming its own K range through a private LDS ring (below);
-//   * linear_kernel otherwise.  A workgroup owns a 128 x 64 tile of y and one K slice; its four
-//     waves own 32 rows x 64 columns each (2 blocks of v_mfma_f32_32x32x2_f32).  Two workgroups
-//     share a CU (48 KB of LDS, 88 VGPRs each), so while one waits at its barrier the other's
-//     MFMAs run on every SIMD: with one 128 x 128 workgroup of eight waves per CU, both waves of
-//     a SIMD stopped at the same barrier every tile (28% of wave cycles waiting, MFMA busy 0.77,
-//     against 0.93 of the fp32 peak here on large GEMMs).
-//   * x and W are both K-contiguous, so the A operand (x rows) and the B operand (W rows) are
-//     read the same way: for each 8-wide K step a lane (i, h) reads one float4 of its row
-//     (elements 4h .. 4h + 3 of the step), which feeds 4 MFMAs -- MFMA s contracts
-//     k = {s, 4 + s} of the step, a permutation that A and B share.
-//   * K tiles of 32 are copied HBM -> LDS with buffer loads that write LDS directly, from a
-//     wave-uniform base (row m0 / n0, column kt) plus fixed 32-bit lane offsets (rows past the
-//     matrix edge repeat its last row; their sums are never stored).  Each 128-byte row of a
-//     tile has its 16-byte chunks XOR-swizzled by ((row >> 1) & 7): measured free of LDS bank
-//     conflicts.  The copies are issued through copy16_to_lds_async, so the compiler adds no wait
-//     on them before the LDS reads of another stage.
-//   * Double-buffered, one barrier per K tile, placed before the tile's last 8-k step: the last
-//     step's fragments are already in registers, so the barrier (every wave has read this
-//     stage, and the next tile has landed) is followed at once by the next tile's copies into
-//     this stage and by MFMAs.  The next step's fragments are read while the current step's 8
-//     MFMAs run.
+//   * linear_kernel otherwise: 128 x 128 tiles on the fp16 matrix units, each fp32 operand as
+//     two scaled fp16 parts and each product as three (split_f16.h), 5.3 times the rate of
+//     v_mfma_f32.  K tiles of 64: every wave loads a share of the next tile into registers
+//     while the current one is multiplied, splits it and writes the parts to LDS
+//     (double-buffered, 128 KB; chunks XOR-swizzled, free of bank conflicts).  Bound by the
+//     board's power: with one scale per tile, 4096 x 2048 -> 1024 took 69 us alone at 2.41 GHz
+//     and 82 us back to back at 2.0 GHz, whatever the order of its loads and products (K tiles
+//     of 32: 91 us; operand reads ahead of their products: 83 us); the scales per row cost 8%
+//     more.  Against fp32 matrix instructions on the same boxes: 4096 x 2048 -> 1024 128 -> 72
+//     and 145 -> 88 us, 1959 x 5120 -> 5120 759 -> 432, 665 x 2048 -> 2048 76 -> 44, 229 x 4096
+//     -> 2560 54 -> 35; rel-L2 against float64 8.1e-7 -> 5.0e-7.
 //   * Output block layout (32 x 32, 16 values per lane): value r of lane (i, h) is row
 //     8 * (r / 4) + 4 * h + r % 4, column i -- lanes 0..31 write 128 contiguous bytes.
 //   * Tiles are assigned so that each XCD's workgroups cover one rectangle of the tile grid
@@ -47,15 +37,15 @@
 // Algorithmic work: 2 * M * N * K flops; HBM bytes (once): 4 * (M * K + N * K + M * N).
 #include "nva_internal.h"
 #include "nva_device.h"
+#include "split_f16.h"
 
 namespace nva {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
-constexpr int BM = 128, BN = 64, BK = 32;  // linear_kernel tile
+constexpr int BM = 128, BN = 128, BK = 64;  // linear_kernel tile
 constexpr int kSkinnyWaves = 8;  // waves of a skinny_kernel workgroup (two per SIMD)
 
 __device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
@@ -65,9 +55,9 @@ __device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast
 // 128-row band of x over all eight L2s, each fetching it again.  When the tile grid divides
 // into 8 equal rectangles of gm row bands x gn column tiles (gm * gn = 8), XCD slot t % 8 runs
 // rectangle t % 8 and t / 8 walks it row-major: each L2 then fetches 1/gm of x and 1/gn of W.
-// gm minimises that sum (x bands are BM rows, W tiles BN rows; ties go to the smaller gm: at
-// 4096 x 2048 -> 1024, 4 x 2 rectangles fetched 65 MB against 81 MB as 8 x 1 bands and 142 MB
-// in launch order, in the same time).  Any other grid keeps the launch order.  A bijection
+// gm minimises that sum (x bands are BM rows, W tiles BN rows; ties go to the smaller gm: with
+// 128 x 64 tiles at 4096 x 2048 -> 1024, 4 x 2 rectangles fetched 65 MB against 81 MB as 8 x 1
+// bands and 142 MB in launch order, in the same time).  Any other grid keeps the launch order.  A bijection
 // either way, so the result does not depend on where a workgroup actually runs.
 __device__ __forceinline__ void xcd_tile(int &tn, int &tm) {
   const int nt = gridDim.x, mt = gridDim.y;
@@ -94,168 +84,227 @@ __device__ __forceinline__ void xcd_tile(int &tn, int &tm) {
 }
 
 template <int N> struct IntC { static constexpr int value = N; };
-template <bool B> struct BoolC { static constexpr bool value = B; };
+
+// Offset (in fp16) of 16-byte chunk c (0..7) of row r of a tile's part: 16 rows at any one column
+// touch every LDS bank once.
+__device__ __forceinline__ int tile_pos(int r, int c) { return r * BK + ((c ^ ((r >> 1) & 7)) << 3); }
+
+// The dot product of x and w over [kb, ke) on fp32 instructions (kb and ke multiples of 4).
+__device__ float dot_fp32(const float *x, const float *w, int kb, int ke) {
+  float v = 0.0f;
+#pragma unroll 1
+  for (int k = kb; k < ke; k += 4) {
+    const float4 p = ld4(x + k), q = ld4(w + k);
+    v = fmaf(p.x, q.x, v);
+    v = fmaf(p.y, q.y, v);
+    v = fmaf(p.z, q.z, v);
+    v = fmaf(p.w, q.w, v);
+  }
+  return v;
+}
+
+// A row's scale: its exponent (of the largest magnitude it holds), the scale and the magnitude
+// from which it must be raised.
+struct RowScale {
+  int exp;
+  float scale, limit;
+};
+__device__ __forceinline__ RowScale row_scale(int e) {
+  return RowScale{e, split_scale(e), __uint_as_float((uint32_t)min(e + 1, 255) << 23)};
+}
 
 }  // namespace
 
-// One 128 x 64 tile of y (or of a K slice's partial plane) per workgroup; wave w owns rows
-// 32 w .. 32 w + 31 as two 32 x 32 blocks.
-__global__ void __launch_bounds__(256) linear_kernel(LinearLaunch a) {
-  constexpr int LA = BM / 32, LB = BN / 32;  // copy instructions per wave per tile (8 rows each)
-  constexpr int OPS = LA + LB;
-  constexpr int STAGE = (BM + BN) * BK;      // floats: A rows, then B rows
-  __shared__ __attribute__((aligned(16))) float lds[2 * STAGE];
+// One BM x BN tile of y (or of a K slice's partial plane) per workgroup of eight waves; wave w
+// owns rows 32 (w / 2) .. + 31 and columns 64 (w % 2) .. + 63 as two 32 x 32 blocks.
+//
+// Every row of x and of W has its own scale, that of its largest magnitude so far in the slice:
+// each row keeps the precision of its own size whatever its neighbours hold.  y's sums are in the
+// units of their row's and column's scales; a tile that raises one (the first, and a few
+// after it) says so in LDS and its readers rescale their sums.
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
+linear_kernel(LinearLaunch a) {
+  constexpr int PART = 128 * BK;  // fp16 values of one part of one operand's tile
+  constexpr int CPR = BK / 8;     // 8-value chunks per row
+  constexpr int RPU = 64 / CPR;   // rows per 64 chunks
+  constexpr int UW = 16 / RPU;    // 64-chunk units per wave and operand
+  static_assert(BM == 128 && BN == 128 && BK == 64, "the wave and lane maps below");
+  __shared__ __attribute__((aligned(16))) _Float16 sx[2][2 * PART], sw[2][2 * PART];
+  __shared__ __attribute__((aligned(16))) int sexp[2][128];  // scale exponents of the rows of x, w
+  __shared__ int schanged[2];  // by tile parity: the last tile that raised one
 
   int tn, tm;
   xcd_tile(tn, tm);
-  const int n0 = tn * BN;
-  const int m0 = tm * BM;
+  const int n0 = tn * BN, m0 = tm * BM;
   const int kb = blockIdx.z * a.k_per_split;
   const int ke = min(a.k, kb + a.k_per_split);
   const int ntiles = (ke - kb + BK - 1) / BK;
-  const bool ragged = (ke - kb) % BK != 0;  // the last tile ends inside a K tile
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int i = lane & 31;  // MFMA row (A) / column (B) index of this lane
-  const int h = lane >> 5;  // which float4 of an 8-wide K step this lane supplies
+  const int i = lane & 31, half = lane >> 5;
+  const int wm = 32 * (wave >> 1), wn = 64 * (wave & 1);
 
-  f32x16 acc0, acc1;
+  // This lane's share of every tile: eight k of UW rows of x and of w (rows past the edge repeat
+  // the last one; their sums are not stored).
+  const int lrow = 16 * wave + lane / CPR, lchunk = lane % CPR;
+  const float *xp[UW], *wp[UW];
+  int pos[UW];
+  RowScale xs[UW], ws[UW];
 #pragma unroll
-  for (int r = 0; r < 16; r++) {
-    acc0[r] = 0.0f;
-    acc1[r] = 0.0f;
+  for (int u = 0; u < UW; u++) {
+    xp[u] = a.x + (size_t)min(m0 + lrow + RPU * u, a.m - 1) * a.k + 8 * lchunk;
+    wp[u] = a.w + (size_t)min(n0 + lrow + RPU * u, a.n - 1) * a.k + 8 * lchunk;
+    pos[u] = tile_pos(lrow + RPU * u, lchunk);
+    xs[u] = ws[u] = row_scale(kMinExp);
   }
-
-  // Copy instruction p of wave w moves rows [8g, 8g + 8), g = 4p + w, of A (p < LA) or of B:
-  // lane l takes row 8g + l / 8 at LDS chunk position l % 8, i.e. global chunk
-  // (l % 8) ^ ((row >> 1) & 7).  Offsets are 32-bit: 128 rows of k floats stay below 2 GiB.
-  const int lrow = lane >> 3, lpos = lane & 7;
-  const int rows_a = min(BM, a.m - m0), rows_b = min(BN, a.n - n0);
-  uint32_t off[OPS];
-#pragma unroll
-  for (int p = 0; p < OPS; p++) {
-    const int r = 8 * (4 * (p < LA ? p : p - LA) + wave) + lrow;
-    const int rows = p < LA ? rows_a : rows_b;
-    off[p] = (uint32_t)min(r, rows - 1) * (uint32_t)a.k * 4u +
-             (uint32_t)(lpos ^ ((r >> 1) & 7)) * 16u;
-  }
-  const uint32_t lds0 = lds_address(lds);
-  auto issue = [&](int kt, int stage) __attribute__((always_inline)) {
-    // The descriptors end at the last row's column min(kt + BK, k): nothing past the matrix.
-    const int cols = min(BK, a.k - kt);
-    const float *xb = a.x + (size_t)m0 * a.k + kt;
-    const float *wb = a.w + (size_t)n0 * a.k + kt;
-    const uint32_t dst = lds0 + (uint32_t)(stage * STAGE) * 4u;
-#pragma unroll
-    for (int p = 0; p < LA; p++)
-      copy16_to_lds_async(xb, ((rows_a - 1) * a.k + cols) * 4, off[p],
-                          dst + (uint32_t)((4 * p + wave) * 8 * BK) * 4u);
-#pragma unroll
-    for (int p = 0; p < LB; p++)
-      copy16_to_lds_async(wb, ((rows_b - 1) * a.k + cols) * 4, off[LA + p],
-                          dst + (uint32_t)((BM + (4 * p + wave) * 8) * BK) * 4u);
+  f32x8 rx[UW], rw[UW];
+  auto load8 = [&](const float *p, int k) {
+    float4 u = make_float4(0.f, 0.f, 0.f, 0.f), v = u;
+    if (k + 4 <= ke) u = ld4(p);
+    if (k + 8 <= ke) v = ld4(p + 4);
+    return f32x8{u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
   };
-
-  // Fragments of 8-k step kk of a stage: A rows 32 w + i, B rows i and 32 + i, chunk 2 kk + h.
-  const int ra = 32 * wave + i;
-  const int xa = 4 * ((ra >> 1) & 7), xb = 4 * ((i >> 1) & 7);  // chunk swizzles (B: same for i, 32 + i)
-  auto frag = [&](int stage, int kk, float4 &av, float4 &b0, float4 &b1) __attribute__((always_inline)) {
-    const float *s = lds + stage * STAGE;
-    const int c = 4 * (2 * kk + h);
-    av = ld4(s + ra * BK + (c ^ xa));
-    b0 = ld4(s + (BM + i) * BK + (c ^ xb));
-    b1 = ld4(s + (BM + 32 + i) * BK + (c ^ xb));
-  };
-  // Chunks of a ragged last tile past the slice end are zero in both operands.
-  auto mask = [&](int kt, int kk, float4 &av, float4 &b0, float4 &b1) __attribute__((always_inline)) {
-    if (kt + 4 * (2 * kk + h) >= ke) {
-      av = make_float4(0.f, 0.f, 0.f, 0.f);
-      b0 = av;
-      b1 = av;
+  auto load_tile = [&](int kt) {
+    if (kt + BK <= ke) {
+#pragma unroll
+      for (int u = 0; u < UW; u++) {
+        const float4 e = ld4(xp[u] + kt), f = ld4(xp[u] + kt + 4);
+        rx[u] = f32x8{e.x, e.y, e.z, e.w, f.x, f.y, f.z, f.w};
+        const float4 g = ld4(wp[u] + kt), h = ld4(wp[u] + kt + 4);
+        rw[u] = f32x8{g.x, g.y, g.z, g.w, h.x, h.y, h.z, h.w};
+      }
+    } else {  // past the slice end: zeros
+#pragma unroll
+      for (int u = 0; u < UW; u++) {
+        rx[u] = load8(xp[u] + kt, kt + 8 * lchunk);
+        rw[u] = load8(wp[u] + kt, kt + 8 * lchunk);
+      }
     }
   };
-  // The two blocks' accumulations alternate, so no MFMA waits on the one before it.
-  auto mma = [&](const float4 &av, const float4 &b0, const float4 &b1) __attribute__((always_inline)) {
-    acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(av.x, b0.x, acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(av.x, b1.x, acc1, 0, 0, 0);
-    acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(av.y, b0.y, acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(av.y, b1.y, acc1, 0, 0, 0);
-    acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(av.z, b0.z, acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(av.z, b1.z, acc1, 0, 0, 0);
-    acc0 = __builtin_amdgcn_mfma_f32_32x32x2f32(av.w, b0.w, acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(av.w, b1.w, acc1, 0, 0, 0);
+  // Tile t (in rx / rw): the rows' scales raised where they do not hold it, its parts to buffer b.
+  auto row_max = [&](const f32x8 &r) {
+    uint32_t m = __float_as_uint(abs_max(0.0f, r));
+    m = max(m, dpp<0xB1>(m));  // over the row's eight lanes: lane ^ 1, ^ 2, then 7 - lane
+    m = max(m, dpp<0x4E>(m));
+    return __uint_as_float(max(m, dpp<0x141>(m)));
+  };
+  auto raise = [&](RowScale &s, float m, int operand, int row) {
+    const int e = (int)(__float_as_uint(m) >> 23);
+    if (e <= s.exp) return false;
+    s = row_scale(e);
+    if (lchunk == 0) sexp[operand][row] = e;
+    return true;
+  };
+  auto store_tile = [&](int t, int b) __attribute__((always_inline)) {
+    float mx[UW], mw[UW];
+    bool over = false;
+#pragma unroll
+    for (int u = 0; u < UW; u++) {
+      mx[u] = row_max(rx[u]);
+      mw[u] = row_max(rw[u]);
+      over |= mx[u] >= xs[u].limit || mw[u] >= ws[u].limit;
+    }
+    if (__any(over)) {
+      bool raised = false;
+#pragma unroll
+      for (int u = 0; u < UW; u++) {
+        raised |= raise(xs[u], mx[u], 0, lrow + RPU * u);
+        raised |= raise(ws[u], mw[u], 1, lrow + RPU * u);
+      }
+      if (__any(raised) && lane == 0) schanged[t & 1] = t;
+    }
+#pragma unroll
+    for (int u = 0; u < UW; u++) {
+      const Split8 x = split8(rx[u], xs[u].scale);
+      *reinterpret_cast<f16x8 *>(sx[b] + pos[u]) = x.hi;
+      *reinterpret_cast<f16x8 *>(sx[b] + PART + pos[u]) = x.lo;
+      const Split8 w = split8(rw[u], ws[u].scale);
+      *reinterpret_cast<f16x8 *>(sw[b] + pos[u]) = w.hi;
+      *reinterpret_cast<f16x8 *>(sw[b] + PART + pos[u]) = w.lo;
+    }
+  };
+  auto operand = [&](const _Float16 *t, int row, int chunk) {
+    const _Float16 *p = t + tile_pos(row, chunk);
+    return Split8{*reinterpret_cast<const f16x8 *>(p), *reinterpret_cast<const f16x8 *>(p + PART)};
   };
 
-  float4 fa0, fb00, fb01, fa1, fb10, fb11;  // two fragment sets: steps 0/2 and 1/3
+  f32x16 acc[2];
+#pragma unroll
+  for (int c = 0; c < 2; c++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[c][r] = 0.0f;
+  // Row of y (within the tile) of value r, column of block c.
+  auto row_of = [&](int r) { return wm + 8 * (r >> 2) + 4 * half + (r & 3); };
+  auto col_of = [&](int c) { return wn + 32 * c + i; };
+
+  int row_exp[16], col_exp[2];  // the units of acc
+#pragma unroll
+  for (int r = 0; r < 16; r++) row_exp[r] = kMinExp;
+  col_exp[0] = col_exp[1] = kMinExp;
+
+  // At the barrier of tile t every wave is done with tile t - 1, whose buffer takes tile t + 1,
+  // and tile t is in LDS.
+  if (threadIdx.x < 256) sexp[threadIdx.x >> 7][threadIdx.x & 127] = kMinExp;
+  if (threadIdx.x < 2) schanged[threadIdx.x] = -1;
+  __syncthreads();
   if (ntiles > 0) {
-    issue(kb, 0);
-    if (ntiles > 1) {
-      issue(kb + BK, 1);
-      wait_copies<OPS>();
-    } else {
-      wait_copies<0>();
-    }
-    lds_barrier();
-    frag(0, 0, fa0, fb00, fb01);
+    load_tile(kb);
+    store_tile(0, 0);
+    if (ntiles > 1) load_tile(kb + BK);
   }
-  // Tile t in stage s (a constant: two tiles per loop iteration).  RAGGED (the last tile of a
-  // slice that ends inside it) zeroes the chunks past the slice end; it is a separate copy of
-  // the body, so the common body is straight-line code the compiler can interleave.
-  auto tile = [&](int t, auto s_, auto ragged_) __attribute__((always_inline)) {
-    constexpr int s = decltype(s_)::value;
-    constexpr bool RAGGED = decltype(ragged_)::value;
-    const int kt = kb + t * BK;
-    frag(s, 1, fa1, fb10, fb11);
-    if (RAGGED) mask(kt, 0, fa0, fb00, fb01);
-    mma(fa0, fb00, fb01);
-    frag(s, 2, fa0, fb00, fb01);
-    if (RAGGED) mask(kt, 1, fa1, fb10, fb11);
-    mma(fa1, fb10, fb11);
-    frag(s, 3, fa1, fb10, fb11);
-    if (RAGGED) mask(kt, 2, fa0, fb00, fb01);
-    mma(fa0, fb00, fb01);
-    if (t + 1 < ntiles) {
-      // This wave's reads of stage s have returned (step 3 is in registers) and its copies of
-      // tile t + 1 have landed (tile t + 2's are not issued yet); after the barrier the same
-      // holds for every wave, so stage s takes tile t + 2 and tile t + 1 is read.
-      wait_lds_reads();
-      wait_copies<0>();
-      lds_barrier();
-      if (t + 2 < ntiles) issue(kt + 2 * BK, s);
-      frag(s ^ 1, 0, fa0, fb00, fb01);
+  auto tile = [&](int t, auto b_) __attribute__((always_inline)) {
+    constexpr int b = decltype(b_)::value;
+    __syncthreads();
+    if (schanged[b] == t) {
+      auto down = [](int d) { return __uint_as_float((uint32_t)max(0, 127 + d) << 23); };
+      float fc[2];
+#pragma unroll
+      for (int c = 0; c < 2; c++) {
+        const int e = sexp[1][col_of(c)];
+        fc[c] = down(col_exp[c] - e);
+        col_exp[c] = e;
+      }
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const int e = sexp[0][row_of(r)];
+        const float f = down(row_exp[r] - e);
+        row_exp[r] = e;
+        acc[0][r] *= f * fc[0];
+        acc[1][r] *= f * fc[1];
+      }
+      __syncthreads();  // before tile t + 1 raises them again
     }
-    if (RAGGED) mask(kt, 3, fa1, fb10, fb11);
-    mma(fa1, fb10, fb11);
+#pragma unroll
+    for (int s = 0; s < BK / 16; s++) {
+      const Split8 x = operand(sx[b], wm + i, 2 * s + half);
+#pragma unroll
+      for (int c = 0; c < 2; c++)
+        acc[c] = mfma_split(x, operand(sw[b], wn + 32 * c + i, 2 * s + half), acc[c]);
+    }
+    if (t + 1 < ntiles) store_tile(t + 1, b ^ 1);
+    if (t + 2 < ntiles) load_tile(kb + (t + 2) * BK);
   };
-  const int full_tiles = ragged ? ntiles - 1 : ntiles;
-  int t = 0;
-  for (; t + 1 < full_tiles; t += 2) {
-    tile(t, IntC<0>{}, BoolC<false>{});
-    tile(t + 1, IntC<1>{}, BoolC<false>{});
-  }
-  if (t < full_tiles) {
-    tile(t, IntC<0>{}, BoolC<false>{});
-    t++;
-  }
-  if (t < ntiles) {  // the ragged last tile, in stage t % 2
-    if (t & 1)
-      tile(t, IntC<1>{}, BoolC<true>{});
-    else
-      tile(t, IntC<0>{}, BoolC<true>{});
+  for (int t = 0; t < ntiles; t += 2) {
+    tile(t, IntC<0>{});
+    if (t + 1 < ntiles) tile(t + 1, IntC<1>{});
   }
 
   const bool direct = a.splits == 1;
   float *dst = direct ? a.y : a.part + (size_t)blockIdx.z * a.m * a.n;
 #pragma unroll
-  for (int bn = 0; bn < 2; bn++) {
-    const int col = n0 + bn * 32 + i;
+  for (int c = 0; c < 2; c++) {
+    const int col = n0 + col_of(c);
     if (col >= a.n) continue;
+    const float fc = split_unscale(col_exp[c]);
     const float bias = direct && a.bias ? a.bias[col] : 0.0f;
-    const f32x16 &acc = bn == 0 ? acc0 : acc1;
 #pragma unroll
     for (int r = 0; r < 16; r++) {
-      const int row = m0 + 32 * wave + 8 * (r >> 2) + 4 * h + (r & 3);
-      if (row < a.m) dst[(size_t)row * a.n + col] = acc[r] + bias;
+      const int row = m0 + row_of(r);
+      if (row >= a.m) continue;
+      float v = acc[c][r] * split_unscale(row_exp[r]) * fc;
+      if (v != v)  // an infinity (or NaN) in the row or column
+        v = dot_fp32(a.x + (size_t)row * a.k, a.w + (size_t)col * a.k, kb, ke);
+      dst[(size_t)row * a.n + col] = v + bias;
     }
   }
 }
@@ -681,7 +730,7 @@ hipError_t launch_reduce(const LinearLaunch &a, hipStream_t s) {
 hipError_t launch_linear(const LinearLaunch &a, hipStream_t s) {
   if (a.m <= 0 || a.n <= 0) return hipSuccess;
   const dim3 grid((a.n + BN - 1) / BN, (a.m + BM - 1) / BM, a.splits);
-  hipLaunchKernelGGL(linear_kernel, grid, dim3(256), 0, s, a);
+  hipLaunchKernelGGL(linear_kernel, grid, dim3(512), 0, s, a);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || a.splits == 1) return e;
   return launch_reduce(a, s);
