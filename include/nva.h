@@ -290,7 +290,7 @@ nva_status nva_rms_norm_forward(nva_ctx *ctx, const nva_rms_norm *norm, const fl
  * y[rows, out] = x[rows, in] weight[out, in]^T (+ bias[out]).  x, weight, bias and y are
  * DEVICE pointers (x and weight 16-byte aligned, in % 4 == 0); bias may be NULL.  x is
  * typically the attention output [tokens, num_heads * head_dim] used in place (in < 4194304).
- * fp32 on MFMA; the sum order differs from the reference's gemv panels (fp32 rounding only).
+ * fp32 precision on MFMA; the sum order differs from the reference's gemv panels (fp32 rounding only).
  * Up to 16 rows run the library's weight-streaming GEMV, batches whose 32 x 32 output blocks fit
  * one per CU its 16 x 16- or 32 x 32-block kernels, and larger GEMMs its 128 x 64-tile kernel. */
 nva_status nva_linear_forward(nva_ctx *ctx, const float *x, int rows, int in,
