@@ -921,8 +921,7 @@ KvView make_dense_view(const float *k, const float *v) {
 // is longer, plus the split kernel's later start.  The constants were fitted to the two kernels
 // on 54 drawn steps; fp32 / split us a layer at 40 q / 8 KV heads, d = 128: 2 + 16 + 208+3 tokens
 // 17.1 / 25.1, 230+11 and 211+15 21.1 / 27.5, 57 tokens 18.1 / 20.6, 280 tokens 45.7 / 36.7; at
-// d = 64, 140 and 245+58 tokens 27.4 / 29.3, 241+333 43.0 / 37.0; at d = 256, 1553+48 27.8 / 29.2,
-// 3736+100 43.6 / 38.9.
+// d = 64, 140 and 245+58 tokens 27.4 / 29.3, 241+333 43.0 / 37.0; at d = 256, 1553+48 27.8 / 29.2.
 bool use_fp32_tiles(nva_ctx *ctx, const nva_attn_desc &d, int hpw_fp32, int hpw_split, int window) {
   struct Cost {
     double floor, per_wave;  // CU us per key tile: at least, and per active wave
@@ -938,9 +937,10 @@ bool use_fp32_tiles(nva_ctx *ctx, const nva_attn_desc &d, int hpw_fp32, int hpw_
                      : dim == 128 ? Cost{2.5, 0.41, 1, 32}
                      : dim == 256 ? Cost{6.5, 0.0, 1, 32}
                                   : Cost{7.0, 0.0, 1, 32};
-  // us; at d = 512 with the per-row loads of segments that end inside a key tile (300+200 and 300
-  // tokens: 63.5 / 73.3 us a layer, while 400 take 52.0 / 46.3).
-  const double later = dim == 512 ? 10.0 : dim == 64 ? 3.5 : 2.0;
+  // us; at d = 256 and 512 with the per-row loads of segments that end inside a key tile (d = 256,
+  // 77+700 tokens: 45.6 / 51.5 us a layer, 2005+333 60.4 / 64.3; d = 512, 300+200 and 300 tokens:
+  // 63.5 / 73.3).
+  const double later = dim == 512 ? 10.0 : dim == 256 ? 9.0 : dim == 64 ? 3.5 : 2.0;
   auto estimate = [&](const Cost &c, int hpw, int tile_q) {
     double sum = 0.0, longest = 0.0;
     for (int b = 0; b < ctx->num_seqs; b++) {
