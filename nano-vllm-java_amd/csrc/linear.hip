@@ -14,17 +14,20 @@
 //   * skinny_kernel when the 32 x 32 blocks of y number at most one per CU (decode batches of
 //     tens to a few hundred rows): one block per workgroup, K split over its eight waves, each
 //     streaming its own K range through a private LDS ring (below);
-//   * linear_kernel otherwise: 128 x 128 tiles on the fp16 matrix units, each fp32 operand as
-//     two scaled fp16 parts and each product as three (split_f16.h), 5.3 times the rate of
-//     v_mfma_f32.  K tiles of 64: every wave loads a share of the next tile into registers
-//     while the current one is multiplied, splits it and writes the parts to LDS
-//     (double-buffered, 128 KB; chunks XOR-swizzled, free of bank conflicts).  Bound by the
-//     board's power: with one scale per tile, 4096 x 2048 -> 1024 took 69 us alone at 2.41 GHz
-//     and 82 us back to back at 2.0 GHz, whatever the order of its loads and products (K tiles
-//     of 32: 91 us; operand reads ahead of their products: 83 us); the scales per row cost 8%
-//     more.  Against fp32 matrix instructions on the same boxes: 4096 x 2048 -> 1024 128 -> 72
-//     and 145 -> 88 us, 1959 x 5120 -> 5120 759 -> 432, 665 x 2048 -> 2048 76 -> 44, 229 x 4096
-//     -> 2560 54 -> 35; rel-L2 against float64 8.1e-7 -> 5.0e-7.
+//   * linear_kernel otherwise: 128 x 128 tiles on the bf16 matrix units, each fp32 operand as
+//     three bf16 parts that hold all its 24 bits and each product as six, 2.7 times the rate of
+//     v_mfma_f32.  K tiles of 32: every wave loads a share of the tile two ahead into registers,
+//     splits the next one between the products of the current one and writes its parts to LDS
+//     (double-buffered, 96 KB; chunks XOR-swizzled, free of bank conflicts).  A wave multiplies
+//     64 x 64, half of the tile's k: 12 operand reads per 24 products, where 32 x 64 over all
+//     of them takes 9 per 12 and 3% longer.  Bound by the board's power (2.1 GHz, matrix units
+//     47% busy; interleaving split and products 4%, order of the two waves of a SIMD nothing).
+//     Against fp32 matrix instructions: 4096 x 2048 -> 1024 128 -> 103 us; rel-L2 against float64
+//     of the worst row or column at 1030 x 2052 -> 300 3.0e-7 -> 2.2e-7, at any spread of sizes
+//     within a row.  Two scaled fp16 parts take 86 us with one scale per row, but bits of values
+//     far below the row's largest are lost (2^24 below it: 6e-5).  Results that the parts do not
+//     hold (infinities, NaN, magnitudes below 2^-70) are taken again on v_mfma_f32: with one such
+//     row of x 208 us, with a NaN in all of them 295.
 //   * Output block layout (32 x 32, 16 values per lane): value r of lane (i, h) is row
 //     8 * (r / 4) + 4 * h + r % 4, column i -- lanes 0..31 write 128 contiguous bytes.
 //   * Tiles are assigned so that each XCD's workgroups cover one rectangle of the tile grid
@@ -45,7 +48,7 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 namespace {
 
-constexpr int BM = 128, BN = 128, BK = 64;  // linear_kernel tile
+constexpr int BM = 128, BN = 128, BK = 32;  // linear_kernel tile
 constexpr int kSkinnyWaves = 8;  // waves of a skinny_kernel workgroup (two per SIMD)
 
 __device__ __forceinline__ float4 ld4(const float *p) { return *reinterpret_cast<const float4 *>(p); }
@@ -85,53 +88,55 @@ __device__ __forceinline__ void xcd_tile(int &tn, int &tm) {
 
 template <int N> struct IntC { static constexpr int value = N; };
 
-// Offset (in fp16) of 16-byte chunk c (0..7) of row r of a tile's part: 16 rows at any one column
-// touch every LDS bank once.
-__device__ __forceinline__ int tile_pos(int r, int c) { return r * BK + ((c ^ ((r >> 1) & 7)) << 3); }
-
-// The dot product of x and w over [kb, ke) on fp32 instructions (kb and ke multiples of 4).
-__device__ float dot_fp32(const float *x, const float *w, int kb, int ke) {
-  float v = 0.0f;
-#pragma unroll 1
-  for (int k = kb; k < ke; k += 4) {
-    const float4 p = ld4(x + k), q = ld4(w + k);
-    v = fmaf(p.x, q.x, v);
-    v = fmaf(p.y, q.y, v);
-    v = fmaf(p.z, q.z, v);
-    v = fmaf(p.w, q.w, v);
+// An fp32 value is the sum of three bf16 ones, hi + mid + lo, each the rest rounded to nearest: 8
+// significant bits a part, all 24 of x together, and bf16 has fp32's exponents, so there is no scale
+// to choose and no value too small beside its neighbours (the last bits of values below 2^-110 fall
+// under bf16's smallest step: see retake).  A product is taken as six: mid mid', lo hi', hi lo', mid hi',
+// hi mid' and hi hi', the largest last; the three left out are below 2^-26 of it, a quarter of an
+// fp32 rounding.  An infinity becomes NaN in mid, and so in the sums it enters.
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+struct Split3 {
+  bf16x8 hi, mid, lo;
+};
+__device__ __forceinline__ uint32_t round2(float a, float b) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
+}
+__device__ __forceinline__ Split3 split3(const f32x8 &x) {
+  u32x4 hi, mid, lo;
+#pragma unroll
+  for (int j = 0; j < 4; j++) {
+    float a = x[2 * j], b = x[2 * j + 1];
+    hi[j] = round2(a, b);
+    a -= __uint_as_float(hi[j] << 16);
+    b -= __uint_as_float(hi[j] & 0xffff0000u);
+    mid[j] = round2(a, b);
+    a -= __uint_as_float(mid[j] << 16);
+    b -= __uint_as_float(mid[j] & 0xffff0000u);
+    lo[j] = round2(a, b);
   }
-  return v;
+  return Split3{__builtin_bit_cast(bf16x8, hi), __builtin_bit_cast(bf16x8, mid),
+                __builtin_bit_cast(bf16x8, lo)};
 }
 
-// A row's scale: its exponent (of the largest magnitude it holds), the scale and the magnitude
-// from which it must be raised.
-struct RowScale {
-  int exp;
-  float scale, limit;
-};
-__device__ __forceinline__ RowScale row_scale(int e) {
-  return RowScale{e, split_scale(e), __uint_as_float((uint32_t)min(e + 1, 255) << 23)};
+// Whether a sum of split products cannot stand: it is not finite (an infinity or NaN in its row or
+// column, or a part rounded up to infinity), or so small that parts below bf16's smallest step,
+// 2^-133, may show in it (beside operands of up to 2^33).
+constexpr float kSmallest = 0x1p-70f;
+__device__ __forceinline__ bool retake(float v) {
+  return !(fabsf(v) < INFINITY) || (fabsf(v) < kSmallest && v != 0.0f);
 }
 
 }  // namespace
 
-// One BM x BN tile of y (or of a K slice's partial plane) per workgroup of eight waves; wave w
-// owns rows 32 (w / 2) .. + 31 and columns 64 (w % 2) .. + 63 as two 32 x 32 blocks.
-//
-// Every row of x and of W has its own scale, that of its largest magnitude so far in the slice:
-// each row keeps the precision of its own size whatever its neighbours hold.  y's sums are in the
-// units of their row's and column's scales; a tile that raises one (the first, and a few
-// after it) says so in LDS and its readers rescale their sums.
+// One BM x BN tile of y (or of a K slice's partial plane) per workgroup of eight waves: wave w owns
+// the 64 x 64 quarter w % 4 as 2 x 2 blocks, over the first (w < 4) or second 16 k of every K tile.
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
 linear_kernel(LinearLaunch a) {
-  constexpr int PART = 128 * BK;  // fp16 values of one part of one operand's tile
-  constexpr int CPR = BK / 8;     // 8-value chunks per row
-  constexpr int RPU = 64 / CPR;   // rows per 64 chunks
-  constexpr int UW = 16 / RPU;    // 64-chunk units per wave and operand
-  static_assert(BM == 128 && BN == 128 && BK == 64, "the wave and lane maps below");
-  __shared__ __attribute__((aligned(16))) _Float16 sx[2][2 * PART], sw[2][2 * PART];
-  __shared__ __attribute__((aligned(16))) int sexp[2][128];  // scale exponents of the rows of x, w
-  __shared__ int schanged[2];  // by tile parity: the last tile that raised one
+  constexpr int PART = 128 * BK;  // bf16 values of one part of one operand's tile
+  static_assert(BM == 128 && BN == 128 && BK == 32, "the wave and lane maps below");
+  __shared__ __attribute__((aligned(16))) uint16_t lds[4][3 * PART];
+  uint16_t (*const sx)[3 * PART] = lds, (*const sw)[3 * PART] = lds + 2;
 
   int tn, tm;
   xcd_tile(tn, tm);
@@ -142,169 +147,161 @@ linear_kernel(LinearLaunch a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   const int i = lane & 31, half = lane >> 5;
-  const int wm = 32 * (wave >> 1), wn = 64 * (wave & 1);
+  const int wk = wave >> 2, wm = 64 * ((wave >> 1) & 1), wn = 64 * (wave & 1);
 
-  // This lane's share of every tile: eight k of UW rows of x and of w (rows past the edge repeat
+  // This lane's share of every tile: eight k of one row of x and of w (rows past the edge repeat
   // the last one; their sums are not stored).
-  const int lrow = 16 * wave + lane / CPR, lchunk = lane % CPR;
-  const float *xp[UW], *wp[UW];
-  int pos[UW];
-  RowScale xs[UW], ws[UW];
-#pragma unroll
-  for (int u = 0; u < UW; u++) {
-    xp[u] = a.x + (size_t)min(m0 + lrow + RPU * u, a.m - 1) * a.k + 8 * lchunk;
-    wp[u] = a.w + (size_t)min(n0 + lrow + RPU * u, a.n - 1) * a.k + 8 * lchunk;
-    pos[u] = tile_pos(lrow + RPU * u, lchunk);
-    xs[u] = ws[u] = row_scale(kMinExp);
-  }
-  f32x8 rx[UW], rw[UW];
+  const int lrow = 16 * wave + (lane >> 2), lchunk = lane & 3;
+  const float *xp = a.x + (size_t)min(m0 + lrow, a.m - 1) * a.k + 8 * lchunk;
+  const float *wp = a.w + (size_t)min(n0 + lrow, a.n - 1) * a.k + 8 * lchunk;
+  const int pos = part_pos(lrow, lchunk);
+  struct Share {
+    f32x8 x, w;
+  };
   auto load8 = [&](const float *p, int k) {
     float4 u = make_float4(0.f, 0.f, 0.f, 0.f), v = u;
     if (k + 4 <= ke) u = ld4(p);
     if (k + 8 <= ke) v = ld4(p + 4);
     return f32x8{u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
   };
-  auto load_tile = [&](int kt) {
+  auto load_tile = [&](int kt, Share &r) __attribute__((always_inline)) {
     if (kt + BK <= ke) {
-#pragma unroll
-      for (int u = 0; u < UW; u++) {
-        const float4 e = ld4(xp[u] + kt), f = ld4(xp[u] + kt + 4);
-        rx[u] = f32x8{e.x, e.y, e.z, e.w, f.x, f.y, f.z, f.w};
-        const float4 g = ld4(wp[u] + kt), h = ld4(wp[u] + kt + 4);
-        rw[u] = f32x8{g.x, g.y, g.z, g.w, h.x, h.y, h.z, h.w};
-      }
+      const float4 e = ld4(xp + kt), f = ld4(xp + kt + 4), g = ld4(wp + kt), h = ld4(wp + kt + 4);
+      r.x = f32x8{e.x, e.y, e.z, e.w, f.x, f.y, f.z, f.w};
+      r.w = f32x8{g.x, g.y, g.z, g.w, h.x, h.y, h.z, h.w};
     } else {  // past the slice end: zeros
-#pragma unroll
-      for (int u = 0; u < UW; u++) {
-        rx[u] = load8(xp[u] + kt, kt + 8 * lchunk);
-        rw[u] = load8(wp[u] + kt, kt + 8 * lchunk);
-      }
+      r.x = load8(xp + kt, kt + 8 * lchunk);
+      r.w = load8(wp + kt, kt + 8 * lchunk);
     }
   };
-  // Tile t (in rx / rw): the rows' scales raised where they do not hold it, its parts to buffer b.
-  auto row_max = [&](const f32x8 &r) {
-    uint32_t m = __float_as_uint(abs_max(0.0f, r));
-    m = max(m, dpp<0xB1>(m));  // over the row's eight lanes: lane ^ 1, ^ 2, then 7 - lane
-    m = max(m, dpp<0x4E>(m));
-    return __uint_as_float(max(m, dpp<0x141>(m)));
+  auto store_parts = [&](const f32x8 &r, uint16_t *dst) __attribute__((always_inline)) {
+    const Split3 p = split3(r);
+    *reinterpret_cast<bf16x8 *>(dst + pos) = p.hi;
+    *reinterpret_cast<bf16x8 *>(dst + PART + pos) = p.mid;
+    *reinterpret_cast<bf16x8 *>(dst + 2 * PART + pos) = p.lo;
   };
-  auto raise = [&](RowScale &s, float m, int operand, int row) {
-    const int e = (int)(__float_as_uint(m) >> 23);
-    if (e <= s.exp) return false;
-    s = row_scale(e);
-    if (lchunk == 0) sexp[operand][row] = e;
-    return true;
-  };
-  auto store_tile = [&](int t, int b) __attribute__((always_inline)) {
-    float mx[UW], mw[UW];
-    bool over = false;
+  auto read = [&](const uint16_t *t, int part, int row, bf16x8 (&r)[2]) __attribute__((always_inline)) {
 #pragma unroll
-    for (int u = 0; u < UW; u++) {
-      mx[u] = row_max(rx[u]);
-      mw[u] = row_max(rw[u]);
-      over |= mx[u] >= xs[u].limit || mw[u] >= ws[u].limit;
-    }
-    if (__any(over)) {
-      bool raised = false;
-#pragma unroll
-      for (int u = 0; u < UW; u++) {
-        raised |= raise(xs[u], mx[u], 0, lrow + RPU * u);
-        raised |= raise(ws[u], mw[u], 1, lrow + RPU * u);
-      }
-      if (__any(raised) && lane == 0) schanged[t & 1] = t;
-    }
-#pragma unroll
-    for (int u = 0; u < UW; u++) {
-      const Split8 x = split8(rx[u], xs[u].scale);
-      *reinterpret_cast<f16x8 *>(sx[b] + pos[u]) = x.hi;
-      *reinterpret_cast<f16x8 *>(sx[b] + PART + pos[u]) = x.lo;
-      const Split8 w = split8(rw[u], ws[u].scale);
-      *reinterpret_cast<f16x8 *>(sw[b] + pos[u]) = w.hi;
-      *reinterpret_cast<f16x8 *>(sw[b] + PART + pos[u]) = w.lo;
-    }
-  };
-  auto operand = [&](const _Float16 *t, int row, int chunk) {
-    const _Float16 *p = t + tile_pos(row, chunk);
-    return Split8{*reinterpret_cast<const f16x8 *>(p), *reinterpret_cast<const f16x8 *>(p + PART)};
+    for (int c = 0; c < 2; c++)
+      r[c] = *reinterpret_cast<const bf16x8 *>(t + part * PART + part_pos(row + 32 * c + i, 2 * wk + half));
   };
 
-  f32x16 acc[2];
+  f32x16 acc[2][2];
+#pragma unroll
+  for (int c = 0; c < 4; c++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) acc[c >> 1][c & 1][r] = 0.0f;
+  // acc += x w on one part of each; the four blocks' sums alternate.
+  auto mma = [&](const bf16x8 (&x)[2], const bf16x8 (&w)[2]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+      acc[c >> 1][c & 1] =
+          __builtin_amdgcn_mfma_f32_32x32x16_bf16(x[c >> 1], w[c & 1], acc[c >> 1][c & 1], 0, 0, 0);
+  };
+
+  // At the barrier of tile t every wave is done with tile t - 1, whose buffer takes tile t + 1,
+  // and tile t is in LDS.  Tile t + 1 is in registers, t + 2 on its way to others.
+  Share r1, r2;
+  load_tile(kb, r1);
+  load_tile(kb + BK, r2);  // (past the slice end: zeros, without a load)
+  store_parts(r1.x, sx[0]);
+  store_parts(r1.w, sw[0]);
+  r1 = r2;
+  if (ntiles > 2) load_tile(kb + 2 * BK, r2);
+  auto tile = [&](int t, auto b_, Share &next) __attribute__((always_inline)) {
+    constexpr int b = decltype(b_)::value;
+    __syncthreads();
+    bf16x8 xh[2], xm[2], xl[2], wh[2], wm_[2], wl[2];
+    read(sx[b], 1, wm, xm);
+    read(sw[b], 1, wn, wm_);
+    read(sx[b], 2, wm, xl);
+    read(sw[b], 0, wn, wh);
+    read(sx[b], 0, wm, xh);
+    read(sw[b], 2, wn, wl);
+    mma(xm, wm_);
+    mma(xl, wh);
+    mma(xh, wl);
+    mma(xm, wh);
+    mma(xh, wm_);
+    mma(xh, wh);
+    // (The last tile stores an old one, where nothing reads it.)
+    store_parts(next.x, sx[b ^ 1]);
+    store_parts(next.w, sw[b ^ 1]);
+#pragma unroll
+    for (int g = 0; g < 24; g++) {  // a product, then five instructions of the split
+      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x2, 5, 0);
+    }
+    if (t + 3 < ntiles) load_tile(kb + (t + 3) * BK, next);
+  };
+  for (int t = 0; t < ntiles; t += 2) {
+    tile(t, IntC<0>{}, r1);
+    if (t + 1 < ntiles) tile(t + 1, IntC<1>{}, r2);
+  }
+
+  // The second k half's sums go to the first half's waves: two blocks each way through LDS.
+  __syncthreads();
+  float *sum = reinterpret_cast<float *>(lds) + (wave & 3) * 4096;
+  static_assert(sizeof(lds) >= 4 * 4 * 4096, "the sums exchanged through LDS");
+#pragma unroll
+  for (int r = 0; r < 16; r++)
+#pragma unroll
+    for (int c = 0; c < 2; c++)
+      sum[((wk * 2 + c) * 16 + r) * 64 + lane] = wk ? acc[0][c][r] : acc[1][c][r];
+  __syncthreads();
+  f32x16 y[2];
+  // The results' bits without the sign (least: less one, so that 0 wraps to the top): three
+  // instructions a result, where testing each took 2-4 us of small calls.
+  uint32_t most = 0, least = ~0u;
 #pragma unroll
   for (int c = 0; c < 2; c++)
 #pragma unroll
-    for (int r = 0; r < 16; r++) acc[c][r] = 0.0f;
-  // Row of y (within the tile) of value r, column of block c.
-  auto row_of = [&](int r) { return wm + 8 * (r >> 2) + 4 * half + (r & 3); };
-  auto col_of = [&](int c) { return wn + 32 * c + i; };
-
-  int row_exp[16], col_exp[2];  // the units of acc
+    for (int r = 0; r < 16; r++) {
+      y[c][r] = (wk ? acc[1][c][r] : acc[0][c][r]) + sum[(((wk ^ 1) * 2 + c) * 16 + r) * 64 + lane];
+      const uint32_t u = __float_as_uint(y[c][r]);
+      most = max(most, 2 * u);
+      least = min(least, 2 * u - 1);
+    }
+  const int m1 = m0 + wm + 32 * wk, n1 = n0 + wn;  // this wave's 32 x 64 of y
+  if (__any(most >= 2 * 0x7f800000u || least < 2 * __float_as_uint(kSmallest) - 1)) {
+    // Those (retake) again on fp32 matrix instructions, operands straight from memory.
+    const float *xr = a.x + (size_t)min(m1 + i, a.m - 1) * a.k + 4 * half;
+    const float *wr[2];
+    f32x16 z[2];
 #pragma unroll
-  for (int r = 0; r < 16; r++) row_exp[r] = kMinExp;
-  col_exp[0] = col_exp[1] = kMinExp;
-
-  // At the barrier of tile t every wave is done with tile t - 1, whose buffer takes tile t + 1,
-  // and tile t is in LDS.
-  if (threadIdx.x < 256) sexp[threadIdx.x >> 7][threadIdx.x & 127] = kMinExp;
-  if (threadIdx.x < 2) schanged[threadIdx.x] = -1;
-  __syncthreads();
-  if (ntiles > 0) {
-    load_tile(kb);
-    store_tile(0, 0);
-    if (ntiles > 1) load_tile(kb + BK);
-  }
-  auto tile = [&](int t, auto b_) __attribute__((always_inline)) {
-    constexpr int b = decltype(b_)::value;
-    __syncthreads();
-    if (schanged[b] == t) {
-      auto down = [](int d) { return __uint_as_float((uint32_t)max(0, 127 + d) << 23); };
-      float fc[2];
+    for (int c = 0; c < 2; c++) {
+      wr[c] = a.w + (size_t)min(n1 + 32 * c + i, a.n - 1) * a.k + 4 * half;
+#pragma unroll
+      for (int r = 0; r < 16; r++) z[c][r] = 0.0f;
+    }
+#pragma unroll 1
+    for (int k = kb; k < ke; k += 8) {
+      float4 p = make_float4(0.f, 0.f, 0.f, 0.f), q[2] = {p, p};
+      if (k + 4 * half < ke) p = ld4(xr + k), q[0] = ld4(wr[0] + k), q[1] = ld4(wr[1] + k);
 #pragma unroll
       for (int c = 0; c < 2; c++) {
-        const int e = sexp[1][col_of(c)];
-        fc[c] = down(col_exp[c] - e);
-        col_exp[c] = e;
+        z[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(p.x, q[c].x, z[c], 0, 0, 0);
+        z[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(p.y, q[c].y, z[c], 0, 0, 0);
+        z[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(p.z, q[c].z, z[c], 0, 0, 0);
+        z[c] = __builtin_amdgcn_mfma_f32_32x32x2f32(p.w, q[c].w, z[c], 0, 0, 0);
       }
-#pragma unroll
-      for (int r = 0; r < 16; r++) {
-        const int e = sexp[0][row_of(r)];
-        const float f = down(row_exp[r] - e);
-        row_exp[r] = e;
-        acc[0][r] *= f * fc[0];
-        acc[1][r] *= f * fc[1];
-      }
-      __syncthreads();  // before tile t + 1 raises them again
     }
 #pragma unroll
-    for (int s = 0; s < BK / 16; s++) {
-      const Split8 x = operand(sx[b], wm + i, 2 * s + half);
+    for (int c = 0; c < 2; c++)
 #pragma unroll
-      for (int c = 0; c < 2; c++)
-        acc[c] = mfma_split(x, operand(sw[b], wn + 32 * c + i, 2 * s + half), acc[c]);
-    }
-    if (t + 1 < ntiles) store_tile(t + 1, b ^ 1);
-    if (t + 2 < ntiles) load_tile(kb + (t + 2) * BK);
-  };
-  for (int t = 0; t < ntiles; t += 2) {
-    tile(t, IntC<0>{});
-    if (t + 1 < ntiles) tile(t + 1, IntC<1>{});
+      for (int r = 0; r < 16; r++) y[c][r] = retake(y[c][r]) ? z[c][r] : y[c][r];
   }
-
   const bool direct = a.splits == 1;
   float *dst = direct ? a.y : a.part + (size_t)blockIdx.z * a.m * a.n;
 #pragma unroll
   for (int c = 0; c < 2; c++) {
-    const int col = n0 + col_of(c);
+    const int col = n1 + 32 * c + i;
     if (col >= a.n) continue;
-    const float fc = split_unscale(col_exp[c]);
     const float bias = direct && a.bias ? a.bias[col] : 0.0f;
 #pragma unroll
     for (int r = 0; r < 16; r++) {
-      const int row = m0 + row_of(r);
-      if (row >= a.m) continue;
-      float v = acc[c][r] * split_unscale(row_exp[r]) * fc;
-      if (v != v)  // an infinity (or NaN) in the row or column
-        v = dot_fp32(a.x + (size_t)row * a.k, a.w + (size_t)col * a.k, kb, ke);
-      dst[(size_t)row * a.n + col] = v + bias;
+      const int row = m1 + 8 * (r >> 2) + 4 * half + (r & 3);
+      if (row < a.m) dst[(size_t)row * a.n + col] = y[c][r] + bias;
     }
   }
 }
