@@ -30,9 +30,9 @@
 //   * S^T[key][query] = K Q^T, then O^T[dim][query] += V^T P^T: S^T leaves 16 keys of one query
 //     in each lane, which are the lane's B operand of PV once the contraction takes its keys in
 //     that order, so P never leaves registers.
-//   * Softmax in the log2 domain; the running max is moved, and O rescaled, only when a tile's
-//     max exceeds it by more than 2^8.  Only tiles that cross the causal diagonal, the window
-//     edge or the end of the keys are masked.
+//   * Softmax in the log2 domain, relative to a reference that moves, and O with it, only when a
+//     tile's max exceeds it by more than 2^4 or lies more than 2^10 below it.  Only tiles that
+//     cross the causal diagonal, the window edge or the end of the keys are masked.
 //   * A wave whose sums are not finite at the end of a segment (infinities in the inputs), or
 //     whose results are so small beside a tile's largest |k| or |v| that the steps of the split
 //     would show in them, takes its queries again on fp32 instructions (scan_segment).
@@ -58,8 +58,11 @@ namespace nva {
 namespace {
 
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kLazyRescale = 8.0f;  // log2 units
-constexpr int kProbExp = 7;            // probabilities, at most 2^8, are split as 2^7 p < 2^16
+constexpr int kProbExp = 11;  // probabilities, at most 2^kRaise, are split as 2^11 p <= 2^15
+// Log2 units.  The reference that a query's probabilities are relative to moves up to a tile's max
+// that exceeds it by more than kRaise, and down to kMargin above one that lies kLower further below,
+// but no more than kRefSpan below the largest max so far.
+constexpr float kRaise = 4.0f, kMargin = 4.0f, kLower = 6.0f, kRefSpan = 40.0f;
 // Largest factor from products of scaled q and k (off by about 2^-7 from the steps of the split)
 // to scores: their error stays below 2^-20.
 constexpr float kMaxScoreUnit = 0x1p-13f;
@@ -201,11 +204,29 @@ __device__ void scan_segment(const TileLaunch &a, const TileItem &it, const int3
   }
 }
 
+// The reference of a query's probabilities from a tile of this max on; its sums are to be
+// multiplied by exp2(m - result).  It follows the tiles' maxima both ways: the probabilities are
+// split beside 2^kProbExp, and in tiles far below the largest max (where one key of little or no V
+// has most of the weight, all others) the split's steps would show.  top: the largest max so far.
+__device__ __forceinline__ float reference(float mx, float m, float &top) {
+  top = fmaxf(top, mx);
+  const float low = fmaxf(mx + kMargin, top - kRefSpan);
+  const bool down = mx > -INFINITY && m > low + kLower;
+  return mx > m + kRaise ? mx : down ? low : m;
+}
+
+// What the steps of the split add to the error of a query's o in one tile, p being the sum of the
+// lane's (scaled) probabilities: half a step of lo, 2^-25 and 2^-25.8 on average, in each of 16
+// probabilities beside |v| of up to 2^15, and in each v.
+__device__ __forceinline__ float split_steps(float p) {
+  return fmaf(p, 0x1p-26f, fminf(p * 0x1p15f, 0x1p-9f));
+}
+
 // Whether a query's sums (o in units of 2^kProbExp and the V scale; every lane of the query has
-// its part) cannot stand: one is not finite, or the result lies more than 2^14 below the largest
-// |v|, where the steps of the split V would show in it.
+// its part) cannot stand: one is not finite, or the split's steps, e, are more than 2^-21 of the
+// largest result.
 template <int NB>
-__device__ __forceinline__ bool unsound(const f32x16 (&o)[NB], float l, int o_exp) {
+__device__ __forceinline__ bool unsound(const f32x16 (&o)[NB], float l, float e, int o_exp) {
   float zero = 0.0f * l, top = 0.0f;
 #pragma unroll
   for (int b = 0; b < NB; b++)
@@ -216,7 +237,18 @@ __device__ __forceinline__ bool unsound(const f32x16 (&o)[NB], float l, int o_ex
     }
   top = max_halves(top);
   // (At the smallest scale, V holds nothing but zeros and values below 2^-105.)
-  return !(zero == 0.0f) || (top < l * (float)(1 << kProbExp) && o_exp > kMinExp);
+  return !(zero == 0.0f) || (top < e * 0x1p21f && o_exp > kMinExp);
+}
+
+// The factor of a query's sums in its result: 1 / l or, in a partial, to the largest max.
+__device__ __forceinline__ float result_factor(const Dest &d, float l, float m, float top) {
+  if (d.partial) return m == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(m - top);
+  return l == 0.0f ? 0.0f : 1.0f / l;
+}
+__device__ __forceinline__ float4 result4(const f32x16 &o, int r, float f, int o_exp) {
+  const int e = o_exp - 141 - kProbExp;  // the scales of V and of the probabilities
+  return make_float4(__builtin_ldexpf(o[r] * f, e), __builtin_ldexpf(o[r + 1] * f, e),
+                     __builtin_ldexpf(o[r + 2] * f, e), __builtin_ldexpf(o[r + 3] * f, e));
 }
 
 // A wave's share of the workgroup's tiles: UW units of 64 lanes x 8 floats of K (RPU whole rows
@@ -448,8 +480,8 @@ prefill_split_kernel(TileLaunch a) {
     for (int b = 0; b < NB; b++)
 #pragma unroll
       for (int r = 0; r < 16; r++) o[b][r] = 0.0f;
-    float m_run = -INFINITY;  // log2 units
-    float l_run = 0.0f;
+    float m_run = -INFINITY, m_top = -INFINITY;  // reference and largest max, log2 units
+    float l_run = 0.0f, e_run = 0.0f;
     int o_exp = kMinExp;  // exponent of the V scale that o is in
     bool coarse = false;  // the split's steps show in this query's result
 
@@ -525,17 +557,18 @@ prefill_split_kernel(TileLaunch a) {
       const float c = fmaxf(qscale * split_unscale(k_exp), 0x1p-126f);  // 0 * -inf is NaN
       coarse |= c > kMaxScoreUnit;
       mx = max_halves(mx) * c;
-      const bool need = mx > m_run + kLazyRescale;
-      if (__any(need)) {
-        const float mn = need ? mx : m_run;
+      const float mn = reference(mx, m_run, m_top);
+      if (__any(mn != m_run)) {
         const float alpha = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - mn);
         l_run *= alpha;
+        e_run *= alpha;
 #pragma unroll
         for (int b = 0; b < NB; b++) o[b] *= alpha;
         m_run = mn;
       }
       if (v_max != o_exp) {
         const float alpha = __uint_as_float((uint32_t)max(0, 127 + o_exp - v_max) << 23);
+        e_run *= alpha;
 #pragma unroll
         for (int b = 0; b < NB; b++) o[b] *= alpha;
         o_exp = v_max;
@@ -552,6 +585,7 @@ prefill_split_kernel(TileLaunch a) {
         lt[s] = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
         p[s] = split8_unscaled(e, one);
       }
+      e_run += split_steps(lt[0] + lt[1]);
       // One addition to the long sum per tile, without the probabilities' scale.
       l_run = fmaf(lt[0] + lt[1], __uint_as_float((uint32_t)(127 - p_exp) << 23), l_run);
 
@@ -584,25 +618,23 @@ prefill_split_kernel(TileLaunch a) {
 
     if (!wave_active) continue;
     const float l_tot = sum_halves(l_run);
-    if (__any(coarse || unsound<NB>(o, l_tot, o_exp))) {
+    if (__any(coarse || unsound<NB>(o, l_tot, sum_halves(e_run), o_exp))) {
       scan_segment<D, 1>(a, it, stab, share.blk0, kvh, h, wq0);
       continue;
     }
     if (!qvalid) continue;
     const Dest d = destination(a, it, qi, h, D);
-    const float inv = d.partial ? 1.0f : (l_tot == 0.0f ? 0.0f : 1.0f / l_tot);
-    const float vs = split_unscale(o_exp - kProbExp);
+    const float f = result_factor(d, l_tot, m_run, m_top);
     // Register r of o[b] is dim 32 b + 8 (r / 4) + 4 half + r % 4.
 #pragma unroll
     for (int b = 0; b < NB; b++)
 #pragma unroll
       for (int r = 0; r < 16; r += 4)
         *reinterpret_cast<float4 *>(d.row + 32 * b + 2 * r + 4 * half) =
-            make_float4(o[b][r] * vs * inv, o[b][r + 1] * vs * inv, o[b][r + 2] * vs * inv,
-                        o[b][r + 3] * vs * inv);
+            result4(o[b], r, f, o_exp);
     if (d.partial && half == 0) {
-      a.part_m[d.pidx] = m_run;
-      a.part_l[d.pidx] = l_tot;
+      a.part_m[d.pidx] = m_top;
+      a.part_l[d.pidx] = l_tot * f;
     }
   }
 }
@@ -697,8 +729,8 @@ prefill_split_wide_kernel(TileLaunch a) {
     for (int b = 0; b < NB; b++)
 #pragma unroll
       for (int r = 0; r < 16; r++) o[b][r] = 0.0f;
-    float m_run = -INFINITY;  // log2 units
-    float l_run = 0.0f;
+    float m_run = -INFINITY, m_top = -INFINITY;  // reference and largest max, log2 units
+    float l_run = 0.0f, e_run = 0.0f;
     int o_exp = kMinExp;  // exponent of the V scale that o is in
     bool coarse = false;  // the split's steps show in this query's result
 
@@ -815,17 +847,18 @@ prefill_split_wide_kernel(TileLaunch a) {
 #pragma unroll
         for (int r = 0; r < 16; r++) mx = fmaxf(mx, st[r]);
         mx = max_halves(mx) * sl2;
-        const bool need = mx > m_run + kLazyRescale;
-        if (__any(need)) {
-          const float mn = need ? mx : m_run;
+        const float mn = reference(mx, m_run, m_top);
+        if (__any(mn != m_run)) {
           const float alpha = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - mn);
           l_run *= alpha;
+          e_run *= alpha;
 #pragma unroll
           for (int b = 0; b < NB; b++) o[b] *= alpha;
           m_run = mn;
         }
         if (v_max != o_exp) {
           const float alpha = __uint_as_float((uint32_t)max(0, 127 + o_exp - v_max) << 23);
+          e_run *= alpha;
 #pragma unroll
           for (int b = 0; b < NB; b++) o[b] *= alpha;
           o_exp = v_max;
@@ -842,6 +875,7 @@ prefill_split_wide_kernel(TileLaunch a) {
           lt[s] = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
           p[s] = split8_unscaled(e, one);
         }
+        e_run += split_steps(lt[0] + lt[1]);
         l_run = fmaf(lt[0] + lt[1], __uint_as_float((uint32_t)(127 - p_exp) << 23), l_run);
         auto read_v = [&](int u) {
           return read_split(sv + part_pos(DW * ds + 32 * (u % NB) + i, 2 * (u / NB) + half));
@@ -861,25 +895,23 @@ prefill_split_wide_kernel(TileLaunch a) {
     }
 
     const float l_tot = sum_halves(l_run);
-    if (__syncthreads_or(coarse || unsound<NB>(o, l_tot, o_exp))) {
+    if (__syncthreads_or(coarse || unsound<NB>(o, l_tot, sum_halves(e_run), o_exp))) {
       const int q0 = wq0 + ds * (QW / DS);
       if (q0 < it.qlen) scan_segment<D, DS>(a, it, stab, share.blk0, kvh, h, q0);
       continue;
     }
     if (!qvalid) continue;
     const Dest d = destination(a, it, qi, h, D);
-    const float inv = d.partial ? 1.0f : (l_tot == 0.0f ? 0.0f : 1.0f / l_tot);
-    const float vs = split_unscale(o_exp - kProbExp);
+    const float f = result_factor(d, l_tot, m_run, m_top);
 #pragma unroll
     for (int b = 0; b < NB; b++)
 #pragma unroll
       for (int r = 0; r < 16; r += 4)
         *reinterpret_cast<float4 *>(d.row + DW * ds + 32 * b + 2 * r + 4 * half) =
-            make_float4(o[b][r] * vs * inv, o[b][r + 1] * vs * inv, o[b][r + 2] * vs * inv,
-                        o[b][r + 3] * vs * inv);
+            result4(o[b], r, f, o_exp);
     if (d.partial && half == 0 && ds == 0) {
-      a.part_m[d.pidx] = m_run;
-      a.part_l[d.pidx] = l_tot;
+      a.part_m[d.pidx] = m_top;
+      a.part_l[d.pidx] = l_tot * f;
     }
   }
 }

@@ -1,0 +1,93 @@
+"""Prefill where one key, V row or V channel dwarfs what the result is made of.
+
+The split kernel holds probabilities and V in fp16 parts beside a power of two, so their steps are
+fixed beside the largest value in their units.  Here most of the weight (or the largest |v|) sits
+where it adds nothing to the result: a sink key with no V, a V row that no query weighs, V tiles
+of unlike size, a V channel far above the others.  Each query row of each head is compared with
+float64 by itself (channels of unlike size by themselves).
+
+Bar: 1e-5, the attention bar: up to 4096 fp32 products per output give sqrt(4096) * 2^-24 = 3.8e-6 if
+their roundings are independent, a few times that where they cancel."""
+
+import numpy as np
+import pytest
+import torch
+
+from cases import Case
+from gpu_checks import dev, load_arena, say
+from nanollvm_amd import Attention, Context
+from nanollvm_amd import workloads as W
+from test_gpu_prefill_split import exact
+
+pytestmark = pytest.mark.gpu
+
+BAR = 1e-5
+N = 4096
+HEADS = [(64, 1), (64, 4), (128, 2), (256, 4), (512, 2)]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = Context(0)
+    yield c
+    c.close()
+
+
+def build(d, rep, seed, seqs=((0, N), (0, 77))):
+    rng = np.random.default_rng(seed)
+    wl = W.build(f"range d{d} rep{rep}", list(seqs), is_prefill=True, hq=2 * rep, hkv=2, d=d,
+                 scale=float(np.float32(d ** -0.5)), rng=rng, block_size=256, pool_cap=20000)
+    case = Case(wl, seed=seed)
+    # Dim 0 sets the score of single keys: every query has the same 4 there, the keys 0.
+    case.q[:, :, 0] = 4.0
+    case.k[:, :, 0] = 0.0
+    return case
+
+
+def set_score(case, key, score):
+    case.k[key] = 0.0
+    case.k[key, :, 0] = score / (4.0 * case.wl.scale)
+
+
+def sink_score(weight, keys):
+    """Score that takes this share of the softmax beside `keys` others of score N(0, 1)."""
+    return np.log(weight / (1.0 - weight) * keys) + 0.5
+
+
+def check(ctx, case, name, channels=slice(None), rows=slice(None), bar=BAR):
+    wl, m = case.wl, case.wl.meta
+    say(name)
+    arena = load_arena(ctx, case)
+    try:
+        ctx.set(**m.context_args())
+        ctx.bind_kv_cache(arena)
+        out = Attention(wl.hq, wl.d, wl.scale, wl.hkv, wl.window, 0).forward(
+            dev(case.q), dev(case.k), dev(case.v), ctx)
+        ctx.sync()
+        got = out.cpu().numpy().astype(np.float64)
+    finally:
+        ctx.clear()
+        arena.close()
+    kc, vc = case.k_cache.copy(), case.v_cache.copy()
+    slots = np.asarray(m.slot_mapping, np.int64)
+    kc.reshape(-1, wl.hkv, wl.d)[slots] = case.k
+    vc.reshape(-1, wl.hkv, wl.d)[slots] = case.v
+    want = exact(case, kc, vc)
+    assert np.all(np.isfinite(got))
+    err = np.linalg.norm((got - want)[rows][..., channels], axis=-1)
+    size = np.linalg.norm(want[rows][..., channels], axis=-1)
+    worst = float(np.max(err / np.where(size > 0, size, 1.0)))
+    say(f"{name}: worst row rel_l2={worst:.3e}")
+    assert worst <= bar, worst
+
+
+@pytest.mark.parametrize("v", [0.0, 1e-3])
+@pytest.mark.parametrize("weight", [0.7, 0.98])
+@pytest.mark.parametrize("d,rep", HEADS)
+def test_sink_key(ctx, d, rep, weight, v):
+    """The first key takes most of the weight (of the last row; more of the earlier ones) and adds
+    little or nothing."""
+    case = build(d, rep, seed=11)
+    set_score(case, 0, sink_score(weight, N))
+    case.v[0] *= np.float32(v)
+    check(ctx, case, f"sink d{d} rep{rep} weight {weight} v {v}")
