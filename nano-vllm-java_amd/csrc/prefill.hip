@@ -24,9 +24,8 @@
 //     that any 16 rows read at one column touch every bank once.
 //   * Scales: q per query; K and V per tile, from the tile's largest magnitude, which the waves
 //     exchange through LDS ahead of the barrier that the split waits for anyway.  A K tile's
-//     scale goes into the factor of its scores.  O^T is kept in the units of the largest V
-//     scale of the segment so far; a V tile whose own scale is smaller gets the difference
-//     through its probabilities.
+//     scale goes into the factor of its scores.  O^T is kept in the units of V's scale, which
+//     stays for tiles down to 2^-3 of it.
 //   * S^T[key][query] = K Q^T, then O^T[dim][query] += V^T P^T: S^T leaves 16 keys of one query
 //     in each lane, which are the lane's B operand of PV once the contraction takes its keys in
 //     that order, so P never leaves registers.
@@ -66,7 +65,9 @@ constexpr float kRaise = 4.0f, kMargin = 4.0f, kLower = 6.0f, kRefSpan = 40.0f;
 // Largest factor from products of scaled q and k (off by about 2^-7 from the steps of the split)
 // to scores: their error stays below 2^-20.
 constexpr float kMaxScoreUnit = 0x1p-13f;
-constexpr int kVExpSpan = 40;          // a V tile's scale stays within 2^40 of the largest one's
+// The exponent of V's scale stays for tiles of up to kUnitSlack below it and within kUnitSpan of the
+// largest one's.
+constexpr int kUnitSlack = 3, kUnitSpan = 32;
 constexpr int KT = 32;                // keys per tile
 constexpr int kAhead = 2;             // operand reads in flight ahead of their products
 constexpr int kKeepReads = 0x6;       // sched_barrier: only VALU and SALU move across
@@ -215,6 +216,16 @@ __device__ __forceinline__ float reference(float mx, float m, float &top) {
   return mx > m + kRaise ? mx : down ? low : m;
 }
 
+// The exponent of V's scale, in which O is kept, for a tile of exponent e.  It follows the tiles both
+// ways, so that neither V nor the probabilities lose bits to a larger V before or after them.  top:
+// the largest e so far.  (Tiles of zeros leave it as it is.)
+__device__ __forceinline__ int value_unit(int e, int unit, int &top) {
+  top = max(top, e);
+  return e > unit                                      ? e
+         : e > kMinExp && e < unit - kUnitSlack ? max(e, top - kUnitSpan)
+                                                : unit;
+}
+
 // What the steps of the split add to the error of a query's o in one tile, p being the sum of the
 // lane's (scaled) probabilities: half a step of lo, 2^-25 and 2^-25.8 on average, in each of 16
 // probabilities beside |v| of up to 2^15, and in each v.
@@ -226,7 +237,7 @@ __device__ __forceinline__ float split_steps(float p) {
 // its part) cannot stand: one is not finite, or the split's steps, e, are more than 2^-21 of the
 // largest result.
 template <int NB>
-__device__ __forceinline__ bool unsound(const f32x16 (&o)[NB], float l, float e, int o_exp) {
+__device__ __forceinline__ bool unsound(const f32x16 (&o)[NB], float l, float e, int v_top) {
   float zero = 0.0f * l, top = 0.0f;
 #pragma unroll
   for (int b = 0; b < NB; b++)
@@ -237,7 +248,7 @@ __device__ __forceinline__ bool unsound(const f32x16 (&o)[NB], float l, float e,
     }
   top = max_halves(top);
   // (At the smallest scale, V holds nothing but zeros and values below 2^-105.)
-  return !(zero == 0.0f) || (top < e * 0x1p21f && o_exp > kMinExp);
+  return !(zero == 0.0f) || (top < e * 0x1p21f && v_top > kMinExp);
 }
 
 // The factor of a query's sums in its result: 1 / l or, in a partial, to the largest max.
@@ -491,27 +502,26 @@ prefill_split_kernel(TileLaunch a) {
       const float m = max_waves(share.largest(rk), share.largest(rv));
       if (i == 0) smax[b][half][wave] = m;
     };
-    int k_exp_in = kMinExp, v_exp_in = kMinExp, v_exp_max = kMinExp;
+    int k_exp_in = kMinExp, v_unit = kMinExp, v_top = kMinExp;
     auto take_scales = [&](int b) {
       const TileExps sc = tile_exps<NW>(smax[b][half][lane & (NW - 1)]);
       k_exp_in = sc.a;
-      v_exp_max = max(v_exp_max, sc.b);
-      v_exp_in = max(sc.b, v_exp_max - kVExpSpan);
+      v_unit = value_unit(sc.b, v_unit, v_top);
     };
     auto store_tile = [&](int b) {
       share.store_k(rk, split_scale(k_exp_in), sk[b]);
-      share.store_v(rv, split_scale(v_exp_in), sv[b]);
+      share.store_v(rv, split_scale(v_unit), sv[b]);
     };
     auto read_split = [&](const _Float16 *p) {
       return Split8{*reinterpret_cast<const f16x8 *>(p),
                     *reinterpret_cast<const f16x8 *>(p + PART)};
     };
 
-    // k_exp, v_exp: the tile's; v_max: the largest of the segment up to it, v_max >= v_exp.
+    // k_exp, v_exp: the exponents of the tile's scales.
     // The next tile (in rk / rv) is split and stored to buffer nb among the products of QK, and
     // the one after it loaded (next_kt; none if < 0).
     auto compute_tile = [&](int kt, const _Float16 *tk, const _Float16 *tv, int k_exp, int v_exp,
-                            int v_max, int nb, int next_kt) {
+                            int nb, int next_kt) {
       if (!wave_active || kt >= whi_max || kt + KT <= wlo_min) {
         store_tile(nb);
         if (next_kt >= 0) load_tile(next_kt);
@@ -566,15 +576,14 @@ prefill_split_kernel(TileLaunch a) {
         for (int b = 0; b < NB; b++) o[b] *= alpha;
         m_run = mn;
       }
-      if (v_max != o_exp) {
-        const float alpha = __uint_as_float((uint32_t)max(0, 127 + o_exp - v_max) << 23);
+      if (v_exp != o_exp) {
+        const float alpha = __uint_as_float((uint32_t)max(0, 127 + o_exp - v_exp) << 23);
         e_run *= alpha;
 #pragma unroll
         for (int b = 0; b < NB; b++) o[b] *= alpha;
-        o_exp = v_max;
+        o_exp = v_exp;
       }
-      const int p_exp = kProbExp + v_exp - v_max;
-      const float ms = (m_run == -INFINITY ? 0.0f : m_run) - (float)p_exp;
+      const float ms = (m_run == -INFINITY ? 0.0f : m_run) - (float)kProbExp;
       Split8 p[2];
       float lt[2];
 #pragma unroll
@@ -587,7 +596,7 @@ prefill_split_kernel(TileLaunch a) {
       }
       e_run += split_steps(lt[0] + lt[1]);
       // One addition to the long sum per tile, without the probabilities' scale.
-      l_run = fmaf(lt[0] + lt[1], __uint_as_float((uint32_t)(127 - p_exp) << 23), l_run);
+      l_run = fmaf(lt[0] + lt[1], 1.0f / (1 << kProbExp), l_run);
 
       // O^T += V^T P^T, 16 keys a step (V chunk 2 s + half holds the lane's keys).
 #pragma unroll
@@ -609,16 +618,16 @@ prefill_split_kernel(TileLaunch a) {
     for (int t = 0; t < ntiles; t++) {
       const int kt = it.ks + t * KT;
       const int b = t & 1;
-      const int k_exp = k_exp_in, v_exp = v_exp_in, v_max = v_exp_max;
+      const int k_exp = k_exp_in, v_exp = v_unit;
       share_max(b ^ 1);  // the last tile stores itself once more, where nothing reads it
       __syncthreads();
       take_scales(b ^ 1);
-      compute_tile(kt, sk[b], sv[b], k_exp, v_exp, v_max, b ^ 1, t + 2 < ntiles ? kt + 2 * KT : -1);
+      compute_tile(kt, sk[b], sv[b], k_exp, v_exp, b ^ 1, t + 2 < ntiles ? kt + 2 * KT : -1);
     }
 
     if (!wave_active) continue;
     const float l_tot = sum_halves(l_run);
-    if (__any(coarse || unsound<NB>(o, l_tot, sum_halves(e_run), o_exp))) {
+    if (__any(coarse || unsound<NB>(o, l_tot, sum_halves(e_run), v_top))) {
       scan_segment<D, 1>(a, it, stab, share.blk0, kvh, h, wq0);
       continue;
     }
@@ -734,7 +743,7 @@ prefill_split_wide_kernel(TileLaunch a) {
     int o_exp = kMinExp;  // exponent of the V scale that o is in
     bool coarse = false;  // the split's steps show in this query's result
 
-    int k_exp_in = kMinExp, v_exp = kMinExp, v_max = kMinExp;
+    int k_exp_in = kMinExp, v_exp = kMinExp, v_top = kMinExp;
     auto share_max = [&](int t, float m) {
       const float x = max_waves(m, m);
       if (lane == 0) smax[t][wave] = x;
@@ -746,8 +755,7 @@ prefill_split_wide_kernel(TileLaunch a) {
     };
     auto store_v = [&]() {
       const TileExps sc = tile_exps<NW>(smax[1][lane & 7]);
-      v_max = max(v_max, sc.a);
-      v_exp = max(sc.a, v_max - kVExpSpan);
+      v_exp = value_unit(sc.a, v_exp, v_top);
       share.store_v(rv, split_scale(v_exp), sv);
     };
     auto read_split = [&](const _Float16 *p) {
@@ -856,15 +864,14 @@ prefill_split_wide_kernel(TileLaunch a) {
           for (int b = 0; b < NB; b++) o[b] *= alpha;
           m_run = mn;
         }
-        if (v_max != o_exp) {
-          const float alpha = __uint_as_float((uint32_t)max(0, 127 + o_exp - v_max) << 23);
+        if (v_exp != o_exp) {
+          const float alpha = __uint_as_float((uint32_t)max(0, 127 + o_exp - v_exp) << 23);
           e_run *= alpha;
 #pragma unroll
           for (int b = 0; b < NB; b++) o[b] *= alpha;
-          o_exp = v_max;
+          o_exp = v_exp;
         }
-        const int p_exp = kProbExp + v_exp - v_max;
-        const float ms = (m_run == -INFINITY ? 0.0f : m_run) - (float)p_exp;
+        const float ms = (m_run == -INFINITY ? 0.0f : m_run) - (float)kProbExp;
         Split8 p[2];
         float lt[2];
 #pragma unroll
@@ -876,7 +883,7 @@ prefill_split_wide_kernel(TileLaunch a) {
           p[s] = split8_unscaled(e, one);
         }
         e_run += split_steps(lt[0] + lt[1]);
-        l_run = fmaf(lt[0] + lt[1], __uint_as_float((uint32_t)(127 - p_exp) << 23), l_run);
+        l_run = fmaf(lt[0] + lt[1], 1.0f / (1 << kProbExp), l_run);
         auto read_v = [&](int u) {
           return read_split(sv + part_pos(DW * ds + 32 * (u % NB) + i, 2 * (u / NB) + half));
         };
@@ -895,7 +902,7 @@ prefill_split_wide_kernel(TileLaunch a) {
     }
 
     const float l_tot = sum_halves(l_run);
-    if (__syncthreads_or(coarse || unsound<NB>(o, l_tot, sum_halves(e_run), o_exp))) {
+    if (__syncthreads_or(coarse || unsound<NB>(o, l_tot, sum_halves(e_run), v_top))) {
       const int q0 = wq0 + ds * (QW / DS);
       if (q0 < it.qlen) scan_segment<D, DS>(a, it, stab, share.blk0, kvh, h, q0);
       continue;

@@ -91,3 +91,26 @@ def test_sink_key(ctx, d, rep, weight, v):
     set_score(case, 0, sink_score(weight, N))
     case.v[0] *= np.float32(v)
     check(ctx, case, f"sink d{d} rep{rep} weight {weight} v {v}")
+
+
+@pytest.mark.parametrize("factor", [2.0 ** 10, 2.0 ** 12, 8000.0, 2.0 ** 20])
+@pytest.mark.parametrize("d,rep", HEADS)
+def test_v_row_without_weight(ctx, d, rep, factor):
+    """Most of the weight on one key, and beside it a large V row that no query weighs."""
+    case = build(d, rep, seed=12)
+    set_score(case, 5, sink_score(0.64, N))
+    set_score(case, 40, -60.0)
+    case.v[40] *= np.float32(factor)
+    check(ctx, case, f"v row d{d} rep{rep} factor {factor}")
+
+
+@pytest.mark.parametrize("span", [8, 14])
+@pytest.mark.parametrize("d,rep", HEADS)
+def test_v_tiles_of_unlike_size(ctx, d, rep, span):
+    """V over 2^-span .. 2^0 by tiles of 32 keys; the weight on a row of the smallest."""
+    case = build(d, rep, seed=13)
+    t = np.arange(case.wl.tokens) // 32
+    case.v *= np.exp2(-((t * 5) % (span + 1))).astype(np.float32)[:, None, None]
+    small = 32 * int(np.argmax((t[::32] * 5) % (span + 1) == span))
+    set_score(case, small + 3, sink_score(1.0 - 2.0 ** -(span + 1), N))
+    check(ctx, case, f"v tiles d{d} rep{rep} span {span}")
