@@ -32,9 +32,12 @@
 //   * Softmax in the log2 domain, relative to a reference that moves, and O with it, only when a
 //     tile's max exceeds it by more than 2^4 or lies more than 2^10 below it.  Only tiles that
 //     cross the causal diagonal, the window edge or the end of the keys are masked.
-//   * A wave whose sums are not finite at the end of a segment (infinities in the inputs), or
-//     whose results are so small beside a tile's largest |k| or |v| that the steps of the split
-//     would show in them, takes its queries again on fp32 instructions (scan_segment).
+//   * Every query adds up what the steps of the split can have done to its sums.  A wave with a
+//     query where that is more than 2^-21 of the result, whose sums are not finite (infinities in
+//     the inputs) or whose scores the steps would show in takes the segment's 32 queries again on
+//     fp32 matrix instructions, after all segments (fp32_segment; a call whose every query sees
+//     an infinity takes 3 to 5 times as long, up to 2.1 ms at 12289 cached + 2048 tokens before
+//     with the keys taken one by one: 9 to 20 times).
 //   * Operands are read from LDS two steps ahead of their products and the next tile is split
 //     and stored after QK: 14% fewer cycles than in source order, 4% less time.
 //
@@ -125,81 +128,137 @@ __device__ __forceinline__ Dest destination(const TileLaunch &a, const TileItem 
   return d;
 }
 
-// The segment's result for 32 / DS queries (from tile query q0 on) on fp32 instructions, key by
-// key: 2 DS lanes share a query, D / (2 DS) dims each.  For segments that the split does not
-// fit; a few times slower than v_mfma_f32 tiles.
-template <int D, int DS>
-__device__ void scan_segment(const TileLaunch &a, const TileItem &it, const int32_t *stab, int blk0,
-                             int kvh, int h, int q0) {
-  constexpr int QN = QW / DS, DH = D / (2 * DS);
+// The segment's result for a wave's 32 queries (from tile query q0 on) and dims [v0, v0 + 32 NB) of V
+// on fp32 matrix instructions, operands straight from memory: for segments that the split does not
+// fit.  Lanes and registers of S^T and O^T are those of the split products; a step of PV contracts
+// the keys of one S^T register.  O^T is added up over the tiles' own sums, one rounding a tile.
+template <int D, int NB>
+__device__ void fp32_segment(const TileLaunch &a, const TileItem &it, int kvh, int h, int q0, int v0) {
   const int lane = threadIdx.x & 63;
-  const int dpart = lane / QN;
-  const int qi = q0 + lane % QN;
-  const bool qvalid = qi < it.qlen;
+  const int i = lane & 31, half = lane >> 5;
+  const int W = a.window;
   const int off = it.klen - it.qlen;
+  const int qi = q0 + i;
+  const bool qvalid = qi < it.qlen;
   const int aq = off + (qvalid ? qi : it.qlen - 1);
-  const int lo = a.window > 0 ? max(0, aq - a.window + 1) : 0;
+  const int vis_lo = W > 0 ? max(0, aq - W + 1) : 0;
+  const int q1 = min(q0 + QW, it.qlen) - 1;
+  const int all_lo = W > 0 ? max(0, off + q1 - W + 1) : 0;  // keys that every query sees
+  const int all_hi = off + q0 + 1;
+  const int any_lo = W > 0 ? max(0, off + q0 - W + 1) : 0;
+  const int any_hi = min(it.ke, off + q1 + 1);
+  const int32_t *table = a.kv.table + (size_t)it.seq * a.kv.bt_stride;
   const float sl2 = a.scale * kLog2e;
-  const float *qp = a.q + ((size_t)(it.qstart + aq - off) * a.hq + h) * D + DH * dpart;
-  float q[DH], o[DH];
-#pragma unroll
-  for (int s = 0; s < DH; s += 4) {
-    const float4 x = ld4(qp + s);
-    q[s] = x.x, q[s + 1] = x.y, q[s + 2] = x.z, q[s + 3] = x.w;
-    o[s] = o[s + 1] = o[s + 2] = o[s + 3] = 0.0f;
-  }
-  float m = -INFINITY, l = 0.0f;
   const size_t rs = (size_t)a.hkv * D;
-  const int q_last = min(q0 + QN, it.qlen) - 1;
-  const int k0 = max(it.ks, a.window > 0 ? max(0, off + q0 - a.window + 1) : 0);
-  const int k1 = min(it.ke, off + q_last + 1);
+  const float *qp = a.q + ((size_t)(it.qstart + aq - off) * a.hq + h) * D + 4 * half;
+  const float *kbase = a.kv.k + (size_t)kvh * D + 4 * half;
+  const float *vbase = a.kv.v + (size_t)kvh * D + v0;
+  f32x16 o[NB];
+#pragma unroll
+  for (int b = 0; b < NB; b++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) o[b][r] = 0.0f;
+  float m = -INFINITY, l = 0.0f;
 #pragma unroll 1
-  for (int key = k0; key < k1; key++) {
-    const size_t at = (size_t)key_row(a.kv, stab, blk0, it.kbase, key) * rs + (size_t)kvh * D +
-                      (size_t)(DH * dpart);
-    float s = 0.0f;
+  for (int kt = it.ks; kt < any_hi; kt += KT) {
+    if (kt + KT <= any_lo) continue;
+    const bool full = kt >= all_lo && kt + KT <= min(all_hi, it.ke);
+    const int64_t row = key_row(a.kv, table, 0, it.kbase, min(kt + i, it.ke - 1));
+    const float *kp = kbase + (size_t)row * rs;
+    f32x16 st, su;
 #pragma unroll
-    for (int c = 0; c < DH; c += 4) {
-      const float4 x = ld4(a.kv.k + at + c);
-      s = fmaf(x.x, q[c], s);
-      s = fmaf(x.y, q[c + 1], s);
-      s = fmaf(x.z, q[c + 2], s);
-      s = fmaf(x.w, q[c + 3], s);
+    for (int r = 0; r < 16; r++) st[r] = su[r] = 0.0f;
+#pragma unroll 2
+    for (int s = 0; s < D; s += 16) {
+      const float4 x = ld4(kp + s), y = ld4(qp + s), z = ld4(kp + s + 8), w = ld4(qp + s + 8);
+      st = __builtin_amdgcn_mfma_f32_32x32x2f32(x.x, y.x, st, 0, 0, 0);
+      su = __builtin_amdgcn_mfma_f32_32x32x2f32(z.x, w.x, su, 0, 0, 0);
+      st = __builtin_amdgcn_mfma_f32_32x32x2f32(x.y, y.y, st, 0, 0, 0);
+      su = __builtin_amdgcn_mfma_f32_32x32x2f32(z.y, w.y, su, 0, 0, 0);
+      st = __builtin_amdgcn_mfma_f32_32x32x2f32(x.z, y.z, st, 0, 0, 0);
+      su = __builtin_amdgcn_mfma_f32_32x32x2f32(z.z, w.z, su, 0, 0, 0);
+      st = __builtin_amdgcn_mfma_f32_32x32x2f32(x.w, y.w, st, 0, 0, 0);
+      su = __builtin_amdgcn_mfma_f32_32x32x2f32(z.w, w.w, su, 0, 0, 0);
     }
+    st += su;
+    float mx = -INFINITY;
 #pragma unroll
-    for (int x = 32; x >= QN; x >>= 1) s += __shfl_xor(s, x, 64);
-    s *= sl2;
-    const bool seen = key >= lo && key <= aq;
-    const float mn = seen && s > m ? s : m;
+    for (int r = 0; r < 16; r++) {
+      const int key = kt + 8 * (r >> 2) + 4 * half + (r & 3);
+      st[r] = full || (key >= vis_lo && key <= aq && key < it.ke) ? st[r] * sl2 : -INFINITY;
+      mx = fmaxf(mx, st[r]);
+    }
+    const float mn = fmaxf(m, max_halves(mx));
+    const float alpha = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - mn);
     const float ms = mn == -INFINITY ? 0.0f : mn;
-    const float alpha = m == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m - ms);
-    const float p = seen ? __builtin_amdgcn_exp2f(s - ms) : 0.0f;
-    if (mn != m) {
-      l *= alpha;
+    m = mn;
+    float lt[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-      for (int c = 0; c < DH; c++) o[c] *= alpha;
-      m = mn;
+    for (int r = 0; r < 16; r++) {
+      st[r] = __builtin_amdgcn_exp2f(st[r] - ms);
+      lt[r >> 2] += st[r];
     }
-    if (seen) {
-      l += p;
+    l = fmaf(l, alpha, (lt[0] + lt[1]) + (lt[2] + lt[3]));
+    f32x16 t[NB];
 #pragma unroll
-      for (int c = 0; c < DH; c += 4) {
-        const float4 x = ld4(a.kv.v + at + c);
-        o[c] = fmaf(p, x.x, o[c]);
-        o[c + 1] = fmaf(p, x.y, o[c + 1]);
-        o[c + 2] = fmaf(p, x.z, o[c + 2]);
-        o[c + 3] = fmaf(p, x.w, o[c + 3]);
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) t[b][r] = 0.0f;
+    bool odd = false;  // an infinity or NaN in V: no product with the 0 of a query that does not see it
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      if (r % 4 == 0) __builtin_amdgcn_sched_barrier(0);  // four steps' loads in flight
+      const int64_t vrow = __shfl((long long)row, 8 * (r >> 2) + 4 * half + (r & 3), 64);
+      const float *vp = vbase + (size_t)vrow * rs + i;
+#pragma unroll
+      for (int b = 0; b < NB; b++) {
+        const float v = vp[32 * b];
+        odd |= !(fabsf(v) < INFINITY);
+        t[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(v, st[r], t[b], 0, 0, 0);
       }
     }
+    if (!full && __any(odd)) {
+#pragma unroll
+      for (int b = 0; b < NB; b++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) t[b][r] = 0.0f;
+#pragma unroll 1
+      for (int k = 0; k < min(KT, any_hi - kt); k++) {
+        float p = st[0];  // of key k, in the lanes that hold it, then in both halves
+#pragma unroll
+        for (int r = 1; r < 16; r++) p = r == 4 * (k >> 3) + (k & 3) ? st[r] : p;
+        p = __shfl(p, i + 32 * ((k >> 2) & 1), 64);
+        const float *vp = vbase + (size_t)__shfl((long long)row, k, 64) * rs + 4 * half;
+        const bool seen = kt + k >= vis_lo && kt + k <= aq;
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+          for (int r = 0; r < 16; r += 4) {
+            if (r == 0) __builtin_amdgcn_sched_barrier(0);
+            const float4 v = ld4(vp + 32 * b + 2 * r);
+            t[b][r] = seen ? fmaf(p, v.x, t[b][r]) : t[b][r];
+            t[b][r + 1] = seen ? fmaf(p, v.y, t[b][r + 1]) : t[b][r + 1];
+            t[b][r + 2] = seen ? fmaf(p, v.z, t[b][r + 2]) : t[b][r + 2];
+            t[b][r + 3] = seen ? fmaf(p, v.w, t[b][r + 3]) : t[b][r + 3];
+          }
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < NB; b++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) o[b][r] = fmaf(o[b][r], alpha, t[b][r]);
   }
+  l = sum_halves(l);
   if (!qvalid) return;
   const Dest d = destination(a, it, qi, h, D);
-  const float inv = d.partial ? 1.0f : (l == 0.0f ? 0.0f : 1.0f / l);
+  const float f = d.partial ? 1.0f : l == 0.0f ? 0.0f : 1.0f / l;
 #pragma unroll
-  for (int c = 0; c < DH; c += 4)
-    *reinterpret_cast<float4 *>(d.row + DH * dpart + c) =
-        make_float4(o[c] * inv, o[c + 1] * inv, o[c + 2] * inv, o[c + 3] * inv);
-  if (d.partial && dpart == 0) {
+  for (int b = 0; b < NB; b++)
+#pragma unroll
+    for (int r = 0; r < 16; r += 4)
+      *reinterpret_cast<float4 *>(d.row + v0 + 32 * b + 2 * r + 4 * half) =
+          make_float4(o[b][r] * f, o[b][r + 1] * f, o[b][r + 2] * f, o[b][r + 3] * f);
+  if (d.partial && half == 0 && v0 == 0) {
     a.part_m[d.pidx] = m;
     a.part_l[d.pidx] = l;
   }
@@ -226,6 +285,19 @@ __device__ __forceinline__ int value_unit(int e, int unit, int &top) {
                                                 : unit;
 }
 
+// The segments of a slot that a wave takes again, after all of them (in the loop over the segments
+// that code would take registers from the tiles).  From the 64th on they share a bit: some may be
+// taken again for nothing.
+struct Again {
+  int first;
+  uint64_t bits;
+  __device__ void add(int seg) { bits |= 1ull << min(seg - first, 63); }
+  __device__ int next(int seg, int end) const {
+    while (seg < end && !(bits >> min(seg - first, 63) & 1)) seg++;
+    return seg;
+  }
+};
+
 // What the steps of the split add to the error of a query's o in one tile, p being the sum of the
 // lane's (scaled) probabilities: half a step of lo, 2^-25 and 2^-25.8 on average, in each of 16
 // probabilities beside |v| of up to 2^15, and in each v.
@@ -233,11 +305,9 @@ __device__ __forceinline__ float split_steps(float p) {
   return fmaf(p, 0x1p-26f, fminf(p * 0x1p15f, 0x1p-9f));
 }
 
-// Whether a query's sums (o in units of 2^kProbExp and the V scale; every lane of the query has
-// its part) cannot stand: one is not finite, or the split's steps, e, are more than 2^-21 of the
-// largest result.
+// A query's largest result over a wave's dims; -INFINITY if one of them is not finite.
 template <int NB>
-__device__ __forceinline__ bool unsound(const f32x16 (&o)[NB], float l, float e, int v_top) {
+__device__ __forceinline__ float largest_result(const f32x16 (&o)[NB], float l) {
   float zero = 0.0f * l, top = 0.0f;
 #pragma unroll
   for (int b = 0; b < NB; b++)
@@ -246,9 +316,18 @@ __device__ __forceinline__ bool unsound(const f32x16 (&o)[NB], float l, float e,
       zero = fmaf(0.0f, o[b][r], zero);  // NaN if any is not finite
       top = fmaxf(top, fabsf(o[b][r]));
     }
-  top = max_halves(top);
-  // (At the smallest scale, V holds nothing but zeros and values below 2^-105.)
-  return !(zero == 0.0f) || (top < e * 0x1p21f && v_top > kMinExp);
+  const float x = zero == 0.0f ? top : -INFINITY;
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
+                                                  false);
+  const float y = __uint_as_float(r[0]), z = __uint_as_float(r[1]);
+  return fminf(y, z) < 0.0f ? -INFINITY : fmaxf(y, z);
+}
+
+// Whether a query's sums (o in units of 2^kProbExp and the V scale) cannot stand: one is not finite,
+// or the split's steps, e, are more than 2^-21 of the largest result.  (At the smallest scale, V
+// holds nothing but zeros and values below 2^-105.)
+__device__ __forceinline__ bool unsound(float result, float e, int v_top) {
+  return result < 0.0f || (result < e * 0x1p21f && v_top > kMinExp);
 }
 
 // The factor of a query's sums in its result: 1 / l or, in a partial, to the largest max.
@@ -436,7 +515,8 @@ prefill_split_kernel(TileLaunch a) {
   const float *vbase = a.kv.v + (size_t)kvh * D;
   const float one = opaque_one();
 
-  for (int seg = a.seg_off[slot]; seg < seg_end; seg++) {
+  Again again{a.seg_off[slot], 0};
+  for (int seg = again.first; seg < seg_end; seg++) {
     // Every wave is done with the previous segment's LDS tiles and table before they are reused.
     __syncthreads();
     const TileItem it = a.items[seg];
@@ -627,8 +707,8 @@ prefill_split_kernel(TileLaunch a) {
 
     if (!wave_active) continue;
     const float l_tot = sum_halves(l_run);
-    if (__any(coarse || unsound<NB>(o, l_tot, sum_halves(e_run), v_top))) {
-      scan_segment<D, 1>(a, it, stab, share.blk0, kvh, h, wq0);
+    if (__any(coarse || unsound(largest_result<NB>(o, l_tot), sum_halves(e_run), v_top))) {
+      again.add(seg);
       continue;
     }
     if (!qvalid) continue;
@@ -645,6 +725,10 @@ prefill_split_kernel(TileLaunch a) {
       a.part_m[d.pidx] = m_top;
       a.part_l[d.pidx] = l_tot * f;
     }
+  }
+  for (int seg = again.next(again.first, seg_end); seg < seg_end; seg = again.next(seg + 1, seg_end)) {
+    const TileItem it = a.items[seg];
+    if (it.q0 + qb * QW < it.qlen) fp32_segment<D, NB>(a, it, kvh, h, it.q0 + qb * QW, 0);
   }
 }
 
@@ -691,7 +775,8 @@ prefill_split_wide_kernel(TileLaunch a) {
   const size_t rs = (size_t)a.hkv * D;
   const float one = opaque_one();
 
-  for (int seg = a.seg_off[slot]; seg < seg_end; seg++) {
+  Again again{a.seg_off[slot], 0};
+  for (int seg = again.first; seg < seg_end; seg++) {
     __syncthreads();
     const TileItem it = a.items[seg];
     const int off = it.klen - it.qlen;
@@ -902,9 +987,18 @@ prefill_split_wide_kernel(TileLaunch a) {
     }
 
     const float l_tot = sum_halves(l_run);
-    if (__syncthreads_or(coarse || unsound<NB>(o, l_tot, sum_halves(e_run), v_top))) {
-      const int q0 = wq0 + ds * (QW / DS);
-      if (q0 < it.qlen) scan_segment<D, DS>(a, it, stab, share.blk0, kvh, h, q0);
+    // The waves that share the queries decide together, over all of their dims.
+    float result = coarse ? -INFINITY : largest_result<NB>(o, l_tot);
+    float *results = &spart[0][0][0][0];
+    if (half == 0) results[wave * QW + i] = result;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < DS; j++) {
+      const float x = results[(qg * DS + j) * QW + i];
+      result = result < 0.0f || x < 0.0f ? -INFINITY : fmaxf(result, x);
+    }
+    if (__any(unsound(result, sum_halves(e_run), v_top))) {
+      again.add(seg);
       continue;
     }
     if (!qvalid) continue;
@@ -920,6 +1014,10 @@ prefill_split_wide_kernel(TileLaunch a) {
       a.part_m[d.pidx] = m_top;
       a.part_l[d.pidx] = l_tot * f;
     }
+  }
+  for (int seg = again.next(again.first, seg_end); seg < seg_end; seg = again.next(seg + 1, seg_end)) {
+    const TileItem it = a.items[seg];
+    if (it.q0 + qb * QW < it.qlen) fp32_segment<D, NB>(a, it, kvh, h, it.q0 + qb * QW, DW * ds);
   }
 }
 

@@ -6,8 +6,8 @@ where it adds nothing to the result: a sink key with no V, a V row that no query
 of unlike size, a V channel far above the others.  Each query row of each head is compared with
 float64 by itself (channels of unlike size by themselves).
 
-Bar: 1e-5, the attention bar: up to 4096 fp32 products per output give sqrt(4096) * 2^-24 = 3.8e-6 if
-their roundings are independent, a few times that where they cancel."""
+Bar: 4e-6.  Up to 4096 fp32 products per output give sqrt(4096) * 2^-24 = 3.8e-6 if their
+roundings are independent.  (The fp32 tiles reach 0.6e-6 to 7e-6 on these inputs.)"""
 
 import numpy as np
 import pytest
@@ -21,7 +21,7 @@ from test_gpu_prefill_split import exact
 
 pytestmark = pytest.mark.gpu
 
-BAR = 1e-5
+BAR = 4e-6
 N = 4096
 HEADS = [(64, 1), (64, 4), (128, 2), (256, 4), (512, 2)]
 
@@ -82,7 +82,7 @@ def check(ctx, case, name, channels=slice(None), rows=slice(None), bar=BAR):
 
 
 @pytest.mark.parametrize("v", [0.0, 1e-3])
-@pytest.mark.parametrize("weight", [0.7, 0.98])
+@pytest.mark.parametrize("weight", [0.7, 0.98, 0.9995])
 @pytest.mark.parametrize("d,rep", HEADS)
 def test_sink_key(ctx, d, rep, weight, v):
     """The first key takes most of the weight (of the last row; more of the earlier ones) and adds
@@ -114,3 +114,12 @@ def test_v_tiles_of_unlike_size(ctx, d, rep, span):
     small = 32 * int(np.argmax((t[::32] * 5) % (span + 1) == span))
     set_score(case, small + 3, sink_score(1.0 - 2.0 ** -(span + 1), N))
     check(ctx, case, f"v tiles d{d} rep{rep} span {span}")
+
+
+@pytest.mark.parametrize("d,rep", HEADS)
+def test_zero_dims(ctx, d, rep):
+    """Half of V's dims zero (at d = 256 and 512 those of whole waves), and keys without any V."""
+    case = build(d, rep, seed=16)
+    case.v[:, :, d // 2:] = 0.0
+    case.v[100:400] = 0.0
+    check(ctx, case, f"zero dims d{d} rep{rep}")
