@@ -71,6 +71,11 @@ constexpr float kMaxScoreUnit = 0x1p-13f;
 // The exponent of V's scale stays for tiles of up to kUnitSlack below it and within kUnitSpan of the
 // largest one's.
 constexpr int kUnitSlack = 3, kUnitSpan = 32;
+// Eight keys of a V dim are held to 2^-22 of the largest of them, or better, if that is at least
+// 2^-kDimBits of the most that the scale takes: 2^-14 (a tile at the low end of kUnitSlack) to 2^-18
+// of the tile's largest |v|.  A segment with a smaller chunk (a channel far above the others) is not
+// for the split: the row as a whole would not show what those dims lose.
+constexpr int kDimBits = 18;
 constexpr int KT = 32;                // keys per tile
 constexpr int kAhead = 2;             // operand reads in flight ahead of their products
 constexpr int kKeepReads = 0x6;       // sched_barrier: only VALU and SALU move across
@@ -298,6 +303,11 @@ struct Again {
   }
 };
 
+// The size below which a dim's keys are too small for a V scale of this exponent.
+__device__ __forceinline__ float dim_limit(int unit) {
+  return __uint_as_float((uint32_t)max(unit + 1 - kDimBits, 0) << 23);
+}
+
 // What the steps of the split add to the error of a query's o in one tile, p being the sum of the
 // lane's (scaled) probabilities: half a step of lo, 2^-25 and 2^-25.8 on average, in each of 16
 // probabilities beside |v| of up to 2^15, and in each v.
@@ -352,7 +362,7 @@ struct TileShare {
   const float *k, *v;  // of this KV head
   size_t rs;           // floats per token
   const int32_t *stab;
-  int blk0, kbase, ke;
+  int blk0, kbase, ks, ke;
   int wave, lane;
   int cur_page, cur_id;  // page whose block id cur_id holds (wave-uniform)
 
@@ -462,6 +472,22 @@ struct TileShare {
     for (int u = 0; u < UW; u++) m = abs_max(m, r[u]);
     return m;
   }
+  // Whether least_chunk() of the segment's tile t says something about the dims: not where rows past
+  // the end repeat its last key, unless there is no other tile.
+  __device__ bool dims_count(int t) const {
+    return ks + (t + 1) * KT <= ke || ke - ks <= KT;
+  }
+  // The smallest of the lane's V chunks (eight keys of one dim), by the largest value of each; chunks
+  // of zeros don't count.
+  static __device__ float least_chunk(const f32x8 (&r)[UW]) {
+    float m = INFINITY;
+#pragma unroll
+    for (int u = 0; u < UW; u++) {
+      const float x = abs_max(0.0f, r[u]);
+      m = fminf(m, x > 0.0f ? x : INFINITY);
+    }
+    return m;
+  }
 };
 
 // Stages a segment's block ids in LDS, so that the tile loads never wait on a global load;
@@ -492,6 +518,7 @@ prefill_split_kernel(TileLaunch a) {
   __shared__ __attribute__((aligned(16))) _Float16 sv[2][2 * PART];
   __shared__ __attribute__((aligned(16))) float smax[2][2][NW];  // each wave's largest |k|, |v|
   __shared__ int32_t stab[kPrefillTablePages];  // block ids of the pages this chunk touches
+  __shared__ int uneven;  // a tile's V dims are too unlike for one scale
 
   const int slot = blockIdx.x;
   const int seg_end = a.seg_off[slot + 1];
@@ -519,6 +546,7 @@ prefill_split_kernel(TileLaunch a) {
   for (int seg = again.first; seg < seg_end; seg++) {
     // Every wave is done with the previous segment's LDS tiles and table before they are reused.
     __syncthreads();
+    if (threadIdx.x == 0) uneven = 0;
     const TileItem it = a.items[seg];
     const int off = it.klen - it.qlen;  // absolute position of query 0
     // This lane's query (column i of S^T) and its visible key range.
@@ -538,7 +566,7 @@ prefill_split_kernel(TileLaunch a) {
     const int whi_max = off + wq1 + 1;
 
     // The first tile's loads are issued before Q is read: a short segment waits once for both.
-    TileShare<D, NW> share{a.kv, kbase, vbase, rs, stab, stage_table(a, it, stab), it.kbase, it.ke,
+    TileShare<D, NW> share{a.kv, kbase, vbase, rs, stab, stage_table(a, it, stab), it.kbase, it.ks, it.ke,
                            wave, lane, -1, 0};
     f32x8 rk[UW], rv[UW];  // this wave's share of the next tile, as loaded
     auto load_tile = [&](int kt) {
@@ -578,8 +606,10 @@ prefill_split_kernel(TileLaunch a) {
 
     // The tile in rk / rv: each wave's largest magnitudes, then (after a barrier) the exponents of
     // its scales, and its parts in LDS.
-    auto share_max = [&](int b) {
+    float v_least = 0.0f;
+    auto share_max = [&](int b, int t) {
       const float m = max_waves(share.largest(rk), share.largest(rv));
+      v_least = share.dims_count(t) ? share.least_chunk(rv) : INFINITY;
       if (i == 0) smax[b][half][wave] = m;
     };
     int k_exp_in = kMinExp, v_unit = kMinExp, v_top = kMinExp;
@@ -589,6 +619,7 @@ prefill_split_kernel(TileLaunch a) {
       v_unit = value_unit(sc.b, v_unit, v_top);
     };
     auto store_tile = [&](int b) {
+      if (__any(v_least < dim_limit(v_unit))) uneven = 1;
       share.store_k(rk, split_scale(k_exp_in), sk[b]);
       share.store_v(rv, split_scale(v_unit), sv[b]);
     };
@@ -690,7 +721,7 @@ prefill_split_kernel(TileLaunch a) {
     // At the barrier of tile t every wave is done with tile t - 1, whose buffer takes tile
     // t + 1, tile t is in LDS, and so are the largest magnitudes of tile t + 1.
     const int ntiles = (it.ke - it.ks + KT - 1) / KT;
-    share_max(0);
+    share_max(0, 0);
     __syncthreads();
     take_scales(0);
     store_tile(0);
@@ -699,7 +730,7 @@ prefill_split_kernel(TileLaunch a) {
       const int kt = it.ks + t * KT;
       const int b = t & 1;
       const int k_exp = k_exp_in, v_exp = v_unit;
-      share_max(b ^ 1);  // the last tile stores itself once more, where nothing reads it
+      share_max(b ^ 1, t + 1);  // the last tile stores itself once more, where nothing reads it
       __syncthreads();
       take_scales(b ^ 1);
       compute_tile(kt, sk[b], sv[b], k_exp, v_exp, b ^ 1, t + 2 < ntiles ? kt + 2 * KT : -1);
@@ -707,7 +738,7 @@ prefill_split_kernel(TileLaunch a) {
 
     if (!wave_active) continue;
     const float l_tot = sum_halves(l_run);
-    if (__any(coarse || unsound(largest_result<NB>(o, l_tot), sum_halves(e_run), v_top))) {
+    if (__any(coarse || uneven || unsound(largest_result<NB>(o, l_tot), sum_halves(e_run), v_top))) {
       again.add(seg);
       continue;
     }
@@ -755,6 +786,7 @@ prefill_split_wide_kernel(TileLaunch a) {
   __shared__ __attribute__((aligned(16))) float spart[SLOTS][4][64][4];  // partial S^T
   __shared__ float smax[2][NW];  // each wave's largest |k| (of the next tile), |v|
   __shared__ int32_t stab[kPrefillTablePages];
+  __shared__ int uneven;  // a tile's V dims are too unlike for one scale
 
   const int slot = blockIdx.x;
   const int seg_end = a.seg_off[slot + 1];
@@ -778,6 +810,7 @@ prefill_split_wide_kernel(TileLaunch a) {
   Again again{a.seg_off[slot], 0};
   for (int seg = again.first; seg < seg_end; seg++) {
     __syncthreads();
+    if (threadIdx.x == 0) uneven = 0;
     const TileItem it = a.items[seg];
     const int off = it.klen - it.qlen;
     const int wq0 = it.q0 + qb * QW;
@@ -796,7 +829,7 @@ prefill_split_wide_kernel(TileLaunch a) {
 
     // The first tile's loads are issued before Q is read: a short segment waits once for both.
     TileShare<D, NW> share{a.kv, a.kv.k + (size_t)kvh * D, a.kv.v + (size_t)kvh * D, rs, stab,
-                           stage_table(a, it, stab), it.kbase, it.ke, wave, lane, -1, 0};
+                           stage_table(a, it, stab), it.kbase, it.ks, it.ke, wave, lane, -1, 0};
     f32x8 rk[UW], rv[UW];
     share.load_k(it.ks, rk);
     share.load_v(it.ks, rv);
@@ -838,9 +871,15 @@ prefill_split_wide_kernel(TileLaunch a) {
       k_exp_in = sc.a;
       share.store_k(rk, split_scale(sc.a), sk);
     };
+    float v_least = 0.0f;
+    auto share_v_max = [&](int t) {
+      share_max(1, share.largest(rv));
+      v_least = share.dims_count(t) ? share.least_chunk(rv) : INFINITY;
+    };
     auto store_v = [&]() {
       const TileExps sc = tile_exps<NW>(smax[1][lane & 7]);
       v_exp = value_unit(sc.a, v_exp, v_top);
+      if (__any(v_least < dim_limit(v_exp))) uneven = 1;
       share.store_v(rv, split_scale(v_exp), sv);
     };
     auto read_split = [&](const _Float16 *p) {
@@ -850,7 +889,7 @@ prefill_split_wide_kernel(TileLaunch a) {
 
     const int ntiles = (it.ke - it.ks + KT - 1) / KT;
     share_max(0, share.largest(rk));
-    share_max(1, share.largest(rv));
+    share_v_max(0);
     __syncthreads();
     store_k();
     if (ntiles > 1) share.load_k(it.ks + KT, rk);
@@ -869,9 +908,10 @@ prefill_split_wide_kernel(TileLaunch a) {
 #pragma unroll
       for (int r = 0; r < 16; r++) st[r] = 0.0f;
       if (active) {
-        auto read_k = [&](int s) {
-          return read_split(sk + k_pos<D>(i, (DW / 8) * ds + 2 * s + half));
-        };
+        // k_pos<D>(i, 16 ds + 2 s + half); opaque, or the compiler keeps all of them, in scratch.
+        int at = k_pos<D>(i, (DW / 8) * ds + half);
+        asm volatile("" : "+v"(at));
+        auto read_k = [&](int s) { return read_split(sk + (at ^ (s << 4))); };
         Split8 f[kAhead + 1];
 #pragma unroll
         for (int s = 0; s < kAhead; s++) f[s] = read_k(s);
@@ -982,13 +1022,13 @@ prefill_split_wide_kernel(TileLaunch a) {
           o[u % NB] = mfma_split(f[u % (kAhead + 1)], p[u / NB], o[u % NB]);
         }
       }
-      if (more) share_max(1, share.largest(rv));
+      if (more) share_v_max(t + 1);
       __syncthreads();
     }
 
     const float l_tot = sum_halves(l_run);
     // The waves that share the queries decide together, over all of their dims.
-    float result = coarse ? -INFINITY : largest_result<NB>(o, l_tot);
+    float result = coarse || uneven ? -INFINITY : largest_result<NB>(o, l_tot);
     float *results = &spart[0][0][0][0];
     if (half == 0) results[wave * QW + i] = result;
     __syncthreads();

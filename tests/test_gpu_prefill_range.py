@@ -116,6 +116,15 @@ def test_v_tiles_of_unlike_size(ctx, d, rep, span):
     check(ctx, case, f"v tiles d{d} rep{rep} span {span}")
 
 
+@pytest.mark.parametrize("bits", [12, 20, 24, 30])
+@pytest.mark.parametrize("d,rep", HEADS)
+def test_v_channel(ctx, d, rep, bits):
+    """One V channel 2^bits above the others, which are compared without it."""
+    case = build(d, rep, seed=14)
+    case.v[:, :, 5] *= np.float32(2.0 ** bits)
+    check(ctx, case, f"v channel d{d} rep{rep} 2^{bits}", channels=np.r_[:5, 6:d])
+
+
 @pytest.mark.parametrize("d,rep", HEADS)
 def test_zero_dims(ctx, d, rep):
     """Half of V's dims zero (at d = 256 and 512 those of whole waves), and keys without any V."""
