@@ -125,6 +125,17 @@ def test_v_channel(ctx, d, rep, bits):
     check(ctx, case, f"v channel d{d} rep{rep} 2^{bits}", channels=np.r_[:5, 6:d])
 
 
+@pytest.mark.parametrize("bits", [8, 12, 13, 14, 15, 17])
+@pytest.mark.parametrize("d,rep", HEADS)
+def test_k_channel(ctx, d, rep, bits):
+    """One K channel 2^bits above the others where q is 0, so that no score shows it: the rows of a
+    few keys, where a score's error shows most.  Bar: 3 sqrt(32) * 2^-24."""
+    case = build(d, rep, seed=15)
+    case.q[:, :, 5] = 0.0
+    case.k[:, :, 5] *= np.float32(2.0 ** bits)
+    check(ctx, case, f"k channel d{d} rep{rep} 2^{bits}", rows=slice(0, 32), bar=1e-6)
+
+
 @pytest.mark.parametrize("d,rep", HEADS)
 def test_zero_dims(ctx, d, rep):
     """Half of V's dims zero (at d = 256 and 512 those of whole waves), and keys without any V."""
