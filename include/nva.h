@@ -97,7 +97,9 @@ const char *nva_status_string(nva_status status);
 /* Per-kernel timing with HIP events on the context's stream (off by default).  Kernel names:
  * "rope_store", "store", "decode", "merge", "prefill", "gather", "linear", "rms_norm";
  * "attention" spans the attention kernels of one call (decode and prefill kernels that
- * overlap count once).  Host-side entries: "plan" (building a step's work plan on the host, once
+ * overlap count once).  "prefill_split" and "prefill_fp32" are the part of "prefill" that each of
+ * its two tile kernels took, "linear_tiles" the part of "linear" of its 128 x 128-tile kernel.
+ * Host-side entries: "plan" (building a step's work plan on the host, once
  * per step and attention configuration, at its first layer) and "plan_upload" (copying it to
  * the device).  The name "device_bytes" instead returns in *launches the bytes of device memory
  * the context's grow-only work buffers hold (arenas and RoPE tables excluded). */

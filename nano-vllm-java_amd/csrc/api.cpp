@@ -200,7 +200,7 @@ struct Scratch {
 };
 
 struct PendingTiming {
-  std::string name;
+  const char *name, *variant;  // variant: null, or the second entry that counts it
   hipEvent_t start, stop;
 };
 
@@ -342,14 +342,15 @@ hipEvent_t take_event(nva_ctx *ctx) {
   return e;
 }
 
-// Brackets one kernel launch with timing events when timing is on.
+// Brackets one kernel launch with timing events when timing is on.  A launch that one of several
+// kernels serves is counted under its own name (variant) too.
 struct Timed {
   nva_ctx *ctx;
-  const char *name;
+  const char *name, *variant;
   hipStream_t stream;
   hipEvent_t start = nullptr;
-  Timed(nva_ctx *c, const char *n, hipStream_t s = nullptr)
-      : ctx(c), name(n), stream(s ? s : c->stream) {
+  Timed(nva_ctx *c, const char *n, hipStream_t s = nullptr, const char *v = nullptr)
+      : ctx(c), name(n), variant(v), stream(s ? s : c->stream) {
     if (ctx->timing) {
       start = take_event(ctx);
       if (start) (void)hipEventRecord(start, stream);
@@ -360,7 +361,7 @@ struct Timed {
     hipEvent_t stop = take_event(ctx);
     if (!stop) return;
     (void)hipEventRecord(stop, stream);
-    ctx->pending.push_back({name, start, stop});
+    ctx->pending.push_back({name, variant, start, stop});
     start = nullptr;
   }
 };
@@ -370,9 +371,12 @@ void resolve_timings(nva_ctx *ctx) {
     float ms = 0.f;
     if (hipEventSynchronize(p.stop) == hipSuccess &&
         hipEventElapsedTime(&ms, p.start, p.stop) == hipSuccess) {
-      auto &s = ctx->stats[p.name];
-      s.launches++;
-      s.ms += ms;
+      for (const char *n : {p.name, p.variant}) {
+        if (!n) continue;
+        auto &s = ctx->stats[n];
+        s.launches++;
+        s.ms += ms;
+      }
     }
     ctx->event_pool.push_back(p.start);
     ctx->event_pool.push_back(p.stop);
@@ -1167,7 +1171,7 @@ nva_status run_attention(nva_ctx *ctx, const nva_attn_desc &d, const KvView &vie
     t.part_m = pm;
     t.part_l = pm + parts;
     t.part_acc = pm + 2 * parts;
-    Timed tm(ctx, "prefill");
+    Timed tm(ctx, "prefill", nullptr, tiles_fp32 ? "prefill_fp32" : "prefill_split");
     HIP_TRY(ctx,
             tiles_fp32 ? launch_prefill_fp32(t, hpw_tile, ctx->stream)
                        : launch_prefill_tiles(t, hpw_tile, ctx->stream),
@@ -2173,7 +2177,7 @@ nva_status nva_linear_forward(nva_ctx *ctx, const float *x, int rows, int in,
             "linear partial buffer");
     a.part = static_cast<float *>(ctx->d_lin.ptr);
   }
-  Timed tm(ctx, "linear");
+  Timed tm(ctx, "linear", nullptr, "linear_tiles");
   HIP_TRY(ctx, launch_linear(a, ctx->stream), "linear kernel launch");
   tm.done();
   return NVA_OK;

@@ -35,8 +35,13 @@ def data(rows, inf, outf, seed):
 
 
 def run(ctx, x, w, b=None):
+    ctx.reset_stats()
+    ctx.set_timing(True)
     y = Linear(dev(w), None if b is None else dev(b)).forward(dev(x), ctx)
     ctx.sync()
+    launches, _ = ctx.kernel_stats("linear_tiles")
+    ctx.set_timing(False)
+    assert launches == 1, "the tiled kernel did not run"
     return y.cpu().numpy().astype(np.float64)
 
 

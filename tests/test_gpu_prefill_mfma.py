@@ -1,7 +1,7 @@
-"""Parity of the fp32 MFMA prefill kernel over its whole configuration space, against the oracle.
+"""Parity of the prefill tile kernels over their configuration space, against the oracle.
 
-The prefill kernel is instantiated for head dims 64, 128, 256 and 512 and for 1, 2, 4 or 8 query
-heads per workgroup (GQA ratio 1, 2, 4, 8).  Each case mixes ragged sequences: a prefix hit
+Steps as small as these run on the fp32 tiles where that kernel is the faster one; the split kernel
+has tests of its own, on larger steps.  Head dims 64, 128, 256 and 512, GQA ratios 1, 2, 4 and 8.  Each case mixes ragged sequences: a prefix hit
 (full pages), a mid-page chunk start, a two-query sequence (the smallest MFMA tile), a one-query
 row (the row kernel) and lengths that leave partial query tiles and partial key tiles.  It runs
 paged with small and with the default page size, and dense (prefillDense), with and without a

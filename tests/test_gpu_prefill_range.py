@@ -61,11 +61,16 @@ def check(ctx, case, name, channels=slice(None), rows=slice(None), bar=BAR):
     try:
         ctx.set(**m.context_args())
         ctx.bind_kv_cache(arena)
+        ctx.reset_stats()
+        ctx.set_timing(True)
         out = Attention(wl.hq, wl.d, wl.scale, wl.hkv, wl.window, 0).forward(
             dev(case.q), dev(case.k), dev(case.v), ctx)
         ctx.sync()
         got = out.cpu().numpy().astype(np.float64)
+        launches, _ = ctx.kernel_stats("prefill_split")
+        assert launches == 1, "the split kernel did not run"
     finally:
+        ctx.set_timing(False)
         ctx.clear()
         arena.close()
     kc, vc = case.k_cache.copy(), case.v_cache.copy()

@@ -21,10 +21,11 @@ from nanollvm_amd import workloads as W
 pytestmark = pytest.mark.gpu
 
 # The last sequence gives the step work enough for the split kernel (steps of short sequences run
-# on the fp32 one).  A window leaves few keys per query, so it takes more queries.
+# on the fp32 one; every case checks which one ran).  A window leaves few keys per query, so it
+# takes more queries.
 SEQS = [(16, 70), (5, 33), (0, 2), (40, 190), (0, 31)]
 DENSE_SEQS = [(0, 70), (0, 33), (0, 2), (0, 190), (0, 31)]
-LONG, LONG_WINDOW = [(0, 2100)], [(0, 6300)]
+LONG, LONG_WINDOW = [(0, 2100)], [(0, 9000)]
 HEADS = [(64, 1), (64, 4), (128, 1), (128, 2), (256, 1), (256, 4), (512, 1), (512, 2)]
 
 
@@ -82,11 +83,16 @@ def check(ctx, case, name):
         ctx.bind_kv_cache(arena)
         with np.errstate(all="ignore"):
             want, kc, vc = case.oracle(threads=8)
+        ctx.reset_stats()
+        ctx.set_timing(True)
         out = Attention(wl.hq, wl.d, wl.scale, wl.hkv, wl.window, 0).forward(
             dev(case.q), dev(case.k), dev(case.v), ctx)
         ctx.sync()
         got = out.cpu().numpy().astype(np.float64)
+        launches, _ = ctx.kernel_stats("prefill_split")
+        assert launches == 1, "the split kernel did not run"
     finally:
+        ctx.set_timing(False)
         ctx.clear()
         arena.close()
     finite = all(np.isfinite(x).all() for x in (case.q, case.k, case.v))
@@ -102,13 +108,21 @@ def check(ctx, case, name):
     assert rel <= 1e-5, rel
 
 
-@pytest.mark.parametrize("layout", ["paged8", "paged16", "paged24", "paged4", "dense"])
+@pytest.mark.parametrize("layout", ["paged8", "paged16", "paged24", "paged4", "dense", "paged32",
+                                    "paged64", "paged256"])
 @pytest.mark.parametrize("window", [0, 37])
 @pytest.mark.parametrize("d,rep", HEADS)
 def test_page_sizes_and_window_starts(ctx, d, rep, window, layout):
-    """Pages of 8 tokens and more are read by whole runs, other sizes and unaligned window
-    starts row by row."""
+    """Full tiles inside one page and, over smaller pages of 8 tokens and more, aligned ones are read
+    by whole runs; other sizes, unaligned window starts and the last tile row by row."""
     check(ctx, build(d, rep, layout, window, seed=1), f"pages d{d} rep{rep} w{window} {layout}")
+
+
+@pytest.mark.parametrize("window", [0, 37])
+@pytest.mark.parametrize("d,rep", [(64, 2), (64, 8), (128, 4), (128, 8), (256, 2), (256, 8), (512, 4),
+                                   (512, 8)])
+def test_other_head_ratios(ctx, d, rep, window):
+    check(ctx, build(d, rep, "paged16", window, seed=8), f"heads d{d} rep{rep} w{window}")
 
 
 @pytest.mark.parametrize("layout", ["paged16", "dense"])
