@@ -533,9 +533,10 @@ nva_status get_plan(nva_ctx *ctx, const PlanKey &key, Plan **out) {
           ti.klen = klen;
           ti.kbase = kbase;
           ti.ks = W > 0 ? std::max(0, aq0 - W + 1) : 0;
-          // Over small pages key tiles start at multiples of 8 keys, where the kernel reads
-          // whole runs of rows from one page (the window masks the keys before it).
-          if (paged && key.block_size < 32 && !key.fp32_tiles) ti.ks &= ~7;
+          // Over pages of 8 and 16 tokens key tiles start at multiples of 8 keys, where the split
+          // kernel reads whole runs of rows from one page (the window masks the keys before it).
+          if (paged && (key.block_size == 8 || key.block_size == 16) && !key.fp32_tiles)
+            ti.ks &= ~7;
           ti.ke = aq1 + 1;
           ti.part = -1;
           ti.nsplit = 1;
