@@ -472,11 +472,10 @@ struct TileShare {
     for (int u = 0; u < UW; u++) m = abs_max(m, r[u]);
     return m;
   }
-  // Whether least_chunk() of the segment's tile t says something about the dims: not where rows past
-  // the end repeat its last key, unless there is no other tile.
-  __device__ bool dims_count(int t) const {
-    return ks + (t + 1) * KT <= ke || ke - ks <= KT;
-  }
+  // Of how many lanes' dims least_chunk() has to be too small in the segment's tile t.  One of eight
+  // keys is; where rows past the end repeat the last key, a chunk may be one value, which is small
+  // now and then, but not in many dims at once.
+  __device__ int dims_needed(int t) const { return ks + (t + 1) * KT <= ke ? 1 : 8; }
   // The smallest of the lane's V chunks (eight keys of one dim), by the largest value of each; chunks
   // of zeros don't count.
   static __device__ float least_chunk(const f32x8 (&r)[UW]) {
@@ -606,10 +605,12 @@ prefill_split_kernel(TileLaunch a) {
 
     // The tile in rk / rv: each wave's largest magnitudes, then (after a barrier) the exponents of
     // its scales, and its parts in LDS.
-    float v_least = 0.0f;
+    float v_least = INFINITY;
+    int v_needed = 1;
     auto share_max = [&](int b, int t) {
       const float m = max_waves(share.largest(rk), share.largest(rv));
-      v_least = share.dims_count(t) ? share.least_chunk(rv) : INFINITY;
+      v_least = share.least_chunk(rv);
+      v_needed = share.dims_needed(t);
       if (i == 0) smax[b][half][wave] = m;
     };
     int k_exp_in = kMinExp, v_unit = kMinExp, v_top = kMinExp;
@@ -619,7 +620,7 @@ prefill_split_kernel(TileLaunch a) {
       v_unit = value_unit(sc.b, v_unit, v_top);
     };
     auto store_tile = [&](int b) {
-      if (__any(v_least < dim_limit(v_unit))) uneven = 1;
+      if (__popcll(__ballot(v_least < dim_limit(v_unit))) >= v_needed) uneven = 1;
       share.store_k(rk, split_scale(k_exp_in), sk[b]);
       share.store_v(rv, split_scale(v_unit), sv[b]);
     };
@@ -871,15 +872,17 @@ prefill_split_wide_kernel(TileLaunch a) {
       k_exp_in = sc.a;
       share.store_k(rk, split_scale(sc.a), sk);
     };
-    float v_least = 0.0f;
+    float v_least = INFINITY;
+    int v_needed = 1;
     auto share_v_max = [&](int t) {
       share_max(1, share.largest(rv));
-      v_least = share.dims_count(t) ? share.least_chunk(rv) : INFINITY;
+      v_least = share.least_chunk(rv);
+      v_needed = share.dims_needed(t);
     };
     auto store_v = [&]() {
       const TileExps sc = tile_exps<NW>(smax[1][lane & 7]);
       v_exp = value_unit(sc.a, v_exp, v_top);
-      if (__any(v_least < dim_limit(v_exp))) uneven = 1;
+      if (__popcll(__ballot(v_least < dim_limit(v_exp))) >= v_needed) uneven = 1;
       share.store_v(rv, split_scale(v_exp), sv);
     };
     auto read_split = [&](const _Float16 *p) {

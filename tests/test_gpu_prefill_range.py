@@ -33,7 +33,7 @@ def ctx():
     c.close()
 
 
-def build(d, rep, seed, seqs=((0, N), (0, 77))):
+def build(d, rep, seed, seqs=((0, N), (0, 77), (0, 5), (0, 13))):
     rng = np.random.default_rng(seed)
     wl = W.build(f"range d{d} rep{rep}", list(seqs), is_prefill=True, hq=2 * rep, hkv=2, d=d,
                  scale=float(np.float32(d ** -0.5)), rng=rng, block_size=256, pool_cap=20000)
