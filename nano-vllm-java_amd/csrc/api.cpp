@@ -204,6 +204,12 @@ struct PendingTiming {
   hipEvent_t start, stop;
 };
 
+// Which tile kernel a layer configuration's prefill runs on in the current step.
+struct TileChoice {
+  int head_dim, num_heads, num_kv_heads, window;
+  bool fp32;
+};
+
 struct KernelStat {
   int64_t launches = 0;
   double ms = 0.0;
@@ -237,6 +243,7 @@ struct nva_ctx {
   size_t off_cu_q = 0, off_cu_k = 0, off_slots = 0, off_ctx = 0, off_tables = 0, off_pos = 0;
 
   std::vector<Plan *> plans;
+  std::vector<TileChoice> tile_choices;
   DevBuf d_part;     // split partials
   DevBuf d_q_rot;    // fused path scratch for rotated q
   DevBuf d_k_rot;    // fused path scratch for rotated k
@@ -921,12 +928,18 @@ KvView make_dense_view(const float *k, const float *v) {
 // Whether a prefill step runs on the fp32 tile kernel (prefill_fp32.hip) rather than the split one.
 // The split kernel multiplies 2.5 times as fast, but its tiles cover twice the queries, with half
 // the workgroups per CU, and a segment starts later; steps of a few short prompts or chunks leave
-// its waves idle.  Both kernels' times are estimated: the CU time of all key tiles (per tile, the
+// its waves idle.
+//
+// At d = 64 and 128 both kernels' times are estimated: the CU time of all key tiles (per tile, the
 // larger of a floor and the time of its active waves) over the CUs, or one tile's latency if that
-// is longer, plus the split kernel's later start.  The constants were fitted to the two kernels
-// on 54 drawn steps; fp32 / split us a layer at 40 q / 8 KV heads, d = 128: 2 + 16 + 208+3 tokens
-// 17.1 / 25.1, 230+11 and 211+15 21.1 / 27.5, 57 tokens 18.1 / 20.6, 280 tokens 45.7 / 36.7; at
-// d = 64, 140 and 245+58 tokens 27.4 / 29.3, 241+333 43.0 / 37.0; at d = 256, 1553+48 27.8 / 29.2.
+// is longer, plus the split kernel's later start.  At d = 512 the fp32 kernel takes steps of less
+// than 0.75 key tiles per CU, at d = 256 none.  On 560 drawn steps of 1-6 prompts or chunks, timed
+// with both kernels (profiles/prefill_tile_choice.md), the rule's time over the better kernel's is
+// 1.005 / 1.007 / 1.002 / 1.004 on average at d = 64 / 128 / 256 / 512.  fp32 / split us a layer
+// call: 32 q / 8 KV heads, d = 64, 70 tokens 14.4 / 16.1, 505 46.0 / 42.4; 16 q / 8 KV, d = 128, 160
+// tokens 23.0 / 27.1, 14+295 35.7 / 33.6; 4 q / 1 KV, d = 256, 22 and 3+7 15.7 / 16.3, 400 33.8 /
+// 32.0, 3736+100 43.6 / 36.6; 8 q / 1 KV, d = 512, 663+23 and 22 28.2 / 29.9, 300 42.2 / 39.0, 400
+// 52.0 / 44.6.
 bool use_fp32_tiles(nva_ctx *ctx, const nva_attn_desc &d, int hpw_fp32, int hpw_split, int window) {
   struct Cost {
     double floor, per_wave;  // CU us per key tile: at least, and per active wave
@@ -934,18 +947,7 @@ bool use_fp32_tiles(nva_ctx *ctx, const nva_attn_desc &d, int hpw_fp32, int hpw_
     int queries;             // queries (times heads) per wave
   };
   const int dim = d.head_dim;
-  const Cost fp32 = dim == 64    ? Cost{0.5, 0.28, 2, 16}
-                    : dim == 128 ? Cost{0.85, 0.56, 2, 16}
-                    : dim == 256 ? Cost{3.6, 1.2, 1, 16}
-                                 : Cost{5.0, 2.8, 1, 16};
-  const Cost split = dim == 64    ? Cost{0.6, 0.2, 3, 32}
-                     : dim == 128 ? Cost{2.5, 0.41, 1, 32}
-                     : dim == 256 ? Cost{6.5, 0.0, 1, 32}
-                                  : Cost{7.0, 0.0, 1, 32};
-  // us; at d = 256 and 512 with the per-row loads of segments that end inside a key tile (d = 256,
-  // 77+700 tokens: 45.6 / 51.5 us a layer, 2005+333 60.4 / 64.3; d = 512, 300+200 and 300 tokens:
-  // 63.5 / 73.3).
-  const double later = dim == 512 ? 10.0 : dim == 256 ? 9.0 : dim == 64 ? 3.5 : 2.0;
+  if (dim == 256) return false;
   auto estimate = [&](const Cost &c, int hpw, int tile_q) {
     double sum = 0.0, longest = 0.0;
     for (int b = 0; b < ctx->num_seqs; b++) {
@@ -963,8 +965,24 @@ bool use_fp32_tiles(nva_ctx *ctx, const nva_attn_desc &d, int hpw_fp32, int hpw_
     }
     return std::max(sum * (d.num_heads / hpw) / ctx->num_cus, longest);
   };
-  return estimate(fp32, hpw_fp32, prefill_fp32_tile_queries(dim, hpw_fp32)) <=
-         estimate(split, hpw_split, prefill_tile_queries(dim, hpw_split)) + later;
+  const int q_fp32 = prefill_fp32_tile_queries(dim, hpw_fp32);
+  const int q_split = prefill_tile_queries(dim, hpw_split);
+  if (dim == 512) return estimate(Cost{1.0, 0.0, 0, 32}, hpw_split, q_split) < 0.75;
+  const Cost fp32 = dim == 64 ? Cost{0.5, 0.28, 2, 16} : Cost{0.85, 0.56, 2, 16};
+  const Cost split = dim == 64 ? Cost{0.6, 0.2, 3, 32} : Cost{2.5, 0.41, 1, 32};
+  const double later = dim == 64 ? 3.5 : 2.0;  // us
+  return estimate(fp32, hpw_fp32, q_fp32) <= estimate(split, hpw_split, q_split) + later;
+}
+
+// The same for a layer, estimated once per step and configuration.
+bool fp32_tiles(nva_ctx *ctx, const nva_attn_desc &d, int hpw_fp32, int hpw_split, int window) {
+  for (const TileChoice &c : ctx->tile_choices)
+    if (c.head_dim == d.head_dim && c.num_heads == d.num_heads &&
+        c.num_kv_heads == d.num_kv_heads && c.window == window)
+      return c.fp32;
+  const bool fp32 = use_fp32_tiles(ctx, d, hpw_fp32, hpw_split, window);
+  ctx->tile_choices.push_back({d.head_dim, d.num_heads, d.num_kv_heads, window, fp32});
+  return fp32;
 }
 
 // The plan of one attention call (the descriptor, the step, and whether keys are paged over
@@ -992,7 +1010,7 @@ nva_status attention_plan(nva_ctx *ctx, const nva_attn_desc &d, int paged, int b
   const bool mfma = ctx->is_prefill && prefill_kernel_supports(d.head_dim, *hpw_tile);
   const int window = d.sliding_window > 0 ? d.sliding_window : 0;
   const int hpw_fp32 = largest_pow2_divisor_upto(rep, prefill_fp32_max_heads(d.head_dim));
-  const bool fp32 = mfma && use_fp32_tiles(ctx, d, hpw_fp32, *hpw_tile, window);
+  const bool fp32 = mfma && fp32_tiles(ctx, d, hpw_fp32, *hpw_tile, window);
   if (fp32) *hpw_tile = hpw_fp32;
   if (tiles_fp32) *tiles_fp32 = fp32;
   // The MFMA row kernel carries up to 16 heads of one KV head (it is used from 5).  Rows that
@@ -1716,6 +1734,7 @@ nva_status nva_step_set(nva_ctx *ctx, int is_prefill, const int32_t *cu_q, const
   if (block_tables && bt_stride <= 0 && num_seqs > 0)
     return fail(ctx, NVA_E_ARG, "block tables need bt_stride > 0");
   for (Plan *p : ctx->plans) p->valid = false;
+  ctx->tile_choices.clear();
   ctx->has_step = true;
   ctx->is_prefill = is_prefill != 0;
   ctx->num_seqs = num_seqs;
@@ -1820,6 +1839,7 @@ nva_status nva_step_clear(nva_ctx *ctx) {
   if (!ctx) return NVA_E_ARG;
   ctx->has_step = false;
   for (Plan *p : ctx->plans) p->valid = false;
+  ctx->tile_choices.clear();
   return NVA_OK;
 }
 

@@ -1,7 +1,8 @@
 // Kernel (c) for small steps: varlen causal prefill on fp32 MFMA over dense K/V or the paged KV
 // cache.  Steps of a few short prompts or chunks are bound by the latency of a workgroup's first
 // tiles, which is shorter here (no split, one barrier fewer, half the queries per workgroup, two
-// workgroups per CU) than in prefill.hip; all others run there (use_fp32_tiles).
+// workgroups per CU) than in prefill.hip; all others, and all at d = 256, run there
+// (use_fp32_tiles).
 //
 // Semantics (layers/Attention.java:245-280 prefillDense / prefillWithCache, :328-396
 // attendJobs): query qi of a sequence with qLen queries and kLen keys sits at absolute
@@ -123,12 +124,11 @@ __device__ __forceinline__ int64_t tile_row(const KvView &kv, const int32_t *sta
 
 }  // namespace
 
-// NW waves per workgroup, KT keys per tile.  Four waves per SIMD (at most 128 VGPRs) for
-// d <= 128; d = 256 needs more than 128 registers for its Q and O blocks, and d = 512 keeps
-// its O blocks in AGPRs (one wave per SIMD).
-template <int D, int HPW, int KT, int NW>
-__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(D <= 128 ? 4 : 1)))
+// Head dims 64 and 128: four waves per SIMD (at most 128 VGPRs).
+template <int D, int HPW>
+__global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
 prefill_kernel(TileLaunch a) {
+  constexpr int KT = 32, NW = 8;   // keys per tile, waves per workgroup
   constexpr int KB = KT / 16;      // 16-key MFMA blocks per key tile
   constexpr int DQ = D / 4;        // QK contraction steps per lane group g: dims [DQ*g, DQ*g+DQ)
   constexpr int NB = D / 16;       // O^T blocks of 16 dims: block 4*hh+bb holds dims 64*hh+4r+bb
@@ -650,23 +650,12 @@ prefill512_kernel(TileLaunch a) {
 
 namespace {
 
-// Keys per tile and waves per workgroup for head dim D.
-template <int D>
-constexpr int key_tile() {
-  return D == 512 ? 16 : 32;
-}
-template <int D>
-constexpr int tile_waves() {
-  return 8;
-}
-
 template <int D>
 hipError_t launch_prefill_d(const TileLaunch &a, int hpw, hipStream_t s) {
-  constexpr int KT = key_tile<D>(), NW = tile_waves<D>();
-  const dim3 grid(a.num_slots, a.hkv * ((a.hq / a.hkv) / hpw)), block(64 * NW);
+  const dim3 grid(a.num_slots, a.hkv * ((a.hq / a.hkv) / hpw)), block(512);
   switch (hpw) {
-    case 1: hipLaunchKernelGGL((prefill_kernel<D, 1, KT, NW>), grid, block, 0, s, a); break;
-    case 2: hipLaunchKernelGGL((prefill_kernel<D, 2, KT, NW>), grid, block, 0, s, a); break;
+    case 1: hipLaunchKernelGGL((prefill_kernel<D, 1>), grid, block, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((prefill_kernel<D, 2>), grid, block, 0, s, a); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();
@@ -688,10 +677,9 @@ namespace {
 // current device's properties, so the caller makes its device current first.
 template <int D, int HPW>
 int blocks_per_cu() {
-  constexpr int NW = tile_waves<D>();
   int b = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-          &b, prefill_kernel<D, HPW, key_tile<D>(), NW>, 64 * NW, 0) != hipSuccess ||
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, prefill_kernel<D, HPW>, 512, 0) !=
+          hipSuccess ||
       b < 1)
     b = 1;
   return b;
@@ -706,7 +694,6 @@ int blocks_per_cu_d(int hpw) {
 
 int prefill_fp32_blocks_per_cu(int head_dim, int heads_per_wg) {
   if (head_dim == 64) return blocks_per_cu_d<64>(heads_per_wg);
-  if (head_dim == 256) return blocks_per_cu_d<256>(heads_per_wg);
   if (head_dim == 512) {
     int b = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, prefill512_kernel<1>, 512, 0) !=
@@ -723,7 +710,6 @@ hipError_t launch_prefill_fp32(const TileLaunch &a, int hpw, hipStream_t s) {
   switch (a.head_dim) {
     case 64: return launch_prefill_d<64>(a, hpw, s);
     case 128: return launch_prefill_d<128>(a, hpw, s);
-    case 256: return launch_prefill_d<256>(a, hpw, s);
     case 512:
       if (hpw != 1) return hipErrorInvalidValue;
       hipLaunchKernelGGL((prefill512_kernel<1>), dim3(a.num_slots, a.hq), dim3(512), 0, s, a);

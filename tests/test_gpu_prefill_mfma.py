@@ -1,8 +1,9 @@
 """Parity of the prefill tile kernels over their configuration space, against the oracle.
 
-Steps as small as these run on the fp32 tiles where that kernel is the faster one; the split kernel
-has tests of its own, on larger steps.  Head dims 64, 128, 256 and 512, GQA ratios 1, 2, 4 and 8.  Each case mixes ragged sequences: a prefix hit
-(full pages), a mid-page chunk start, a two-query sequence (the smallest MFMA tile), a one-query
+Steps as small as these run on the fp32 tiles where that kernel is the faster one (head dims 64, 128
+and 512) and on the split tiles at 256; the split kernel has tests of its own, on larger steps.
+Head dims 64, 128, 256 and 512, GQA ratios 1, 2, 4 and 8.  Each case mixes ragged sequences: a
+prefix hit (full pages), a mid-page chunk start, a two-query sequence (the smallest MFMA tile), a one-query
 row (the row kernel) and lengths that leave partial query tiles and partial key tiles.  It runs
 paged with small and with the default page size, and dense (prefillDense), with and without a
 sliding window.  Bar: max-abs 1e-4 and rel-L2 1e-5 against the oracle; K/V pages bit-exact.

@@ -15,7 +15,7 @@ import torch
 
 from cases import Case
 from gpu_checks import dev, load_arena, say
-from nanollvm_amd import Attention, Context
+from nanollvm_amd import Attention, Context, KvCacheArena
 from nanollvm_amd import workloads as W
 
 pytestmark = pytest.mark.gpu
@@ -187,3 +187,32 @@ def test_zeros_and_negative_scale(ctx, d, rep):
     case.v[20:90] = 0.0
     case.q[60:300] = 0.0
     check(ctx, case, f"zeros d{d} rep{rep}")
+
+
+@pytest.mark.parametrize("d,hq,hkv,short,long", [(64, 32, 8, 70, 700), (128, 16, 8, 60, 600),
+                                                 (512, 8, 1, 30, 600), (256, 4, 1, None, 22)])
+def test_kernel_follows_the_step(ctx, d, hq, hkv, short, long):
+    """Short steps run on the fp32 tiles (none at d = 256), long ones on the split tiles, also when
+    the step changes between two calls of one layer configuration."""
+    attn = Attention(hq, d, float(np.float32(d ** -0.5)), hkv, 0, 0)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(d)
+    arena = KvCacheArena(ctx, 1, 2, 16, hkv, d)
+    ctx.set_timing(True)
+    try:
+        for n in [n for n in (short, long, short, long) if n]:
+            q = torch.randn(n, hq, d, device="cuda", generator=g)
+            k, v = torch.randn(2, n, hkv, d, device="cuda", generator=g)
+            ctx.set(True, cu_seqlens_q=[0, n], cu_seqlens_k=[0, n], max_seqlen_q=n, max_seqlen_k=n)
+            ctx.bind_kv_cache(arena)
+            ctx.reset_stats()
+            out = attn.forward(q, k, v, ctx)
+            ctx.sync()
+            fp32, _ = ctx.kernel_stats("prefill_fp32")
+            split, _ = ctx.kernel_stats("prefill_split")
+            assert (fp32, split) == ((1, 0) if n == short else (0, 1)), (n, fp32, split)
+            assert torch.isfinite(out).all()
+    finally:
+        ctx.set_timing(False)
+        ctx.clear()
+        arena.close()
