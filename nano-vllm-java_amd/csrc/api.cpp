@@ -429,15 +429,22 @@ int largest_pow2_divisor_upto(int rep, int cap) {
 // the two kernels: the tiles' time scales as 1/f, while the rows, being HBM-bound, keep
 // 1 - f^1.8 of the whole chip's bandwidth.  That is below what the rows keep alone on the
 // remaining CUs of a CU-masked stream (85% on half of the CUs, 68% on 3/8, 49% on 1/4), since
-// beside tile workgroups they lose bandwidth too.  Rates: rows 6.5 TB/s, tiles 200 TFLOP/s at
-// head dim <= 128 (the fp32 tiles of small steps 100), 80 / 70 at 256 / 512.  The tile rate is
-// what the model fits best with, below the 330 that the tiles reach alone: four 512-token chunks
-// beside 64 rows of 4096-16384 keys at 32 q / 8 KV heads take 1040 us at 100, 1005 at 150, 955 at
-// 200, 988 at 250, 1020 at 350 and 1300 at 500.
+// beside tile workgroups they lose bandwidth too.  Rates: rows 6.5 TB/s; split tiles, one workgroup
+// on a CU, 60 / 200 / 150 / 170 TFLOP/s at d = 64 / 128 / 256 / 512 (at d = 64 a workgroup is four
+// waves and three fill a CU), the fp32 tiles of small steps 100 (70 at d = 512).  The rates are what
+// the model fits best with on 240 drawn mixed steps of all head shapes (profiles/mixed_tile_share.md):
+// 144 further steps take 0.93 / 1.00 / 1.00 / 0.97 of the time at 200 / 200 / 80 / 70 on average, 32 q /
+// 8 KV heads at d = 64 down to half (8 rows beside 752 new tokens 374 -> 197 us).  At d = 128 rates
+// of 150 to 260 are within 1%: four 512-token chunks beside 64 rows of 4096-16384 keys at 32 q / 8 KV
+// heads take 1040 us at 100, 1005 at 150, 955 at 200, 988 at 250 and 1020 at 350.
 int64_t mixed_tile_cus(int num_cus, double row_bytes, double tile_flops, int head_dim, bool fp32) {
   const double tr = row_bytes / 6.5e12;
-  const double tt =
-      tile_flops / (head_dim <= 128 ? (fp32 ? 100e12 : 200e12) : head_dim <= 256 ? 80e12 : 70e12);
+  const double rate = fp32              ? (head_dim == 512 ? 70e12 : 100e12)
+                      : head_dim == 64  ? 60e12
+                      : head_dim == 128 ? 200e12
+                      : head_dim == 256 ? 150e12
+                                        : 170e12;
+  const double tt = tile_flops / rate;
   int best_s = 8;
   double best = 1e300;
   for (int s = 1; s < 16; s++) {
