@@ -60,7 +60,9 @@ namespace nva {
 namespace {
 
 constexpr float kLog2e = 1.4426950408889634f;
-constexpr int kProbExp = 11;  // probabilities, at most 2^kRaise, are split as 2^11 p <= 2^15
+// Probabilities, at most 2^kRaise, are split as 2^11 p <= 2^15.  (The factor is not taken in the
+// exponential: beside 11, the argument of a probability near 1 is rounded to 2^-21.)
+constexpr int kProbExp = 11;
 // Log2 units.  The reference that a query's probabilities are relative to moves up to a tile's max
 // that exceeds it by more than kRaise, and down to kMargin above one that lies kLower further below,
 // but no more than kRefSpan below the largest max so far.
@@ -272,12 +274,14 @@ __device__ void fp32_segment(const TileLaunch &a, const TileItem &it, int kvh, i
 // The reference of a query's probabilities from a tile of this max on; its sums are to be
 // multiplied by exp2(m - result).  It follows the tiles' maxima both ways: the probabilities are
 // split beside 2^kProbExp, and in tiles far below the largest max (where one key of little or no V
-// has most of the weight, all others) the split's steps would show.  top: the largest max so far.
+// has most of the weight, all others) the split's steps would show.  A whole number, so that the
+// factors of the sums are exact.  top: the largest max so far, rounded up.
 __device__ __forceinline__ float reference(float mx, float m, float &top) {
-  top = fmaxf(top, mx);
-  const float low = fmaxf(mx + kMargin, top - kRefSpan);
+  const float up = ceilf(mx);
+  top = fmaxf(top, up);
+  const float low = fmaxf(up + kMargin, top - kRefSpan);
   const bool down = mx > -INFINITY && m > low + kLower;
-  return mx > m + kRaise ? mx : down ? low : m;
+  return mx > m + kRaise ? up : down ? low : m;
 }
 
 // The exponent of V's scale, in which O is kept, for a tile of exponent e.  It follows the tiles both
@@ -312,7 +316,8 @@ __device__ __forceinline__ float dim_limit(int unit) {
 // lane's (scaled) probabilities: half a step of lo, 2^-25 and 2^-25.8 on average, in each of 16
 // probabilities beside |v| of up to 2^15, and in each v.
 __device__ __forceinline__ float split_steps(float p) {
-  return fmaf(p, 0x1p-26f, fminf(p * 0x1p15f, 0x1p-9f));
+  constexpr float scale = 1 << kProbExp;
+  return fmaf(p, scale * 0x1p-26f, fminf(p * (scale * 0x1p15f), 0x1p-9f));
 }
 
 // A query's largest result over a wave's dims; -INFINITY if one of them is not finite.
@@ -539,7 +544,6 @@ prefill_split_kernel(TileLaunch a) {
   const size_t rs = (size_t)a.hkv * D;
   const float *kbase = a.kv.k + (size_t)kvh * D;
   const float *vbase = a.kv.v + (size_t)kvh * D;
-  const float one = opaque_one();
 
   Again again{a.seg_off[slot], 0};
   for (int seg = again.first; seg < seg_end; seg++) {
@@ -695,7 +699,7 @@ prefill_split_kernel(TileLaunch a) {
         for (int b = 0; b < NB; b++) o[b] *= alpha;
         o_exp = v_exp;
       }
-      const float ms = (m_run == -INFINITY ? 0.0f : m_run) - (float)kProbExp;
+      const float ms = m_run == -INFINITY ? 0.0f : m_run;
       Split8 p[2];
       float lt[2];
 #pragma unroll
@@ -704,11 +708,11 @@ prefill_split_kernel(TileLaunch a) {
 #pragma unroll
         for (int j = 0; j < 8; j++) e[j] = __builtin_amdgcn_exp2f(fmaf(st[8 * s + j], c, -ms));
         lt[s] = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
-        p[s] = split8_unscaled(e, one);
+        p[s] = split8(e, (float)(1 << kProbExp));
       }
-      e_run += split_steps(lt[0] + lt[1]);
-      // One addition to the long sum per tile, without the probabilities' scale.
-      l_run = fmaf(lt[0] + lt[1], 1.0f / (1 << kProbExp), l_run);
+      const float l_tile = lt[0] + lt[1];
+      e_run += split_steps(l_tile);
+      l_run += l_tile;  // one addition to the long sum per tile
 
       // O^T += V^T P^T, 16 keys a step (V chunk 2 s + half holds the lane's keys).
 #pragma unroll
@@ -806,7 +810,6 @@ prefill_split_wide_kernel(TileLaunch a) {
   const float sl2 = fmaxf(fabsf(a.scale) * kLog2e, 0x1p-126f);
   const float qsign = a.scale < 0.0f ? -1.0f : 1.0f;
   const size_t rs = (size_t)a.hkv * D;
-  const float one = opaque_one();
 
   Again again{a.seg_off[slot], 0};
   for (int seg = again.first; seg < seg_end; seg++) {
@@ -999,7 +1002,7 @@ prefill_split_wide_kernel(TileLaunch a) {
           for (int b = 0; b < NB; b++) o[b] *= alpha;
           o_exp = v_exp;
         }
-        const float ms = (m_run == -INFINITY ? 0.0f : m_run) - (float)kProbExp;
+        const float ms = m_run == -INFINITY ? 0.0f : m_run;
         Split8 p[2];
         float lt[2];
 #pragma unroll
@@ -1008,10 +1011,11 @@ prefill_split_wide_kernel(TileLaunch a) {
 #pragma unroll
           for (int j = 0; j < 8; j++) e[j] = __builtin_amdgcn_exp2f(fmaf(st[8 * s + j], sl2, -ms));
           lt[s] = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
-          p[s] = split8_unscaled(e, one);
+          p[s] = split8(e, (float)(1 << kProbExp));
         }
-        e_run += split_steps(lt[0] + lt[1]);
-        l_run = fmaf(lt[0] + lt[1], 1.0f / (1 << kProbExp), l_run);
+        const float l_tile = lt[0] + lt[1];
+        e_run += split_steps(l_tile);
+        l_run += l_tile;  // one addition to the long sum per tile
         auto read_v = [&](int u) {
           return read_split(sv + part_pos(DW * ds + 32 * (u % NB) + i, 2 * (u / NB) + half));
         };

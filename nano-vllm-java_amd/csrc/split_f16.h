@@ -53,26 +53,6 @@ __device__ __forceinline__ Split8 split8(f32x8 x, float s) {
   return Split8{__builtin_bit_cast(f16x8, hi), __builtin_bit_cast(f16x8, lo)};
 }
 
-// The parts of x itself.  `one` is 1.0f, opaque to the compiler (see opaque_one): with a
-// constant the residual would take a conversion and a subtraction each.
-__device__ __forceinline__ Split8 split8_unscaled(f32x8 x, float one) {
-  u32x4 hi, lo;
-#pragma unroll
-  for (int j = 0; j < 4; j++) {
-    const float a = x[2 * j], b = x[2 * j + 1];
-    const f16x2 h = __builtin_convertvector(f32x2{a, b}, f16x2);
-    const f32x2 r{fmaf(one, a, -(float)h[0]), fmaf(one, b, -(float)h[1])};
-    hi[j] = __builtin_bit_cast(uint32_t, h);
-    lo[j] = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, f16x2));
-  }
-  return Split8{__builtin_bit_cast(f16x8, hi), __builtin_bit_cast(f16x8, lo)};
-}
-__device__ __forceinline__ float opaque_one() {
-  float one = 1.0f;
-  asm volatile("" : "+s"(one));
-  return one;
-}
-
 // Power-of-two scales of a block by the exponent field e of its largest magnitude (clamped to
 // [kMinExp, 255], so that every factor is a normal float): split_scale(e) takes that magnitude
 // to [2^14, 2^15), split_unscale(e) takes a result back.

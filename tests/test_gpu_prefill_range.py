@@ -54,7 +54,8 @@ def sink_score(weight, keys):
     return np.log(weight / (1.0 - weight) * keys) + 0.5
 
 
-def check(ctx, case, name, channels=slice(None), rows=slice(None), bar=BAR):
+def check(ctx, case, name, channels=slice(None), rows=slice(None), bar=BAR,
+          mean=False):
     wl, m = case.wl, case.wl.meta
     say(name)
     arena = load_arena(ctx, case)
@@ -81,9 +82,10 @@ def check(ctx, case, name, channels=slice(None), rows=slice(None), bar=BAR):
     assert np.all(np.isfinite(got))
     err = np.linalg.norm((got - want)[rows][..., channels], axis=-1)
     size = np.linalg.norm(want[rows][..., channels], axis=-1)
-    worst = float(np.max(err / np.where(size > 0, size, 1.0)))
-    say(f"{name}: worst row rel_l2={worst:.3e}")
-    assert worst <= bar, worst
+    rel = err / np.where(size > 0, size, 1.0)
+    rel = float(np.mean(rel) if mean else np.max(rel))
+    say(f"{name}: {'mean' if mean else 'worst'} row rel_l2={rel:.3e}")
+    assert rel <= bar, rel
 
 
 @pytest.mark.parametrize("v", [0.0, 1e-3])
@@ -148,3 +150,13 @@ def test_zero_dims(ctx, d, rep):
     case.v[:, :, d // 2:] = 0.0
     case.v[100:400] = 0.0
     check(ctx, case, f"zero dims d{d} rep{rep}")
+
+
+@pytest.mark.parametrize("d,rep", HEADS)
+def test_few_keys(ctx, d, rep):
+    """Rows of up to 32 keys, all of one tile: the probabilities' own rounding shows.  Bar, for the
+    mean row: 1.9e-7, between what the products leave (1.5e-7 to 1.75e-7) and that with another
+    2^-22 in the argument of every probability near 1, as beside a term of 8 to 16 (2.0e-7 to
+    2.3e-7)."""
+    case = build(d, rep, seed=17)
+    check(ctx, case, f"few keys d{d} rep{rep}", rows=slice(1, 32), bar=1.9e-7, mean=True)
