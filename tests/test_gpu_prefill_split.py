@@ -165,17 +165,32 @@ def test_rows_beyond_one_scale(ctx, d, rep, layout):
 
 
 @pytest.mark.parametrize("layout", ["paged16", "dense"])
+@pytest.mark.parametrize("value,window", [(np.inf, 0), (np.nan, 0), (-np.inf, 37)])
 @pytest.mark.parametrize("d,rep", HEADS)
-def test_infinities(ctx, d, rep, layout):
-    """An infinite V element reaches the queries that see it and no other; a key whose score is
-    -inf has weight 0."""
-    case = build(d, rep, layout, seed=5)
+def test_infinities(ctx, d, rep, value, window, layout):
+    """An infinite (or NaN) V element reaches the queries that see it and no other; a key whose score
+    is -inf has weight 0."""
+    case = build(d, rep, layout, window, seed=5)
     first = int(case.wl.meta.cu_seqlens_q[3])
     case.q[:, :, 0] = np.abs(case.q[:, :, 0]) + 0.5
-    case.v[first + 100, :, 3] = np.inf
+    case.v[first + 100, :, 3] = value
     case.k[first + 7] = 0.0
     case.k[first + 7, :, 0] = -np.inf
-    check(ctx, case, f"infinities d{d} rep{rep} {layout}")
+    check(ctx, case, f"infinities d{d} rep{rep} {value} w{window} {layout}")
+
+
+@pytest.mark.parametrize("d,rep", [(128, 2), (256, 1), (512, 1)])
+def test_more_segments_than_bits(ctx, d, rep):
+    """Hundreds of short sequences, over 64 to a workgroup, and in some of them an infinity: a wave
+    remembers the segments it takes again in 64 bits."""
+    rng = np.random.default_rng(d)
+    seqs = [(0, int(n)) for n in rng.integers(2, 7, 1500)] + LONG
+    wl = W.build(f"many segments d{d}", seqs, is_prefill=True, hq=16 * rep, hkv=16, d=d,
+                 scale=float(np.float32(d ** -0.5)), rng=rng, block_size=16, pool_cap=20000)
+    case = Case(wl, seed=9)
+    for b in (3, 700, 1400):
+        case.v[int(wl.meta.cu_seqlens_q[b]), :, 5] = np.inf
+    check(ctx, case, wl.name)
 
 
 @pytest.mark.parametrize("d,rep", HEADS)
