@@ -33,8 +33,10 @@ for _p in (ROOT, os.path.join(ROOT, "nano-vllm-java_amd")):
 METRIC = "decode-attn HBM GB/s (% of peak) + prefill-attn TFLOP/s, Qwen3-0.6B shape"
 HBM_PEAK_GBS = 8000.0
 FP32_MFMA_PEAK_TFLOPS = 157.3
-# fp32 products on split fp16 operands, three each at 2.5 PFLOP/s dense (prefill, large o_proj).
+# fp32 products on 16-bit parts at 2.5 PFLOP/s dense: three each on fp16 (prefill), six on bf16
+# (large o_proj).
 SPLIT_F16_PEAK_TFLOPS = 2500.0 / 3
+SPLIT_BF16_PEAK_TFLOPS = 2500.0 / 6
 
 
 def parse():
@@ -503,7 +505,8 @@ def o_proj_kernel(m, n):
                 "K over 8 waves)")
     if blocks <= cus:
         return "skinny_kernel<8,2> (fp32 MFMA 32x32x2, one 32x32 block per workgroup, K over 8 waves)"
-    return "linear_kernel (split fp16 MFMA 32x32x16, 128x128 tiles; K slices from a per-CU cost model)"
+    return ("linear_kernel (three-part bf16 MFMA 32x32x16, 128x128 tiles; K slices from a per-CU cost "
+            "model)")
 
 
 def time_calls(fn, steps, warmup):
@@ -539,7 +542,7 @@ def time_o_proj(ctx, attn_out, wl, steps, warmup, hidden=1024, seed=21):
     ms = time_calls(lambda: lin.forward(x, ctx), max(steps, 20), warmup)
     tf = flops / (ms * 1e-3) / 1e12
     kernel = o_proj_kernel(m, hidden)
-    peak = SPLIT_F16_PEAK_TFLOPS if kernel.startswith("linear") else FP32_MFMA_PEAK_TFLOPS
+    peak = SPLIT_BF16_PEAK_TFLOPS if kernel.startswith("linear") else FP32_MFMA_PEAK_TFLOPS
     return {"kernel": kernel, "shape": f"[{m}, {k}] x [{hidden}, {k}]^T",
             "ms": round(ms, 5), "tflops": round(tf, 2),
             "mfma_frac": round(tf / peak, 4),

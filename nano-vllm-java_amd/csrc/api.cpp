@@ -1009,8 +1009,8 @@ nva_status attention_plan(nva_ctx *ctx, const nva_attn_desc &d, int paged, int b
       *hpw_row = h;
       break;
     }
-  // Query heads per prefill workgroup: at most a quarter of its waves, so a workgroup covers at
-  // least 64 queries of each head (measured: Gemma3 d = 256 prefill 13% faster with 2 heads
+  // Query heads per prefill workgroup: at most two, so that it covers at least 64 queries of each
+  // head (measured on the fp32 tiles: Gemma3 d = 256 prefill 13% faster with 2 heads
   // than with 4, Gemma 4 d = 512 3% faster with 1 than with 4, Qwen3-4B shape 4% faster with 2
   // than with 4).
   *hpw_tile = largest_pow2_divisor_upto(rep, prefill_max_heads(d.head_dim));

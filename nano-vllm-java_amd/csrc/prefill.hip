@@ -13,8 +13,8 @@
 // Mapping onto CDNA4.  The grid is exactly as many workgroups per head group as can be resident
 // at once; each runs the segments of its slot of a stream-K schedule (equal numbers of 32-key
 // tiles per slot; a query tile whose keys straddle slots is split and its partials merged).  A
-// segment is a tile of 32 * NW / HPW queries of one sequence for HPW query heads of one KV head; each
-// wave owns 32 queries of one head, so one LDS read of a K or V operand (two parts, 32 bytes
+// segment is a tile of 32 * NW / HPW queries of one sequence for HPW query heads of one KV head;
+// each wave owns 32 queries of one head, so one LDS read of a K or V operand (two parts, 32 bytes
 // a lane) feeds three 32 x 32 x 16 products.
 //   * Key tiles of 32 rows: each wave loads a share of the next tile's K and V rows into
 //     registers (8 floats of each per lane at a time) while the current tile is computed, then
@@ -33,24 +33,25 @@
 //     tile's max exceeds it by more than 2^4 or lies more than 2^10 below it.  Only tiles that
 //     cross the causal diagonal, the window edge or the end of the keys are masked.
 //   * Every query adds up what the steps of the split can have done to its sums.  A wave with a
-//     query where that is more than 2^-21 of the result, whose sums are not finite (infinities in
-//     the inputs) or whose scores the steps would show in takes the segment's 32 queries again on
-//     fp32 matrix instructions, after all segments (fp32_segment; a call whose every query sees
-//     an infinity takes 3 to 5 times as long, up to 2.1 ms at 12289 cached + 2048 tokens before
-//     with the keys taken one by one: 9 to 20 times).
+//     query where that is more than 2^-21 of its largest result, whose sums are not finite
+//     (infinities in the inputs), whose scores the steps could move by 2^-23, or in whose V tiles
+//     one dim lies far below the others takes the segment's 32 queries again on fp32 matrix
+//     instructions, after all segments (fp32_segment).  Where every query sees an infinity a call
+//     takes 3 to 5 times as long (a 2048-token chunk after 12289 tokens 7.1 ms, 3.4 on the fp32
+//     tiles); with the keys taken one by one it was 7 to 19 times.
 //   * Operands are read from LDS two steps ahead of their products and the next tile is split
 //     and stored after QK: 14% fewer cycles than in source order, 4% less time.
 //
 // Bound by the board's power where steps are large: at d = 128 the matrix units are 47% busy at
-// 2.0 GHz (40% at 2.2 GHz before the reads moved ahead), and splitting the waves into early and
-// late ones, raising their priority around QK or interleaving the split with the products changed
-// nothing.  At d = 512 reloads of spilled registers wait for the V loads in flight.  Measured per
-// layer call, against fp32 matrix instructions: a 2048-token chunk after 12289 cached tokens,
-// 32 q / 8 KV heads, d = 128: 3.31 -> 1.33 ms; prompts of 512-2048 tokens: 16 q / 8 KV heads,
-// d = 128, 270 -> 155 us; 4 q / 1 KV, d = 256, window 512, 126 -> 111 us; 8 q / 1 KV, d = 512,
-// 681 -> 474 us; seven prompts of 5-333 tokens, 32 q / 8 KV, d = 64: 35.1 -> 30.5 us.  Error
-// against float64 (rel-L2): 1.7e-6 -> 1.3e-6, 6.9e-7 -> 4.8e-7, 9.6e-7 -> 4.7e-7, 1.0e-6 ->
-// 6.1e-7, 2.1e-7 -> 1.7e-7.
+// 1.96 GHz, and splitting the waves into early and late ones, raising their priority around QK or
+// interleaving the split with the products changed nothing.  At d = 512 reloads of spilled
+// registers wait for the V loads in flight.  Measured per layer call, against fp32 matrix
+// instructions: a 2048-token chunk after 12289 cached tokens, 32 q / 8 KV heads, d = 128: 3.32 ->
+// 1.37 ms; prompts of 512-2048 tokens: 16 q / 8 KV heads, d = 128, 273 -> 158 us; 4 q / 1 KV, d =
+// 256, window 512, 127 -> 105 us; 8 q / 1 KV, d = 512, 687 -> 484 us; seven prompts of 5-333
+// tokens, 32 q / 8 KV, d = 64: 36.8 -> 31.1 us.  (The checks and the moving units cost 1-3% of
+// these.)  Error against float64 (rel-L2): 1.7e-6 -> 1.3e-6, 7.1e-7 -> 4.8e-7, 9.7e-7 -> 4.6e-7,
+// 1.0e-6 -> 5.9e-7, 2.1e-7 -> 1.65e-7.
 #include "nva_internal.h"
 #include "nva_device.h"
 #include "split_f16.h"
@@ -1095,7 +1096,8 @@ int waves(int head_dim) { return head_dim == 64 ? split_waves<64>() : split_wave
 
 }  // namespace
 
-// Most query heads one prefill workgroup carries at this head dim: a quarter of its waves.
+// Most query heads one prefill workgroup carries at this head dim (it covers at least 64 queries of
+// each).
 int prefill_max_heads(int head_dim) { return head_dim == 64 || head_dim == 512 ? 1 : 2; }
 
 int prefill_tile_queries(int head_dim, int heads_per_wg) {

@@ -3,23 +3,23 @@
 //
 // x = hi + lo + e with hi = fp16(x) and lo = fp16(x - hi), both rounded to nearest (x - hi is
 // exact in fp32): hi holds 11 significant bits and lo, with its own sign and exponent, the next
-// 11 or 12, so |e| <= 2^-23 |x|, half an ulp of the fp32 value's own 24 bits away from it.  A
-// product x y is taken as lo hi' + hi lo' + hi hi', accumulated in fp32 with the largest last;
-// lo lo', below 2^-22 |x y| and of either sign, is left out.  The sum of n such products is off
-// by less than one fp32 accumulation of them, whose n roundings it does not make: the matrix
-// units round once per 16 products.
+// 11 or 12.  e is zero for three values in four and one step of the fp32 value's last bit for the
+// others, |e| <= 2^-23 |x|.  A product x y is taken as lo hi' + hi lo' + hi hi', accumulated in
+// fp32 with the largest last; lo lo', below 2^-22 |x y| and of either sign, is left out.  The
+// matrix units round once per 16 products, so a sum of n of them is off by less than one fp32
+// accumulation of them, which makes n roundings: measured against float64, every timed case and
+// every test of unlike sizes is closer than on v_mfma_f32 (prefill.hip).
 //
 // fp16 has five exponent bits, so operands are scaled by powers of two (exact): the largest
 // magnitude of a block goes to [2^14, 2^15), below fp16's 65504, and the smallest step of lo,
-// 2^-24, is then 2^-38 of that magnitude.  The users of this file choose the blocks, or check
-// their results, so that this step stays below 2^-24 of what it is added to; infinities become
-// NaN in lo and so in the sums they enter, which the users detect.  Both are then taken again on
-// fp32 instructions.
+// 2^-24, is then 2^-38 of that magnitude.  What such steps do to small values beside large ones is
+// bounded by the user of this file, which takes results they could show in again on fp32
+// instructions; infinities become NaN in lo and so in the sums they enter, which it detects.
 //
 // Three v_mfma_f32_32x32x16_f16 do the work of eight v_mfma_f32_32x32x2_f32 at half the cycles
-// each: 5.3 times the fp32 matrix rate.  (Three bf16 parts need no scale but six products: the
-// board's power limit then holds the clock to 1.8 GHz, and the 12K + 2K prefill chunk at 32 query
-// heads took 2.05 ms however it was scheduled.)
+// each: 5.3 times the fp32 matrix rate.  (Three bf16 parts hold every bit and need no scale, but
+// six products, as linear.hip takes them: the board's power limit then holds the clock to 1.8 GHz,
+// and the 12K + 2K prefill chunk at 32 query heads took 2.05 ms however it was scheduled.)
 #pragma once
 
 #include <hip/hip_runtime.h>

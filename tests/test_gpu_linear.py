@@ -1,10 +1,10 @@
-"""o_proj (Linear.Row -> Ops.linear) on fp32 MFMA through the C ABI, against the oracle's
+"""o_proj (Linear.Row -> Ops.linear) through the C ABI, against the oracle's
 restatement of the reference's gemv at decode shapes, and against float64 at the full prefill
 shapes.  Bar: max-abs 1e-4 and rel-L2 1e-5, the path's floating-point tolerance.
 
-The library's kernels by shape: the weight-streaming GEMV up to 8 rows, 32 x 32 blocks (K over
-eight waves, K slices plus the reduce) while the blocks fit one per CU, 128 x 64 tiles (K slices
-when the tiles leave CUs idle) above."""
+The library's kernels by shape: the weight-streaming GEMV up to 16 rows, 16 x 16 or 32 x 32 blocks
+(K over eight waves; K slices plus the reduce) while the blocks fit the CUs, 128 x 128 tiles (K
+slices when the tiles leave CUs idle) above."""
 
 import sys
 
@@ -78,7 +78,7 @@ def check(got, want, name):
     (24, 8192, 256, False),    # 32 K slices of one 32-k stage per wave
     (130, 2048, 1024, False),  # M tail past one 128-row tile
     (256, 2048, 1024, True),   # 256-row decode batch: 256 blocks, one per CU
-    (384, 2048, 1024, True),   # more blocks than CUs: 128 x 64 tiles, K slices plus the reduce
+    (384, 2048, 1024, True),   # more blocks than CUs: 128 x 128 tiles, K slices plus the reduce
     (384, 1028, 1000, True),   # tiles: interior and edge tiles side by side, ragged N and K
     (300, 4100, 520, False),   # tiles: M and N tails, K % 32 == 4 (a ragged last K tile)
     (1000, 100, 70, True),     # tiles: one K tile, ragged (K = 100), N shorter than a tile
@@ -130,7 +130,7 @@ def test_linear_repeatable_bit_for_bit(ctx):
 @pytest.mark.parametrize("seed", range(12))
 def test_linear_fuzz_fp64(ctx, seed):
     """Random shapes across the four kernels and their edges (GEMV forms, 32 x 32 blocks with K
-    slices, 128 x 64 tiles with slices, ragged M / N / K tails, grids that do and do not divide
+    slices, 128 x 128 tiles with slices, ragged M / N / K tails, grids that do and do not divide
     into XCD rectangles), with and without bias, against a float64 product on the device."""
     rng = np.random.default_rng(1000 + seed)
     rows = int(rng.choice([int(rng.integers(1, 9)), int(rng.integers(9, 300)),
