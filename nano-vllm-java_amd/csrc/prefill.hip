@@ -33,7 +33,7 @@
 //     tile's max exceeds it by more than 2^4 or lies more than 2^10 below it.  Only tiles that
 //     cross the causal diagonal, the window edge or the end of the keys are masked.
 //   * Every query adds up what the steps of the split can have done to its sums.  A wave with a
-//     query where that is more than 2^-21 of its largest result, whose sums are not finite
+//     query where that is more than 2^-19 of its largest result, whose sums are not finite
 //     (infinities in the inputs), whose scores the steps could move by 2^-23, or in whose V tiles
 //     one dim lies far below the others takes the segment's 32 queries again on fp32 matrix
 //     instructions, after all segments (fp32_segment).  Where every query sees an infinity a call
@@ -314,8 +314,9 @@ __device__ __forceinline__ float dim_limit(int unit) {
 }
 
 // What the steps of the split add to the error of a query's o in one tile, p being the sum of the
-// lane's (scaled) probabilities: half a step of lo, 2^-25 and 2^-25.8 on average, in each of 16
-// probabilities beside |v| of up to 2^15, and in each v.
+// lane's probabilities: half a step of lo, 2^-25 and 2^-25.8 on average, in each of 16 (scaled)
+// probabilities beside |v| of up to 2^15, and in each v.  (Added up over the tiles by squares: the
+// roundings are independent.)
 __device__ __forceinline__ float split_steps(float p) {
   constexpr float scale = 1 << kProbExp;
   return fmaf(p, scale * 0x1p-26f, fminf(p * (scale * 0x1p15f), 0x1p-9f));
@@ -340,10 +341,11 @@ __device__ __forceinline__ float largest_result(const f32x16 (&o)[NB], float l) 
 }
 
 // Whether a query's sums (o in units of 2^kProbExp and the V scale) cannot stand: one is not finite,
-// or the split's steps, e, are more than 2^-21 of the largest result.  (At the smallest scale, V
+// or the split's steps, e their squares, are more than 2^-19 of the largest result: with |v| at its
+// bound; usually a quarter of that, as |v| mostly lies at a sixth of it.  (At the smallest scale, V
 // holds nothing but zeros and values below 2^-105.)
 __device__ __forceinline__ bool unsound(float result, float e, int v_top) {
-  return result < 0.0f || (result < e * 0x1p21f && v_top > kMinExp);
+  return result < 0.0f || (result < __builtin_sqrtf(e) * 0x1p19f && v_top > kMinExp);
 }
 
 // The factor of a query's sums in its result: 1 / l or, in a partial, to the largest max.
@@ -688,14 +690,14 @@ prefill_split_kernel(TileLaunch a) {
       if (__any(mn != m_run)) {
         const float alpha = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - mn);
         l_run *= alpha;
-        e_run *= alpha;
+        e_run *= alpha * alpha;
 #pragma unroll
         for (int b = 0; b < NB; b++) o[b] *= alpha;
         m_run = mn;
       }
       if (v_exp != o_exp) {
         const float alpha = __uint_as_float((uint32_t)max(0, 127 + o_exp - v_exp) << 23);
-        e_run *= alpha;
+        e_run *= alpha * alpha;
 #pragma unroll
         for (int b = 0; b < NB; b++) o[b] *= alpha;
         o_exp = v_exp;
@@ -712,7 +714,8 @@ prefill_split_kernel(TileLaunch a) {
         p[s] = split8(e, (float)(1 << kProbExp));
       }
       const float l_tile = lt[0] + lt[1];
-      e_run += split_steps(l_tile);
+      const float steps = split_steps(l_tile);
+      e_run = fmaf(steps, steps, e_run);
       l_run += l_tile;  // one addition to the long sum per tile
 
       // O^T += V^T P^T, 16 keys a step (V chunk 2 s + half holds the lane's keys).
@@ -991,14 +994,14 @@ prefill_split_wide_kernel(TileLaunch a) {
         if (__any(mn != m_run)) {
           const float alpha = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - mn);
           l_run *= alpha;
-          e_run *= alpha;
+          e_run *= alpha * alpha;
 #pragma unroll
           for (int b = 0; b < NB; b++) o[b] *= alpha;
           m_run = mn;
         }
         if (v_exp != o_exp) {
           const float alpha = __uint_as_float((uint32_t)max(0, 127 + o_exp - v_exp) << 23);
-          e_run *= alpha;
+          e_run *= alpha * alpha;
 #pragma unroll
           for (int b = 0; b < NB; b++) o[b] *= alpha;
           o_exp = v_exp;
@@ -1015,7 +1018,8 @@ prefill_split_wide_kernel(TileLaunch a) {
           p[s] = split8(e, (float)(1 << kProbExp));
         }
         const float l_tile = lt[0] + lt[1];
-        e_run += split_steps(l_tile);
+        const float steps = split_steps(l_tile);
+        e_run = fmaf(steps, steps, e_run);
         l_run += l_tile;  // one addition to the long sum per tile
         auto read_v = [&](int u) {
           return read_split(sv + part_pos(DW * ds + 32 * (u % NB) + i, 2 * (u / NB) + half));
