@@ -432,7 +432,7 @@ int largest_pow2_divisor_upto(int rep, int cap) {
 // beside tile workgroups they lose bandwidth too.  Rates: rows 6.5 TB/s; split tiles, one workgroup
 // on a CU, 60 / 200 / 150 / 170 TFLOP/s at d = 64 / 128 / 256 / 512 (at d = 64 a workgroup is four
 // waves and three fill a CU), the fp32 tiles of small steps 100 (70 at d = 512).  The rates are what
-// the model fits best with on 240 drawn mixed steps of all head shapes (profiles/mixed_tile_share.md):
+// the model fits best with on 240 drawn mixed steps of all head shapes:
 // 144 further steps take 0.93 / 1.00 / 1.00 / 0.97 of the time at 200 / 200 / 80 / 70 on average, 32 q /
 // 8 KV heads at d = 64 down to half (8 rows beside 752 new tokens 374 -> 197 us).  At d = 128 rates
 // of 150 to 260 are within 1%: four 512-token chunks beside 64 rows of 4096-16384 keys at 32 q / 8 KV
@@ -941,7 +941,7 @@ KvView make_dense_view(const float *k, const float *v) {
 // larger of a floor and the time of its active waves) over the CUs, or one tile's latency if that
 // is longer, plus the split kernel's later start.  At d = 512 the fp32 kernel takes steps of less
 // than 0.75 key tiles per CU, at d = 256 none.  On 560 drawn steps of 1-6 prompts or chunks, timed
-// with both kernels (profiles/prefill_tile_choice.md), the rule's time over the better kernel's is
+// with both kernels, the rule's time over the better kernel's is
 // 1.005 / 1.007 / 1.002 / 1.004 on average at d = 64 / 128 / 256 / 512.  fp32 / split us a layer
 // call: 32 q / 8 KV heads, d = 64, 70 tokens 14.4 / 16.1, 505 46.0 / 42.4; 16 q / 8 KV, d = 128, 160
 // tokens 23.0 / 27.1, 14+295 35.7 / 33.6; 4 q / 1 KV, d = 256, 22 and 3+7 15.7 / 16.3, 400 33.8 /
