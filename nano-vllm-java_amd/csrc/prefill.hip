@@ -69,8 +69,8 @@ constexpr int kProbExp = 11;
 // but no more than kRefSpan below the largest max so far.
 constexpr float kRaise = 4.0f, kMargin = 4.0f, kLower = 6.0f, kRefSpan = 40.0f;
 // Largest factor from products of scaled q and k (off by about 2^-7 from the steps of the split)
-// to scores: their error stays below 2^-23, what fp32 sums leave in scores of 1.
-constexpr float kMaxScoreUnit = 0x1p-16f;
+// to scores: their error stays below 2^-20.
+constexpr float kMaxScoreUnit = 0x1p-13f;
 // The exponent of V's scale stays for tiles of up to kUnitSlack below it and within kUnitSpan of the
 // largest one's.
 constexpr int kUnitSlack = 3, kUnitSpan = 32;
