@@ -34,7 +34,7 @@
 //     cross the causal diagonal, the window edge or the end of the keys are masked.
 //   * Every query adds up what the steps of the split can have done to its sums.  A wave with a
 //     query where that is more than 2^-19 of its largest result, whose sums are not finite
-//     (infinities in the inputs), whose scores the steps could move by 2^-23, or in whose V tiles
+//     (infinities in the inputs), in whose scores the steps could show, or in whose V tiles
 //     one dim lies far below the others takes the segment's 32 queries again on fp32 matrix
 //     instructions, after all segments (fp32_segment).  Where every query sees an infinity a call
 //     takes 3 to 5 times as long (a 2048-token chunk after 12289 tokens 7.1 ms, 3.4 on the fp32
@@ -68,8 +68,10 @@ constexpr int kProbExp = 11;
 // that exceeds it by more than kRaise, and down to kMargin above one that lies kLower further below,
 // but no more than kRefSpan below the largest max so far.
 constexpr float kRaise = 4.0f, kMargin = 4.0f, kLower = 6.0f, kRefSpan = 40.0f;
-// Largest factor from products of scaled q and k (off by about 2^-7 from the steps of the split)
-// to scores: their error stays below 2^-20.
+// Largest factor from products of scaled q and k to scores.  The steps of the split put such a
+// product off by at most about 2^-7 (both operands at their largest in every dim, when fp32 sums are
+// off by more), by about 2^-10 beside a K row or channel far above the others: 2^-23 of a score at
+// this factor.  Rows of such steps move away from float64 from 2^-11 on.
 constexpr float kMaxScoreUnit = 0x1p-13f;
 // The exponent of V's scale stays for tiles of up to kUnitSlack below it and within kUnitSpan of the
 // largest one's.
@@ -139,7 +141,8 @@ __device__ __forceinline__ Dest destination(const TileLaunch &a, const TileItem 
 // The segment's result for a wave's 32 queries (from tile query q0 on) and dims [v0, v0 + 32 NB) of V
 // on fp32 matrix instructions, operands straight from memory: for segments that the split does not
 // fit.  Lanes and registers of S^T and O^T are those of the split products; a step of PV contracts
-// the keys of one S^T register.  O^T is added up over the tiles' own sums, one rounding a tile.
+// the keys of one S^T register.  Scores are added up over sums of 64 dims and O^T over the tiles' own,
+// which leaves 2.2e-7 of a row where the split leaves 2.2e-7 to 2.9e-7.
 template <int D, int NB>
 __device__ void fp32_segment(const TileLaunch &a, const TileItem &it, int kvh, int h, int q0, int v0) {
   const int lane = threadIdx.x & 63;
@@ -173,22 +176,28 @@ __device__ void fp32_segment(const TileLaunch &a, const TileItem &it, int kvh, i
     const bool full = kt >= all_lo && kt + KT <= min(all_hi, it.ke);
     const int64_t row = key_row(a.kv, table, 0, it.kbase, min(kt + i, it.ke - 1));
     const float *kp = kbase + (size_t)row * rs;
-    f32x16 st, su;
+    f32x16 st;
 #pragma unroll
-    for (int r = 0; r < 16; r++) st[r] = su[r] = 0.0f;
+    for (int r = 0; r < 16; r++) st[r] = 0.0f;
+#pragma unroll 1
+    for (int c = 0; c < D; c += 64) {  // 64 dims a sum, in two chains
+      f32x16 sa, sb;
+#pragma unroll
+      for (int r = 0; r < 16; r++) sa[r] = sb[r] = 0.0f;
 #pragma unroll 2
-    for (int s = 0; s < D; s += 16) {
-      const float4 x = ld4(kp + s), y = ld4(qp + s), z = ld4(kp + s + 8), w = ld4(qp + s + 8);
-      st = __builtin_amdgcn_mfma_f32_32x32x2f32(x.x, y.x, st, 0, 0, 0);
-      su = __builtin_amdgcn_mfma_f32_32x32x2f32(z.x, w.x, su, 0, 0, 0);
-      st = __builtin_amdgcn_mfma_f32_32x32x2f32(x.y, y.y, st, 0, 0, 0);
-      su = __builtin_amdgcn_mfma_f32_32x32x2f32(z.y, w.y, su, 0, 0, 0);
-      st = __builtin_amdgcn_mfma_f32_32x32x2f32(x.z, y.z, st, 0, 0, 0);
-      su = __builtin_amdgcn_mfma_f32_32x32x2f32(z.z, w.z, su, 0, 0, 0);
-      st = __builtin_amdgcn_mfma_f32_32x32x2f32(x.w, y.w, st, 0, 0, 0);
-      su = __builtin_amdgcn_mfma_f32_32x32x2f32(z.w, w.w, su, 0, 0, 0);
+      for (int s = c; s < c + 64; s += 16) {
+        const float4 x = ld4(kp + s), y = ld4(qp + s), z = ld4(kp + s + 8), w = ld4(qp + s + 8);
+        sa = __builtin_amdgcn_mfma_f32_32x32x2f32(x.x, y.x, sa, 0, 0, 0);
+        sb = __builtin_amdgcn_mfma_f32_32x32x2f32(z.x, w.x, sb, 0, 0, 0);
+        sa = __builtin_amdgcn_mfma_f32_32x32x2f32(x.y, y.y, sa, 0, 0, 0);
+        sb = __builtin_amdgcn_mfma_f32_32x32x2f32(z.y, w.y, sb, 0, 0, 0);
+        sa = __builtin_amdgcn_mfma_f32_32x32x2f32(x.z, y.z, sa, 0, 0, 0);
+        sb = __builtin_amdgcn_mfma_f32_32x32x2f32(z.z, w.z, sb, 0, 0, 0);
+        sa = __builtin_amdgcn_mfma_f32_32x32x2f32(x.w, y.w, sa, 0, 0, 0);
+        sb = __builtin_amdgcn_mfma_f32_32x32x2f32(z.w, w.w, sb, 0, 0, 0);
+      }
+      st += sa + sb;
     }
-    st += su;
     float mx = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 16; r++) {

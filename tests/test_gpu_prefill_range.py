@@ -166,8 +166,8 @@ def test_few_keys(ctx, d, rep):
 def test_random_magnitudes(ctx, seed):
     """Steps with several of these at once, by chance: V rows, channels and tiles over up to 2^30, a
     few rows far above the others, zero channels, sharper scores, K channels that no score shows,
-    keys with most of the weight.  Bar: 1e-5, the attention bar; on ten times as many seeds the worst
-    row was 5.0e-6 off, on the fp32 tiles 8.3e-6."""
+    keys with most of the weight.  Bar: 1e-5, the attention bar; on twenty times as many seeds the
+    worst row was 7.2e-6 off, on the fp32 tiles 1.1e-5."""
     rng = np.random.default_rng(1000 + seed)
     d = int(rng.choice([64, 128, 256, 512]))
     case = build(d, int(rng.choice([1, 2, 4])), seed=1000 + seed,
